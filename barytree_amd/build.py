@@ -32,6 +32,12 @@ HIP_FLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              # matrix-core results straight into VGPRs (no AGPR copies per pair)
              "-mllvm", "-amdgpu-mfma-vgpr-form",
+             # kernel arguments stay in the constant address space however many
+             # uses they have: past LLVM's default of 300 uses the tensor-grid
+             # kernels copied their 984 bytes of arguments to scratch, per
+             # thread, and read every table pointer back from there (161 VGPRs
+             # instead of 124 as well)
+             "-mllvm", "-instcombine-max-copied-from-constant-users=100000",
              "-munsafe-fp-atomics"]
 
 
