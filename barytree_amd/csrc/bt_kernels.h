@@ -3,6 +3,10 @@
 // them; every pointer here is a device pointer.
 #pragma once
 
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
+
 #include <hip/hip_runtime_api.h>
 #include <hip/hip_vector_types.h>
 
@@ -30,6 +34,38 @@ constexpr int MAX_DEGREE = 12;
 constexpr int DEG_SHIFT = 24;               // (degree << DEG_SHIFT) | slot
 constexpr int SLOT_MASK = (1 << DEG_SHIFT) - 1;
 
+// Constants of e^{-k u} in FP64 (bt_exp.h): c = k EXP_TAB / ln 2 and the
+// largest u evaluated.
+constexpr int EXP_TAB = 256;
+struct ExpRate { double c, umax; };
+// k = 0: e^0 = 1 for every u; k beyond the range of c (an infinite rate,
+// a = 0): the largest that keeps c finite, where e^{-k u} is 0 for every
+// u > 1e-287.  k < 0 (a growing exponential): u is clamped where e^{|k| u}
+// has overflowed.
+inline ExpRate exp_rate(long double k)
+{
+    const long double lim = 1e290L;
+    k = std::max(-lim, std::min(lim, k));
+    ExpRate r;
+    r.c = (double)(k * EXP_TAB / 0.693147180559945309417232121458176568L);
+    const long double um = (k < 0.0L ? -800.0L : 746.0L) / k;
+    r.umax = k == 0.0L || um > DBL_MAX ? DBL_MAX : (double)um;
+    return r;
+}
+// Constants of sin(k r): c + clo = k SIN_TAB / (2 pi); table form below rmax.
+constexpr int SIN_TAB = 512;
+struct SinRate { double c, clo, rmax; };
+inline SinRate sin_rate(double k)
+{
+    const long double c = (long double)k * SIN_TAB / 6.283185307179586476925286766559005768L;
+    SinRate r;
+    r.c = (double)c;
+    r.clo = (double)(c - r.c);
+    r.rmax = k == 0.0 ? DBL_MAX : (double)std::min((long double)DBL_MAX, 0x1p50L / std::fabs(c));
+    if (!(std::fabs(r.c) < 1e300)) r = {0.0, 0.0, 0.0};  // the library's sin throughout
+    return r;
+}
+
 // Kernel parameters, pre-derived on the host.
 struct KParams {
     double p0, p1;      // kernel_params[0], kernel_params[1]
@@ -39,6 +75,8 @@ struct KParams {
     // atan: delta factor sqrt(1 + 1/delta^2) and wadj; mq: (delta/L)^2 and
     // sqrt(1 + 4 (delta/L)^2); rbs-u, rbs-v: delta^2 (in c1)
     double c1, c2;
+    ExpRate ek, eg;  // e^{-p0 r} (p0 = kappa) and e^{-r^2 inv_a2}
+    SinRate sn;      // sin(p0 r)
 };
 
 // Kernel ids beside Coulomb (1), Yukawa (2) and regularized Coulomb (3)

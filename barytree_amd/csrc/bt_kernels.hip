@@ -18,6 +18,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "bt_exp.h"
 #include "bt_kernels.h"
 #include "bt_rsq.h"
 
@@ -31,44 +32,19 @@ constexpr int NQ = TILE_QUEUES;  // tile queues, one per XCD
 constexpr int KC = 1, KY = 2, KR = 3;
 
 
-// ---------------------------------------------------------------------
-// e^x in FP64 for x <= 0, with a table of 2^(j/64), j < 64 (EXP_TAB
-// doubles, filled by exp_table).  x is clamped at -746, where e^x is below
-// half the least subnormal.  x = (64 k + j) ln2/64 + f with t = 64 k + j
-// the integer nearest x 64/ln2 and |f| <= ln2/128 (ln2/64 split in a
-// 36-bit head, exact times |t| < 2^17, and a tail); e^f by its Taylor
-// polynomial to degree 5 (truncation below 3.5e-17 relative); the result
-// 2^k tab[j] e^f is within about 2 ulp of e^x.
-// ---------------------------------------------------------------------
-constexpr int EXP_TAB = 64;
-
-__device__ __forceinline__ void exp_table(double *tab, int tid)
-{
-    if (tid < EXP_TAB) tab[tid] = exp2((double)tid * (1.0 / EXP_TAB));
-}
-
-__device__ __forceinline__ double exp_nonpos(double x, const double *tab)
-{
-    constexpr double INV = 92.33248261689366;                // 64 / ln 2
-    constexpr double HI = 0x1.62e42fefa0000p-7, LO = 2.572804622327669e-14;  // ln2/64
-    x = fmax(x, -746.0);
-    const double t = __builtin_rint(x * INV);
-    const double f = fma(-t, LO, fma(-t, HI, x));
-    const int n = (int)t;
-    double p = fma(f, 1.0 / 120.0, 1.0 / 24.0);
-    p = fma(f, p, 1.0 / 6.0);
-    p = fma(f, p, 0.5);
-    p = fma(f, p, 1.0);
-    p = fma(f, p, 1.0);
-    return __builtin_amdgcn_ldexp(tab[n & (EXP_TAB - 1)] * p, n >> 6);
-}
-
-// e^x, x <= 0: the table form (TAB) or the library's
+// e^{-kappa r} and e^{-r^2 inv_a2}: the table form (TAB, bt_exp.h) or the
+// library's
 template <bool TAB>
-__device__ __forceinline__ double exp_np(double x, const double *tab)
+__device__ __forceinline__ double exp_kr(double r, const KParams &kp, const double *tab)
 {
-    if constexpr (TAB) return exp_nonpos(x, tab);
-    else return exp(x);
+    if constexpr (TAB) return exp_neg(r, kp.ek, tab);
+    else return exp(-kp.p0 * r);
+}
+template <bool TAB>
+__device__ __forceinline__ double exp_r2(double r2, const KParams &kp, const double *tab)
+{
+    if constexpr (TAB) return exp_neg(r2, kp.eg, tab);
+    else return exp(-r2 * kp.inv_a2);
 }
 
 // ---------------------------------------------------------------------
@@ -84,7 +60,8 @@ __device__ __forceinline__ double exp_np(double x, const double *tab)
 // (regularized-yukawa_{pp,ss_pp,pc,ss_pc,cp}.c, atan_{pp,pc}.c,
 // sin-over-r_{pp,pc,cp}.c, mq_{pp,pc}.c, rbs-u_*.c, rbs-v_*.c, user_kernel_*.c)
 // A division by a square root is a product with rsq64 (bt_rsq.h; about 1 ulp, against
-// two correctly rounded operations in the reference's form).  dz/L stays a
+// two correctly rounded operations in the reference's form), and r itself is
+// r^2 rsq64(r^2).  TAB: e^{-kr} and sin(kr) from tables (bt_exp.h).  dz/L stays a
 // division: atan and MQ jump at d = +-1/2, where the wrap must see the
 // reference's rounding of d.
 // ---------------------------------------------------------------------
@@ -98,13 +75,14 @@ __device__ __forceinline__ double wrap_half(double d)
     return d;
 }
 
-template <int KER, bool SS, bool CHECK>
+template <int KER, bool SS, bool CHECK, bool TAB>
 __device__ __forceinline__ double other_term(double dx, double dy, double dz, double r2, double a, double b,
-                                             double tq, const KParams &kp)
+                                             double tq, const KParams &kp, const double *tab)
 {
     if constexpr (KER == KRY) {
-        const double r = sqrt(r2);
-        const double e = exp(-kp.p0 * r) * rsq64(r2 + kp.eps2);
+        // r = 0 for coincident points, which this kernel does not skip
+        const double r = TAB ? r2 * rsq64(fmax(r2, 1e-300)) : sqrt(r2);
+        const double e = exp_kr<TAB>(r, kp, tab) * rsq64(r2 + kp.eps2);
         return (SS ? fma(-tq, b, a) : a) * e;
     } else if constexpr (KER == KAT) {
         const double d = wrap_half(dz / kp.p0);
@@ -116,8 +94,16 @@ __device__ __forceinline__ double other_term(double dx, double dy, double dz, do
         const double r = fma(dy, dy, dx * dx) + kp.c1;
         return (KER == KRU ? 1.0 : -1.0) / (2.0 * M_PI) * a * (KER == KRU ? dy : dx) / r;
     } else {  // KSR, KUS
-        const double r = sqrt(r2), ir = rsq64(r2);
-        double v = (KER == KSR ? sin(kp.p0 * r) : exp(-kp.p0 * r)) * ir;
+        const double ir = rsq64(r2);
+        double r = TAB ? r2 * ir : sqrt(r2), v;
+        if constexpr (KER == KSR) {
+            // the sine sees k times r's rounding: one Newton step makes r
+            // as good as the root (half an ulp)
+            if constexpr (TAB) r = fma(fma(-r, r, r2), 0.5 * ir, r);
+            v = (TAB ? sin_kr(r, kp.p0, kp.sn, tab) : sin(kp.p0 * r)) * ir;
+        } else {
+            v = exp_kr<TAB>(r, kp, tab) * ir;
+        }
         if constexpr (CHECK) v = r > DBL_MIN ? v : 0.0;
         return a * v;
     }
@@ -139,7 +125,7 @@ __device__ __forceinline__ double other_term(double dx, double dy, double dz, do
 // can never trigger; cluster sources never need it (an accepted cluster is
 // separated from its targets).
 // ---------------------------------------------------------------------
-// TAB: exponentials by exp_nonpos from the table tab.
+// TAB: exponentials from the table tab.
 template <int KER, bool SS, bool CHECK, bool TAB = false>
 __device__ __forceinline__ void pair_pot(double dx, double dy, double dz, double a, double b,
                                          double tq, const KParams &kp, double &acc,
@@ -150,19 +136,19 @@ __device__ __forceinline__ void pair_pot(double dx, double dy, double dz, double
         double ir = rsq64(r2);
         if constexpr (CHECK) ir = r2 > (SS ? 0.0 : DBL_MIN) ? ir : 0.0;
         if constexpr (!SS) acc = fma(a, ir, acc);
-        else acc = fma(fma(-tq * b, exp_np<TAB>(-r2 * kp.inv_a2, tab), a), ir, acc);
+        else acc = fma(fma(-tq * b, exp_r2<TAB>(r2, kp, tab), a), ir, acc);
     } else if constexpr (KER == KY) {
         const double ir = rsq64(r2);
-        double e = exp_np<TAB>(-kp.p0 * (r2 * ir), tab) * ir;
+        double e = exp_kr<TAB>(r2 * ir, kp, tab) * ir;
         if constexpr (CHECK) e = r2 > 0.0 ? e : 0.0;
         if constexpr (!SS) acc = fma(a, e, acc);
         else acc = fma(fma(-tq, b, a), e, acc);
     } else if constexpr (KER == KR) {
         const double ir = rsq64(r2 + kp.eps2);
         if constexpr (!SS) acc = fma(a, ir, acc);
-        else acc = fma(fma(-tq * b, exp_np<TAB>(-r2 * kp.inv_a2, tab), a), ir, acc);
+        else acc = fma(fma(-tq * b, exp_r2<TAB>(r2, kp, tab), a), ir, acc);
     } else {
-        acc += other_term<KER, SS, CHECK>(dx, dy, dz, r2, a, b, tq, kp);
+        acc += other_term<KER, SS, CHECK, TAB>(dx, dy, dz, r2, a, b, tq, kp, tab);
     }
 }
 
@@ -182,10 +168,10 @@ __device__ __forceinline__ void grid_term(double r2, double a, double b, const K
     if constexpr (KER == KC) {
         const double ir = rsq64(r2);
         q = fma(a, ir, q);
-        if constexpr (SS) w = fma(exp_np<TAB>(-r2 * kp.inv_a2, tab) * b, ir, w);
+        if constexpr (SS) w = fma(exp_r2<TAB>(r2, kp, tab) * b, ir, w);
     } else if constexpr (KER == KY) {
         const double ir = rsq64(r2);
-        const double e = exp_np<TAB>(-kp.p0 * (r2 * ir), tab) * ir;
+        const double e = exp_kr<TAB>(r2 * ir, kp, tab) * ir;
         q = fma(a, e, q);
         if constexpr (SS) w = fma(b, e, w);
     } else {
@@ -203,7 +189,7 @@ __device__ __forceinline__ void pair_grid(double dx, double dy, double dz, doubl
     if constexpr (KER == KC || KER == KY || KER == KR) {
         grid_term<KER, SS, TAB>(r2, a, b, kp, q, w, tab);
     } else {
-        q += other_term<KER, false, false>(dx, dy, dz, r2, a, 0.0, 0.0, kp);
+        q += other_term<KER, false, false, TAB>(dx, dy, dz, r2, a, 0.0, 0.0, kp, tab);
     }
 }
 
@@ -945,7 +931,7 @@ __global__ __launch_bounds__(256) void k_grid_pencil64(InteractArgs A)
     __shared__ double4 Ls[256];          // source point and its a charge
     __shared__ double Lb[SS ? 256 : 1];  // its b charge (subtraction)
     __shared__ double Lr[(SS ? 2 : 1) * PENCIL_RED];
-    __shared__ double Ltab[EXP_TAB];     // 2^(j/64) for exp_nonpos
+    __shared__ double Ltab[EXP_TAB];     // 2^(j/256) for exp_neg
     if constexpr (SS || KER == KY) exp_table(Ltab, threadIdx.x);  // read after the first staging barrier
     const Tile tile = A.tiles[blockIdx.x];
     if (tile.z == 0) return;  // padding (block-uniform)
@@ -982,9 +968,10 @@ __global__ __launch_bounds__(TPB) void k_interact(InteractArgs A)
     __shared__ double4 Ls[TPB];
     __shared__ double Lb[SS ? TPB : 1];
     __shared__ float2 Lf[MIXED && (SS || GRID) ? TPB : 1];
-    // 2^(j/64) for the FP64 exponentials (read after the first staging barrier)
-    __shared__ double Ltab[EXP_TAB];
-    if constexpr (!MIXED && (SS || KER == KY)) exp_table(Ltab, threadIdx.x);
+    // the FP64 exponentials' or sine's table (read after the first staging barrier)
+    __shared__ alignas(16) double Ltab[KER == KSR ? 2 * SIN_TAB : EXP_TAB];
+    if constexpr (KER == KSR) sin_table(Ltab, threadIdx.x, TPB);
+    else if constexpr (!MIXED && (SS || KER == KY || KER == KRY || KER == KUS)) exp_table(Ltab, threadIdx.x);
     if (!A.persistent) {
         const Tile tile = A.tiles[blockIdx.x];
         if (tile.z == 0) return;  // padding tile (uniform across the block)
@@ -1293,13 +1280,13 @@ __device__ __forceinline__ double group_sum64(double v)
 }
 
 template <int KER, bool SS, int TPT, int G, int NW>
-__global__ __launch_bounds__(64 * NW) void k_near_sym64(SymArgs A)
+__global__ __launch_bounds__(64 * NW, 4) void k_near_sym64(SymArgs A)
 {
     constexpr int NT = 64 * NW;
     __shared__ double4 Ls[NT];          // x, y, z and the source's a (q w or q)
     __shared__ double2 Lw[SS ? NT : 1]; // the source's w and its charge as a target
     __shared__ double Lc[NW][NT];       // per wave: the sources' sums
-    __shared__ double Ltab[EXP_TAB];     // 2^(j/64) for exp_nonpos
+    __shared__ double Ltab[EXP_TAB];     // 2^(j/256) for exp_neg
     const SymItem it = A.items[blockIdx.x];
     const bool check = A.ctr[blockIdx.x].w < 0.0;
     constexpr int NG = 64 / G;
@@ -1374,13 +1361,13 @@ __global__ __launch_bounds__(64 * NW) void k_near_sym64(SymArgs A)
                                 acc[k] = fma(S.w, ir, acc[k]);
                                 if constexpr (TWO) c = fma(Ta[k], ir, c);
                             } else {
-                                const double e = exp_nonpos(-r2 * kp.inv_a2, Ltab);
+                                const double e = exp_neg(r2, kp.eg, Ltab);
                                 acc[k] = fma(fma(Tnq[k] * sw, e, S.w), ir, acc[k]);
                                 if constexpr (TWO) c = fma(fma(-sq * Tw[k], e, Ta[k]), ir, c);
                             }
                         } else if constexpr (KER == KY) {
                             const double ir = rsq64(r2);
-                            double e = exp_nonpos(-kp.p0 * (r2 * ir), Ltab) * ir;
+                            double e = exp_neg(r2 * ir, kp.ek, Ltab) * ir;
                             if constexpr (CHECK) e = r2 > 0.0 ? e : 0.0;
                             if constexpr (!SS) {
                                 acc[k] = fma(S.w, e, acc[k]);

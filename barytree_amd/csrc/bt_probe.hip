@@ -8,13 +8,15 @@
 // counters) by these costs gives the time the VALU needs to issue them:
 // the attainable ceiling of that kernel's instruction mix.
 //
-// Also: the FP64 reciprocal square root of the pair kernels (bt_rsq.h)
-// evaluated on given inputs, for the accuracy test of that function.
+// Also: the FP64 reciprocal square root, exponential and sine of the pair
+// kernels (bt_rsq.h, bt_exp.h) evaluated on given inputs, for the accuracy
+// tests of those functions.
 //
 // Measurement tooling for the benchmark: built into its own library
 // (libbt_probe.so), not into the drop-in libBaryTree_gpu.so.
 #include <hip/hip_runtime.h>
 
+#include "bt_exp.h"
 #include "bt_rsq.h"
 
 namespace btk {
@@ -123,6 +125,36 @@ __global__ void k_rsq64_eval(int n, const double *x, double *y)
     if (i < n) y[i] = rsq64(x[i]);
 }
 
+// y[i] = e^{-k x[i]} (which 0) or sin(k x[i]) (which 1) by the table forms
+__global__ void k_table_eval(int which, double k, ExpRate ex, SinRate sr, int n, const double *x, double *y)
+{
+    __shared__ alignas(16) double tab[2 * SIN_TAB];
+    if (which == 0) exp_table(tab, threadIdx.x);
+    else sin_table(tab, threadIdx.x, 256);
+    __syncthreads();
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) y[i] = which == 0 ? exp_neg(x[i], ex, tab) : sin_kr(x[i], k, sr, tab);
+}
+
+// f(n, device x, device y) on host arrays of n values
+template <class F> int eval_on_device(const double *x, double *y, int n, F f)
+{
+    if (!x || !y || n <= 0) return -1;
+    double *dx = nullptr, *dy = nullptr;
+    const size_t bytes = (size_t)n * sizeof(double);
+    hipError_t e = hipMalloc(&dx, bytes);
+    if (e == hipSuccess) e = hipMalloc(&dy, bytes);
+    if (e == hipSuccess) e = hipMemcpy(dx, x, bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        f(n, dx, dy);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(y, dy, bytes, hipMemcpyDeviceToHost);
+    if (dx) (void)hipFree(dx);
+    if (dy) (void)hipFree(dy);
+    return e == hipSuccess ? 0 : -1;
+}
+
 }  // namespace btk
 
 // ns per wave instruction and SIMD of each kind on the current GPU; returns
@@ -138,18 +170,19 @@ extern "C" int bt_probe_valu(double *ns_per_instr, int n)
 // returns 0, or -1 on a HIP error or bad arguments.
 extern "C" int bt_probe_rsq64(const double *x, double *y, int n)
 {
-    if (!x || !y || n <= 0) return -1;
-    double *dx = nullptr, *dy = nullptr;
-    const size_t bytes = (size_t)n * sizeof(double);
-    hipError_t e = hipMalloc(&dx, bytes);
-    if (e == hipSuccess) e = hipMalloc(&dy, bytes);
-    if (e == hipSuccess) e = hipMemcpy(dx, x, bytes, hipMemcpyHostToDevice);
-    if (e == hipSuccess) {
-        btk::k_rsq64_eval<<<(n + 255) / 256, 256>>>(n, dx, dy);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpy(y, dy, bytes, hipMemcpyDeviceToHost);
-    if (dx) (void)hipFree(dx);
-    if (dy) (void)hipFree(dy);
-    return e == hipSuccess ? 0 : -1;
+    return btk::eval_on_device(x, y, n, [](int m, const double *dx, double *dy) {
+        btk::k_rsq64_eval<<<(m + 255) / 256, 256>>>(m, dx, dy);
+    });
+}
+
+// y[i] = e^{-k x[i]} (which 0) or sin(k x[i]) (which 1), x >= 0, by the pair
+// kernels' table forms (bt_exp.h) on the current GPU; returns 0, or -1.
+extern "C" int bt_probe_table64(int which, double k, const double *x, double *y, int n)
+{
+    if (which != 0 && which != 1) return -1;
+    const btk::ExpRate ex = btk::exp_rate(k);
+    const btk::SinRate sr = btk::sin_rate(k);
+    return btk::eval_on_device(x, y, n, [&](int m, const double *dx, double *dy) {
+        btk::k_table_eval<<<(m + 255) / 256, 256>>>(which, k, ex, sr, m, dx, dy);
+    });
 }

@@ -1236,6 +1236,7 @@ std::string Plan::finish_create(const PlanInput &in, bool host_only, double t2)
         kp_.c1 = prm.kp[0] * prm.kp[0];  // delta^2
     } else if (prm.kernel == K_SIN_OVER_R || prm.kernel == K_USER) {
         // k = kernel_params[0] (p0)
+        if (prm.kernel == K_SIN_OVER_R) kp_.sn = btk::sin_rate(prm.kp[0]);
     } else {
         if (prm.singularity == S_SUBTRACTION) {
             kp_.inv_a2 = 1.0 / (prm.kp[0] * prm.kp[0]);
@@ -1246,6 +1247,8 @@ std::string Plan::finish_create(const PlanInput &in, bool host_only, double t2)
         kp_.ss_param = 2.0 * M_PI * prm.kp[0] * prm.kp[0];
     }
     if (prm.singularity != S_SUBTRACTION) kp_.ss_param = 0.0;
+    kp_.ek = btk::exp_rate(prm.kp[0]);
+    if (kp_.inv_a2 != 0.0) kp_.eg = btk::exp_rate(1.0L / ((long double)prm.kp[0] * prm.kp[0]));
 
     // the particles and the target order are on the device already
     // (device_trees); the work lists and tables follow

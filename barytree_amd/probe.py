@@ -24,6 +24,7 @@ def _load():
         _lib = ctypes.CDLL(PROBE_LIB)
         _lib.bt_probe_valu.restype = ctypes.c_int
         _lib.bt_probe_rsq64.restype = ctypes.c_int
+        _lib.bt_probe_table64.restype = ctypes.c_int
     return _lib
 
 
@@ -35,6 +36,26 @@ def rsq64(x):
     if _load().bt_probe_rsq64(x.ctypes.data_as(dp), y.ctypes.data_as(dp), ctypes.c_int(len(x))) != 0:
         raise RuntimeError("bt_probe_rsq64 failed")
     return y
+
+
+def _table64(which, k, x):
+    x = np.ascontiguousarray(x, dtype=np.float64)
+    y = np.zeros_like(x)
+    dp = ctypes.POINTER(ctypes.c_double)
+    if _load().bt_probe_table64(ctypes.c_int(which), ctypes.c_double(k), x.ctypes.data_as(dp),
+                                y.ctypes.data_as(dp), ctypes.c_int(len(x))) != 0:
+        raise RuntimeError("bt_probe_table64 failed")
+    return y
+
+
+def exp_neg(k, x):
+    """e^{-k x}, x >= 0, by the pair kernels' FP64 table form (csrc/bt_exp.h)."""
+    return _table64(0, k, x)
+
+
+def sin_kr(k, x):
+    """sin(k x), x >= 0, by the pair kernels' FP64 table form (csrc/bt_exp.h)."""
+    return _table64(1, k, x)
 
 
 def probe_valu():
