@@ -56,34 +56,31 @@ constexpr int OFF_W4 = OFF_B3 + MLP_H;
 constexpr int OFF_B4 = OFF_W4 + MLP_OUT * MLP_H;
 constexpr int MLP_PARAMS = OFF_B4 + MLP_OUT;
 
-// Buffers of a batch of b samples (device, feature-major [f][b]): a0 the
-// normalised inputs [8][b], a1..a3 the layer outputs [64][b], d1..d3 the
-// pre-activation gradients [64][b], dz the logits and then their gradients
-// [10][b], loss the per-sample losses [b].
-struct TrainBufs {
-    float *a0, *a1, *a2, *a3, *d1, *d2, *d3, *dz, *loss;
-};
-
-// Inference on x[n][8] raw features, normalised as (x - mean) * scale (tb
-// sized for n samples): logits[n][10] (optional) and degree[n] (optional).
+// Inference on x[n][8] raw features, normalised as (x - mean) * scale:
+// logits[n][10] (optional) and degree[n] (optional).
 // The degree is 3+k for the largest k with sigmoid(logit_k) >= delta (the
 // model gives at least probability delta that degree 2+k is not enough),
 // else 2.
 hipError_t launch_mlp_infer(const float *params, const float *mean, const float *scale, int n,
-                            const float *x, float delta, float *logits, int *degree,
-                            const TrainBufs &tb, hipStream_t st);
+                            const float *x, float delta, float *logits, int *degree, hipStream_t st);
 
-// Training pass over one batch of b samples x[idx[j]] (idx may be null: j):
-// forward, loss, backward into tb.  The loss is the batch mean of
-// sum_k softplus(z_k) - y_k z_k with y_k = [label > 2+k].
-hipError_t launch_mlp_fwdbwd(const float *params, const float *mean, const float *scale,
-                             const float *x, const int *labels, const int *idx, int b,
-                             const TrainBufs &tb, hipStream_t st);
-// Weight gradients from the buffers of launch_mlp_fwdbwd: grad has the
-// parameter layout; dW = D^T A and db = sum over the batch, in batch order.
-hipError_t launch_mlp_wgrad(const TrainBufs &tb, int b, float *grad, hipStream_t st);
-// Adam step t (1-based) on n parameters.
-hipError_t launch_adam(float *params, const float *grad, float *m, float *v, int n, float lr,
-                       float beta1, float beta2, float eps, int t, hipStream_t st);
+// Pass over one batch of b samples x[idx[j]] (idx may be null: j): forward,
+// loss, backward.  The loss is the batch mean of
+// sum_k softplus(z_k) - y_k z_k with y_k = [label > 2+k].  Block k of
+// mlp_parts(b) writes the gradient of its samples' share to part[k] (rows of
+// MLP_PARAMS in the parameter layout) and the sum of its samples' losses to
+// loss[k].  Tiles of MLP_TILE samples, at most MLP_PARTS blocks.
+constexpr int MLP_TILE = 32, MLP_PARTS = 256;
+constexpr int mlp_parts(int b)
+{
+    return b <= 0 ? 0 : (b - 1) / MLP_TILE + 1 < MLP_PARTS ? (b - 1) / MLP_TILE + 1 : MLP_PARTS;
+}
+hipError_t launch_mlp_grad(const float *params, const float *mean, const float *scale, const float *x,
+                           const int *labels, const int *idx, int b, float *part, double *loss, hipStream_t st);
+// grad = the sum of nparts rows, in a fixed order.
+hipError_t launch_mlp_sum(const float *part, int nparts, float *grad, hipStream_t st);
+// Adam step t (1-based) with that sum.
+hipError_t launch_mlp_adam(const float *part, int nparts, float *params, float *m, float *v, float lr,
+                           float beta1, float beta2, float eps, int t, hipStream_t st);
 
 }  // namespace btl

@@ -1,10 +1,9 @@
 // bt_learn.hip -- gfx950 kernels of the learned degree selection:
 //   k_label            : minimal degree of a far-field pair (FP64, one block per pair)
-//   k_input, k_dense   : MLP forward, one layer per launch (FP32, LDS-tiled)
-//   k_loss, k_dense_t  : loss, output gradient and backward through a layer
-//   k_mlp_wgrad        : weight gradients D^T A as LDS-tiled products
-//   k_decide           : degrees from the logits
-//   k_adam             : Adam update
+//   k_mlp_infer        : MLP forward and degrees from the logits (FP32)
+//   k_mlp_grad         : forward, loss, backward and partial weight gradients
+//   k_mlp_sum          : the partial gradients' sum
+//   k_mlp_adam         : the sum and the Adam update
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -243,177 +242,316 @@ __global__ __launch_bounds__(LTPB) void k_label(LabelArgs A)
 }
 
 // ---------------------------------------------------------------------
-// MLP.  Activations are feature-major: H[f][b] for feature f of sample b of
-// a batch of nb samples.  A layer is a product with the (<= 64 x 64) weight
-// matrix held in LDS: a block covers all outputs for 64 samples; thread t
-// takes sample column t % 64 and 16 consecutive output rows, so every lane
-// of a wave reads the same weight (an LDS broadcast) and its own sample.
+// MLP, FP32 on the matrix cores (v_mfma_f32_16x16x4f32: FP32 operands,
+// products and sums).  A block of 4 waves takes tiles of MS = 32 samples;
+// activations and gradients live in LDS feature-major, H[f][s] with rows of
+// MSP = 33 floats, and the weights in registers: wave w owns output rows
+// 16w .. 16w+15 of every 64-wide product and keeps their weights (and the
+// transposed ones of the backward pass) for all its tiles.  Lane l holds
+//   A[l%16][k], B[k][l%16] for k = KQ (l/16) + step,  KQ = K/4,
+//   D[4 (l/16) + v][l%16], v = 0..3
+// (any assignment of k to lanes and steps serves, as long as A and B agree:
+// this one makes a lane's weights consecutive in memory, and puts the four
+// lane groups' rows of H in different LDS banks).
+//
+// The whole pass over a batch -- normalisation, three hidden layers, output,
+// loss, backward and the weight gradients of the block's samples, kept in
+// the accumulators over its tiles -- is one launch; the blocks' partial
+// gradients are added in block order by the launch that applies Adam.  A
+// training step is bound by latency (4096 samples need 2.3e8 flops): 14
+// launches, four of them weight gradients on at most 20 blocks (174 us each),
+// and a copy of the losses after each step took 1.03 ms a step at batch 4096;
+// two launches (16 and 4 us) and no copy take 21 us (24 steps: 24.7 -> 2.3 ms with
+// the call's own host work).
 // ---------------------------------------------------------------------
-constexpr int MTPB = 256;
-constexpr int CS = 64;  // samples per block
-constexpr int RPT = 16; // output rows per thread
+constexpr int MTPB = 256, MWAVES = 4;
+constexpr int MS = MLP_TILE;   // samples per tile
+constexpr int MSP = MS + 1;    // 16 MSP = 16 mod 64 banks
+constexpr int MCT = MS / 16;   // column tiles of 16 samples
+static_assert(MLP_H == 16 * MWAVES && MS == 32 && MLP_OUT <= 16 && MLP_IN == 8, "MLP layout");
+
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + expf(-z)); }
 
-// Hout[i][b] = act(bias[i] + sum_j W[i][j] Hin[j][b]), i < fout, j < fin
-__global__ __launch_bounds__(MTPB) void k_dense(const float *W, const float *bias, const float *Hin, int fin,
-                                               int fout, int nb, float *Hout, int relu)
+// this lane's weights of rows r0 .. r0+15 of W (rows x K, row major); rows
+// outside give zeros
+template <int K>
+__device__ __forceinline__ void load_rows(const float *W, int r0, int rows, int lane, float (&a)[K / 4])
 {
-    __shared__ float Lw[MLP_H * MLP_H + MLP_H];
-    __shared__ float Lh[MLP_H][CS + 1];
-    const int tid = threadIdx.x, c = tid % CS, r0 = (tid / CS) * RPT;
-    const int b0 = blockIdx.x * CS;
-    for (int e = tid; e < fout * fin; e += MTPB) Lw[e] = W[e];
-    for (int e = tid; e < fout; e += MTPB) Lw[MLP_H * MLP_H + e] = bias[e];
-    for (int e = tid; e < fin * CS; e += MTPB) {
-        const int j = e / CS, cc = e % CS;
-        Lh[j][cc] = b0 + cc < nb ? Hin[(size_t)j * nb + b0 + cc] : 0.0f;
-    }
-    __syncthreads();
-    if (r0 >= fout) return;
-    float acc[RPT];
+    const int r = r0 + (lane & 15);
+    const float *p = W + (size_t)(r < rows ? r : 0) * K + (K / 4) * (lane >> 4);
 #pragma unroll
-    for (int r = 0; r < RPT; r++) acc[r] = r0 + r < fout ? Lw[MLP_H * MLP_H + r0 + r] : 0.0f;
-    for (int j = 0; j < fin; j++) {
-        const float h = Lh[j][c];
+    for (int s = 0; s < K / 4; s++) a[s] = r < rows ? p[s] : 0.0f;
+}
+
+// rows c0 .. c0+15 of W^T, W being rows x cols row major, K >= rows
+template <int K>
+__device__ __forceinline__ void load_cols(const float *W, int c0, int rows, int cols, int lane, float (&a)[K / 4])
+{
+    const int c = c0 + (lane & 15);
 #pragma unroll
-        for (int r = 0; r < RPT; r++)
-            if (r0 + r < fout) acc[r] = fmaf(Lw[(r0 + r) * fin + j], h, acc[r]);
-    }
-    if (b0 + c < nb) {
-#pragma unroll
-        for (int r = 0; r < RPT; r++)
-            if (r0 + r < fout) Hout[(size_t)(r0 + r) * nb + b0 + c] = relu ? fmaxf(acc[r], 0.0f) : acc[r];
+    for (int s = 0; s < K / 4; s++) {
+        const int r = (K / 4) * (lane >> 4) + s;
+        a[s] = r < rows ? W[(size_t)r * cols + c] : 0.0f;
     }
 }
 
-// Backward through a layer: G[j][b] = [A[j][b] > 0] * sum_i W[i][j] D[i][b]
-// (W is fout x fin; j < fin, i < fout)
-__global__ __launch_bounds__(MTPB) void k_dense_t(const float *W, const float *D, const float *A, int fin,
-                                                 int fout, int nb, float *G)
+// D += A B for columns 16 ct .. of H (K rows)
+template <int K>
+__device__ __forceinline__ v4f product(const float (&a)[K / 4], const float *H, int ct, int lane, v4f d)
 {
-    __shared__ float Lw[MLP_H * MLP_H];
-    __shared__ float Ld[MLP_H][CS + 1];
-    const int tid = threadIdx.x, c = tid % CS, r0 = (tid / CS) * RPT;
-    const int b0 = blockIdx.x * CS;
-    for (int e = tid; e < fout * fin; e += MTPB) Lw[e] = W[e];
-    for (int e = tid; e < fout * CS; e += MTPB) {
-        const int i = e / CS, cc = e % CS;
-        Ld[i][cc] = b0 + cc < nb ? D[(size_t)i * nb + b0 + cc] : 0.0f;
+    const float *h = H + (K / 4) * (lane >> 4) * MSP + 16 * ct + (lane & 15);
+#pragma unroll
+    for (int s = 0; s < K / 4; s++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], h[s * MSP], d, 0, 0, 0);
+    return d;
+}
+
+// D += X[16 xr ..][samples] Y[16 yr ..][samples]^T over the tile's samples
+__device__ __forceinline__ v4f outer(const float *X, int xr, const float *Y, int yr, int lane, v4f d)
+{
+    const int o = (lane & 15) * MSP + (MS / 4) * (lane >> 4);
+    const float *x = X + 16 * xr * MSP + o, *y = Y + 16 * yr * MSP + o;
+#pragma unroll
+    for (int s = 0; s < MS / 4; s++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], y[s], d, 0, 0, 0);
+    return d;
+}
+
+// the hidden layers' and the output's weights and biases of a wave
+struct MlpForward {
+    float w1[MLP_IN / 4], w2[MLP_H / 4], w3[MLP_H / 4], w4[MLP_H / 4];
+    v4f b1, b2, b3, b4;
+    __device__ __forceinline__ void load(const float *prm, int wv, int lane)
+    {
+        load_rows<MLP_IN>(prm + OFF_W1, 16 * wv, MLP_H, lane, w1);
+        load_rows<MLP_H>(prm + OFF_W2, 16 * wv, MLP_H, lane, w2);
+        load_rows<MLP_H>(prm + OFF_W3, 16 * wv, MLP_H, lane, w3);
+        load_rows<MLP_H>(prm + OFF_W4, 0, MLP_OUT, lane, w4);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int r = 4 * (lane >> 4) + v;
+            b1[v] = prm[OFF_B1 + 16 * wv + r];
+            b2[v] = prm[OFF_B2 + 16 * wv + r];
+            b3[v] = prm[OFF_B3 + 16 * wv + r];
+            b4[v] = r < MLP_OUT ? prm[OFF_B4 + r] : 0.0f;
+        }
     }
-    __syncthreads();
-    if (r0 >= fin) return;
-    float acc[RPT];
+};
+
+// rows 16 wv .. of Hout = relu(A Hin + bias)
+template <int K>
+__device__ __forceinline__ void hidden(const float (&a)[K / 4], v4f bias, const float *Hin, float *Hout, int wv,
+                                       int lane)
+{
 #pragma unroll
-    for (int r = 0; r < RPT; r++) acc[r] = 0.0f;
-    for (int i = 0; i < fout; i++) {
-        const float d = Ld[i][c];
+    for (int ct = 0; ct < MCT; ct++) {
+        const v4f d = product<K>(a, Hin, ct, lane, bias);
 #pragma unroll
-        for (int r = 0; r < RPT; r++)
-            if (r0 + r < fin) acc[r] = fmaf(Lw[i * fin + r0 + r], d, acc[r]);
+        for (int v = 0; v < 4; v++)
+            Hout[(16 * wv + 4 * (lane >> 4) + v) * MSP + 16 * ct + (lane & 15)] = fmaxf(d[v], 0.0f);
     }
-    if (b0 + c < nb) {
+}
+
+// rows 16 wv .. of G = [H > 0] (A D)
+template <int K>
+__device__ __forceinline__ void backward(const float (&a)[K / 4], const float *D, const float *H, float *G, int wv,
+                                         int lane)
+{
 #pragma unroll
-        for (int r = 0; r < RPT; r++) {
-            if (r0 + r >= fin) continue;
-            const size_t o = (size_t)(r0 + r) * nb + b0 + c;
-            G[o] = A[o] > 0.0f ? acc[r] : 0.0f;
+    for (int ct = 0; ct < MCT; ct++) {
+        const v4f d = product<K>(a, D, ct, lane, v4f{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int o = (16 * wv + 4 * (lane >> 4) + v) * MSP + 16 * ct + (lane & 15);
+            G[o] = H[o] > 0.0f ? d[v] : 0.0f;
         }
     }
 }
 
-// Normalised inputs: A0[f][b] = (x[s][f] - mean[f]) * scale[f], s = idx[b] (or b)
-__global__ void k_input(const float *x, const int *idx, const float *mean, const float *scale, int nb,
-                        float *A0)
+// normalised inputs of the tile's samples, H0[f][s] (zero past the batch):
+// thread 8 s + f
+__device__ __forceinline__ void inputs(const float *x, const int *idx, const float *mean, const float *scale, int s0,
+                                       int nb, float *H0)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    const size_t s = idx ? (size_t)idx[b] : (size_t)b;
-#pragma unroll
-    for (int f = 0; f < MLP_IN; f++) A0[(size_t)f * nb + b] = (x[s * MLP_IN + f] - mean[f]) * scale[f];
+    const int f = threadIdx.x & (MLP_IN - 1), s = threadIdx.x / MLP_IN;
+    const int b = s0 + s;
+    float v = 0.0f;
+    if (b < nb) v = (x[(size_t)(idx ? idx[b] : b) * MLP_IN + f] - mean[f]) * scale[f];
+    H0[f * MSP + s] = v;
 }
 
-// Loss and output gradient, in place: Z[k][b] (logits) -> dZ[k][b]
-__global__ void k_loss(const int *labels, const int *idx, int nb, float *Z, float *loss)
+__global__ __launch_bounds__(MTPB) void k_mlp_grad(const float *prm, const float *mean, const float *scale,
+                                                   const float *x, const int *labels, const int *idx, int nb,
+                                                   float *part, double *loss)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    const int lab = labels[idx ? idx[b] : b];
+    __shared__ float H0[16 * MSP], H1[MLP_H * MSP], H2[MLP_H * MSP], H3[MLP_H * MSP];
+    __shared__ float D1[MLP_H * MSP], D2[MLP_H * MSP], D3[MLP_H * MSP], DZ[16 * MSP];
+    __shared__ double Ll[2 * 64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const float inv_b = 1.0f / (float)nb;
-    float l = 0.0f;
+    MlpForward w;
+    w.load(prm, wv, lane);
+    float t2[MLP_H / 4], t3[MLP_H / 4], t4[16 / 4];
+    load_cols<MLP_H>(prm + OFF_W2, 16 * wv, MLP_H, MLP_H, lane, t2);
+    load_cols<MLP_H>(prm + OFF_W3, 16 * wv, MLP_H, MLP_H, lane, t3);
+    load_cols<16>(prm + OFF_W4, 16 * wv, MLP_OUT, MLP_H, lane, t4);
+    // rows 8.. of H0 are only read by the gradient of W1, whose columns 8..
+    // are not stored; row 8 holds ones: column 8 is the bias gradient
+    for (int e = tid; e < 8 * MSP; e += MTPB) H0[8 * MSP + e] = e < MSP ? 1.0f : 0.0f;
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    v4f g1 = zero, g2[4], g3[4], g4 = zero;
 #pragma unroll
-    for (int k = 0; k < MLP_OUT; k++) {
-        const size_t o = (size_t)k * nb + b;
-        const float z = Z[o];
-        const float y = lab > LABEL_DMIN + k ? 1.0f : 0.0f;
-        l += fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))) - y * z;
-        Z[o] = (sigmoidf_(z) - y) * inv_b;
-    }
-    loss[b] = l;
-}
-
-// Degrees (and logits in sample-major order) from Z[k][b]
-__global__ void k_decide(const float *Z, int nb, float delta, float *logits, int *degree)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    int deg = LABEL_DMIN;
+    for (int c = 0; c < 4; c++) { g2[c] = zero; g3[c] = zero; }
+    // bias gradients: thread i of D2's rows, then D3's, then DZ's
+    float gb = 0.0f;
+    double lsum = 0.0;
+    for (int s0 = blockIdx.x * MS; s0 < nb; s0 += gridDim.x * MS) {
+        __syncthreads();  // the previous tile has been read
+        inputs(x, idx, mean, scale, s0, nb, H0);
+        __syncthreads();
+        hidden<MLP_IN>(w.w1, w.b1, H0, H1, wv, lane);
+        __syncthreads();
+        hidden<MLP_H>(w.w2, w.b2, H1, H2, wv, lane);
+        __syncthreads();
+        hidden<MLP_H>(w.w3, w.b3, H2, H3, wv, lane);
+        __syncthreads();
+        if (wv < MCT) {
+            // logits of column tile wv, loss and output gradient
+            const int s = 16 * wv + (lane & 15), b = s0 + s;
+            const bool on = b < nb;
+            const int lab = on ? labels[idx ? idx[b] : b] : 0;
+            const v4f z4 = product<MLP_H>(w.w4, H3, wv, lane, w.b4);
+            float l = 0.0f;
 #pragma unroll
-    for (int k = 0; k < MLP_OUT; k++) {
-        const float z = Z[(size_t)k * nb + b];
-        if (logits) logits[(size_t)b * MLP_OUT + k] = z;
-        if (sigmoidf_(z) >= delta) deg = LABEL_DMIN + 1 + k;
-    }
-    if (degree) degree[b] = deg;
-}
-
-hipError_t forward_pass(const float *prm, const float *mean, const float *scale, const float *x,
-                        const int *idx, int nb, const TrainBufs &tb, hipStream_t st)
-{
-    const int g1 = (nb + 255) / 256, gc = (nb + CS - 1) / CS;
-    k_input<<<g1, 256, 0, st>>>(x, idx, mean, scale, nb, tb.a0);
-    k_dense<<<gc, MTPB, 0, st>>>(prm + OFF_W1, prm + OFF_B1, tb.a0, MLP_IN, MLP_H, nb, tb.a1, 1);
-    k_dense<<<gc, MTPB, 0, st>>>(prm + OFF_W2, prm + OFF_B2, tb.a1, MLP_H, MLP_H, nb, tb.a2, 1);
-    k_dense<<<gc, MTPB, 0, st>>>(prm + OFF_W3, prm + OFF_B3, tb.a2, MLP_H, MLP_H, nb, tb.a3, 1);
-    k_dense<<<gc, MTPB, 0, st>>>(prm + OFF_W4, prm + OFF_B4, tb.a3, MLP_H, MLP_OUT, nb, tb.dz, 0);
-    return hipGetLastError();
-}
-
-// out[i][j] = sum_b D[i][b] A[j][b] (j < J), bias[i] = sum_b D[i][b]
-// (column J); a 16x16 output tile per block, batch chunks of 64 in LDS.
-constexpr int WT = 16, WC = 64;
-__global__ __launch_bounds__(256) void k_mlp_wgrad(const float *D, const float *A, int I, int J, int nb,
-                                                   float *outW, float *outB)
-{
-    __shared__ float Ld[WT][WC + 1], La[WT][WC + 1];
-    const int tid = threadIdx.x, ti = tid / WT, tj = tid % WT;
-    const int i0 = blockIdx.x * WT, j0 = blockIdx.y * WT;
-    float acc = 0.0f;
-    for (int c0 = 0; c0 < nb; c0 += WC) {
-        for (int e = tid; e < WT * WC; e += 256) {
-            const int r = e / WC, c = e % WC, b = c0 + c;
-            const int i = i0 + r, jj = j0 + r;
-            Ld[r][c] = (i < I && b < nb) ? D[(size_t)i * nb + b] : 0.0f;
-            La[r][c] = b < nb ? (jj < J ? A[(size_t)jj * nb + b] : (jj == J ? 1.0f : 0.0f)) : 0.0f;
+            for (int v = 0; v < 4; v++) {
+                const int k = 4 * (lane >> 4) + v;
+                const float z = z4[v], y = lab > LABEL_DMIN + k ? 1.0f : 0.0f;
+                const bool use = on && k < MLP_OUT;
+                if (use) l += fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))) - y * z;
+                DZ[k * MSP + s] = use ? (sigmoidf_(z) - y) * inv_b : 0.0f;
+            }
+            lsum += (double)l;
         }
         __syncthreads();
-#pragma unroll 8
-        for (int c = 0; c < WC; c++) acc = fmaf(Ld[ti][c], La[tj][c], acc);
+        backward<16>(t4, DZ, H3, D3, wv, lane);
         __syncthreads();
+        backward<MLP_H>(t3, D3, H2, D2, wv, lane);
+        __syncthreads();
+        backward<MLP_H>(t2, D2, H1, D1, wv, lane);
+        __syncthreads();
+        g1 = outer(D1, wv, H0, 0, lane, g1);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            g2[c] = outer(D2, wv, H1, c, lane, g2[c]);
+            g3[c] = outer(D3, wv, H2, c, lane, g3[c]);
+        }
+        g4 = outer(DZ, 0, H3, wv, lane, g4);
+        const float *d = tid < MLP_H ? D2 + tid * MSP
+                       : tid < 2 * MLP_H ? D3 + (tid - MLP_H) * MSP
+                       : tid < 2 * MLP_H + MLP_OUT ? DZ + (tid - 2 * MLP_H) * MSP : nullptr;
+        if (d)
+            for (int s = 0; s < MS; s++) gb += d[s];
     }
-    const int i = i0 + ti, jj = j0 + tj;
-    if (i < I) {
-        if (jj < J) outW[(size_t)i * J + jj] = acc;
-        else if (jj == J) outB[i] = acc;
+    // this block's row of partial gradients
+    float *o = part + (size_t)blockIdx.x * MLP_PARAMS;
+    const int col = lane & 15;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int r = 4 * (lane >> 4) + v, i = 16 * wv + r;
+        if (col < MLP_IN) o[OFF_W1 + i * MLP_IN + col] = g1[v];
+        else if (col == MLP_IN) o[OFF_B1 + i] = g1[v];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            o[OFF_W2 + i * MLP_H + 16 * c + col] = g2[c][v];
+            o[OFF_W3 + i * MLP_H + 16 * c + col] = g3[c][v];
+        }
+        if (r < MLP_OUT) o[OFF_W4 + r * MLP_H + 16 * wv + col] = g4[v];
+    }
+    if (tid < MLP_H) o[OFF_B2 + tid] = gb;
+    else if (tid < 2 * MLP_H) o[OFF_B3 + tid - MLP_H] = gb;
+    else if (tid < 2 * MLP_H + MLP_OUT) o[OFF_B4 + tid - 2 * MLP_H] = gb;
+    if (wv < MCT) Ll[tid] = lsum;
+    __syncthreads();
+    if (tid == 0) {
+        double s = 0.0;
+        for (int k = 0; k < 64 * MCT; k++) s += Ll[k];
+        loss[blockIdx.x] = s;
     }
 }
 
-__global__ void k_adam(float *p, const float *g, float *m, float *v, int n, float lr, float b1, float b2,
-                       float eps, float c1, float c2)
+// Logits (sample major, optional) and degrees (optional) of n samples.
+__global__ __launch_bounds__(MTPB) void k_mlp_infer(const float *prm, const float *mean, const float *scale,
+                                                    const float *x, int n, float delta, float *logits, int *degree)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
+    __shared__ float H0[MLP_IN * MSP], HA[MLP_H * MSP], HB[MLP_H * MSP], Z[MS * MLP_OUT];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    MlpForward w;
+    w.load(prm, wv, lane);
+    for (int s0 = blockIdx.x * MS; s0 < n; s0 += gridDim.x * MS) {
+        __syncthreads();
+        inputs(x, nullptr, mean, scale, s0, n, H0);
+        __syncthreads();
+        hidden<MLP_IN>(w.w1, w.b1, H0, HA, wv, lane);
+        __syncthreads();
+        hidden<MLP_H>(w.w2, w.b2, HA, HB, wv, lane);
+        __syncthreads();
+        hidden<MLP_H>(w.w3, w.b3, HB, HA, wv, lane);
+        __syncthreads();
+        if (wv < MCT) {
+            const v4f z4 = product<MLP_H>(w.w4, HA, wv, lane, w.b4);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int k = 4 * (lane >> 4) + v;
+                if (k < MLP_OUT) Z[(16 * wv + (lane & 15)) * MLP_OUT + k] = z4[v];
+            }
+        }
+        __syncthreads();
+        const int m = min(MS, n - s0);
+        if (logits)
+            for (int e = tid; e < m * MLP_OUT; e += MTPB) logits[(size_t)s0 * MLP_OUT + e] = Z[e];
+        if (degree && tid < m) {
+            int deg = LABEL_DMIN;
+#pragma unroll
+            for (int k = 0; k < MLP_OUT; k++)
+                if (sigmoidf_(Z[tid * MLP_OUT + k]) >= delta) deg = LABEL_DMIN + 1 + k;
+            degree[s0 + tid] = deg;
+        }
+    }
+}
+
+// The blocks' rows in block order, four runs of them side by side and then
+// in order: the gradient (grad) or one Adam step with it.
+constexpr int RPB = 64;  // parameters per block
+__device__ __forceinline__ bool reduced(const float *part, int nparts, int &i, float &g)
+{
+    __shared__ float L[4][RPB];
+    const int c = threadIdx.x % RPB, q = threadIdx.x / RPB;
+    i = blockIdx.x * RPB + c;
+    float s = 0.0f;
+    if (i < MLP_PARAMS) {
+        const int e = nparts * (q + 1) / 4;
+#pragma unroll 8
+        for (int k = nparts * q / 4; k < e; k++) s += part[(size_t)k * MLP_PARAMS + i];
+    }
+    L[q][c] = s;
+    __syncthreads();
+    g = ((L[0][c] + L[1][c]) + L[2][c]) + L[3][c];
+    return q == 0 && i < MLP_PARAMS;
+}
+
+__global__ __launch_bounds__(4 * RPB) void k_mlp_sum(const float *part, int nparts, float *grad)
+{
+    int i;
+    float g;
+    if (reduced(part, nparts, i, g)) grad[i] = g;
+}
+
+__global__ __launch_bounds__(4 * RPB) void k_mlp_adam(const float *part, int nparts, float *p, float *m, float *v,
+                                                      float lr, float b1, float b2, float eps, float c1, float c2)
+{
+    int i;
+    float gi;
+    if (!reduced(part, nparts, i, gi)) return;
     const float mi = b1 * m[i] + (1.0f - b1) * gi;
     const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
     m[i] = mi;
@@ -431,51 +569,35 @@ hipError_t launch_label(const LabelArgs &a, hipStream_t st)
 }
 
 hipError_t launch_mlp_infer(const float *params, const float *mean, const float *scale, int n,
-                            const float *x, float delta, float *logits, int *degree, const TrainBufs &tb,
-                            hipStream_t st)
+                            const float *x, float delta, float *logits, int *degree, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    hipError_t e = forward_pass(params, mean, scale, x, nullptr, n, tb, st);
-    if (e != hipSuccess) return e;
-    k_decide<<<(n + 255) / 256, 256, 0, st>>>(tb.dz, n, delta, logits, degree);
+    const int tiles = (n + MS - 1) / MS;
+    k_mlp_infer<<<tiles < 2048 ? tiles : 2048, MTPB, 0, st>>>(params, mean, scale, x, n, delta, logits, degree);
     return hipGetLastError();
 }
 
-hipError_t launch_mlp_fwdbwd(const float *params, const float *mean, const float *scale,
-                             const float *x, const int *labels, const int *idx, int b,
-                             const TrainBufs &tb, hipStream_t st)
+hipError_t launch_mlp_grad(const float *params, const float *mean, const float *scale, const float *x,
+                           const int *labels, const int *idx, int b, float *part, double *loss, hipStream_t st)
 {
     if (b <= 0) return hipSuccess;
-    hipError_t e = forward_pass(params, mean, scale, x, idx, b, tb, st);
-    if (e != hipSuccess) return e;
-    const int g1 = (b + 255) / 256, gc = (b + CS - 1) / CS;
-    k_loss<<<g1, 256, 0, st>>>(labels, idx, b, tb.dz, tb.loss);
-    k_dense_t<<<gc, MTPB, 0, st>>>(params + OFF_W4, tb.dz, tb.a3, MLP_H, MLP_OUT, b, tb.d3);
-    k_dense_t<<<gc, MTPB, 0, st>>>(params + OFF_W3, tb.d3, tb.a2, MLP_H, MLP_H, b, tb.d2);
-    k_dense_t<<<gc, MTPB, 0, st>>>(params + OFF_W2, tb.d2, tb.a1, MLP_H, MLP_H, b, tb.d1);
+    k_mlp_grad<<<mlp_parts(b), MTPB, 0, st>>>(params, mean, scale, x, labels, idx, b, part, loss);
     return hipGetLastError();
 }
 
-hipError_t launch_mlp_wgrad(const TrainBufs &tb, int b, float *grad, hipStream_t st)
+hipError_t launch_mlp_sum(const float *part, int nparts, float *grad, hipStream_t st)
 {
-    auto one = [&](const float *D, const float *A, int I, int J, int offW, int offB) {
-        dim3 g((I + WT - 1) / WT, (J + 1 + WT - 1) / WT);
-        k_mlp_wgrad<<<g, 256, 0, st>>>(D, A, I, J, b, grad + offW, grad + offB);
-    };
-    one(tb.d1, tb.a0, MLP_H, MLP_IN, OFF_W1, OFF_B1);
-    one(tb.d2, tb.a1, MLP_H, MLP_H, OFF_W2, OFF_B2);
-    one(tb.d3, tb.a2, MLP_H, MLP_H, OFF_W3, OFF_B3);
-    one(tb.dz, tb.a3, MLP_OUT, MLP_H, OFF_W4, OFF_B4);
+    k_mlp_sum<<<(MLP_PARAMS + RPB - 1) / RPB, 4 * RPB, 0, st>>>(part, nparts, grad);
     return hipGetLastError();
 }
 
-hipError_t launch_adam(float *params, const float *grad, float *m, float *v, int n, float lr,
-                       float beta1, float beta2, float eps, int t, hipStream_t st)
+hipError_t launch_mlp_adam(const float *part, int nparts, float *params, float *m, float *v, float lr,
+                           float beta1, float beta2, float eps, int t, hipStream_t st)
 {
-    if (n <= 0) return hipSuccess;
     const float c1 = 1.0f / (1.0f - powf(beta1, (float)t));
     const float c2 = 1.0f / (1.0f - powf(beta2, (float)t));
-    k_adam<<<(n + 255) / 256, 256, 0, st>>>(params, grad, m, v, n, lr, beta1, beta2, eps, c1, c2);
+    k_mlp_adam<<<(MLP_PARAMS + RPB - 1) / RPB, 4 * RPB, 0, st>>>(part, nparts, params, m, v, lr, beta1, beta2, eps,
+                                                                 c1, c2);
     return hipGetLastError();
 }
 

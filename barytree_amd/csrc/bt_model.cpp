@@ -45,17 +45,6 @@ struct DevBufs {
         if (e_ != hipSuccess) return std::string(#expr ": ") + hipGetErrorString(e_); \
     } while (0)
 
-bool alloc_train(DevBufs &db, int b, btl::TrainBufs &tb)
-{
-    const size_t H = (size_t)btl::MLP_H * b;
-    tb.a0 = db.get<float>((size_t)btl::MLP_IN * b);
-    tb.a1 = db.get<float>(H); tb.a2 = db.get<float>(H); tb.a3 = db.get<float>(H);
-    tb.d1 = db.get<float>(H); tb.d2 = db.get<float>(H); tb.d3 = db.get<float>(H);
-    tb.dz = db.get<float>((size_t)btl::MLP_OUT * b);
-    tb.loss = db.get<float>(b);
-    return tb.a0 && tb.a1 && tb.a2 && tb.a3 && tb.d1 && tb.d2 && tb.d3 && tb.dz && tb.loss;
-}
-
 }  // namespace
 
 void DegreeModel::init(unsigned long long seed)
@@ -184,21 +173,23 @@ std::string DegreeModel::gradient(int n, const float *x, const int *labels, std:
           *dsc = db.get<float>(btl::MLP_IN), *dx = db.get<float>((size_t)n * btl::MLP_IN),
           *dg = db.get<float>(btl::MLP_PARAMS);
     int *dl = db.get<int>(n);
-    btl::TrainBufs tb;
-    if (!dp || !dmu || !dsc || !dx || !dg || !dl || !alloc_train(db, n, tb)) return "hipMalloc failed";
+    const int np = btl::mlp_parts(n);
+    float *part = db.get<float>((size_t)np * btl::MLP_PARAMS);
+    double *dloss = db.get<double>(np);
+    if (!dp || !dmu || !dsc || !dx || !dg || !dl || !part || !dloss) return "hipMalloc failed";
     CHK(hipMemcpy(dp, params.data(), btl::MLP_PARAMS * sizeof(float), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dmu, mean, sizeof(mean), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dsc, scale, sizeof(scale), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dx, x, (size_t)n * btl::MLP_IN * sizeof(float), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dl, labels, n * sizeof(int), hipMemcpyHostToDevice));
-    CHK(btl::launch_mlp_fwdbwd(dp, dmu, dsc, dx, dl, nullptr, n, tb, nullptr));
-    CHK(btl::launch_mlp_wgrad(tb, n, dg, nullptr));
+    CHK(btl::launch_mlp_grad(dp, dmu, dsc, dx, dl, nullptr, n, part, dloss, nullptr));
+    CHK(btl::launch_mlp_sum(part, np, dg, nullptr));
     grad.assign(btl::MLP_PARAMS, 0.0f);
-    std::vector<float> ls(n);
+    std::vector<double> ls(np);
     CHK(hipMemcpy(grad.data(), dg, btl::MLP_PARAMS * sizeof(float), hipMemcpyDeviceToHost));
-    CHK(hipMemcpy(ls.data(), tb.loss, n * sizeof(float), hipMemcpyDeviceToHost));
+    CHK(hipMemcpy(ls.data(), dloss, np * sizeof(double), hipMemcpyDeviceToHost));
     double s = 0.0;
-    for (float v : ls) s += v;
+    for (double v : ls) s += v;
     loss = s / n;
     return "";
 }
@@ -213,12 +204,13 @@ std::string DegreeModel::train(int n, const float *x, const int *labels, int epo
     DevBufs db;
     float *dp = db.get<float>(btl::MLP_PARAMS), *dmu = db.get<float>(btl::MLP_IN),
           *dsc = db.get<float>(btl::MLP_IN), *dx = db.get<float>((size_t)n * btl::MLP_IN),
-          *dg = db.get<float>(btl::MLP_PARAMS), *dm = db.get<float>(btl::MLP_PARAMS),
-          *dv = db.get<float>(btl::MLP_PARAMS);
+          *dm = db.get<float>(btl::MLP_PARAMS), *dv = db.get<float>(btl::MLP_PARAMS);
     int *dl = db.get<int>(n), *didx = db.get<int>(n);
-    btl::TrainBufs tb;
-    if (!dp || !dmu || !dsc || !dx || !dg || !dm || !dv || !dl || !didx || !alloc_train(db, batch, tb))
-        return "hipMalloc failed";
+    const int nsteps = std::max(1, n / batch);  // full batches only
+    const int np = btl::mlp_parts(batch);
+    float *part = db.get<float>((size_t)np * btl::MLP_PARAMS);
+    double *dloss = db.get<double>((size_t)nsteps * np);  // one epoch's partial losses
+    if (!dp || !dmu || !dsc || !dx || !dm || !dv || !dl || !didx || !part || !dloss) return "hipMalloc failed";
     CHK(hipMemcpy(dp, params.data(), btl::MLP_PARAMS * sizeof(float), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dmu, mean, sizeof(mean), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dsc, scale, sizeof(scale), hipMemcpyHostToDevice));
@@ -229,23 +221,21 @@ std::string DegreeModel::train(int n, const float *x, const int *labels, int epo
     std::mt19937_64 rng(seed);
     std::vector<int> perm(n);
     std::iota(perm.begin(), perm.end(), 0);
-    std::vector<float> ls(batch);
+    std::vector<double> ls((size_t)nsteps * np);
     if (epoch_loss) epoch_loss->clear();
-    const int nsteps = n / batch;  // full batches only
     for (int ep = 0; ep < epochs; ep++) {
         std::shuffle(perm.begin(), perm.end(), rng);
         CHK(hipMemcpy(didx, perm.data(), n * sizeof(int), hipMemcpyHostToDevice));
-        double es = 0.0;
-        for (int k = 0; k < std::max(1, nsteps); k++) {
-            CHK(btl::launch_mlp_fwdbwd(dp, dmu, dsc, dx, dl, didx + (size_t)k * batch, batch, tb, nullptr));
-            CHK(btl::launch_mlp_wgrad(tb, batch, dg, nullptr));
-            CHK(btl::launch_adam(dp, dg, dm, dv, btl::MLP_PARAMS, lr, 0.9f, 0.999f, 1e-8f, ++steps, nullptr));
-            CHK(hipMemcpy(ls.data(), tb.loss, batch * sizeof(float), hipMemcpyDeviceToHost));
-            double s = 0.0;
-            for (float v : ls) s += v;
-            es += s / batch;
+        for (int k = 0; k < nsteps; k++) {
+            CHK(btl::launch_mlp_grad(dp, dmu, dsc, dx, dl, didx + (size_t)k * batch, batch, part,
+                                     dloss + (size_t)k * np, nullptr));
+            CHK(btl::launch_mlp_adam(part, np, dp, dm, dv, lr, 0.9f, 0.999f, 1e-8f, ++steps, nullptr));
         }
-        if (epoch_loss) epoch_loss->push_back((float)(es / std::max(1, nsteps)));
+        // the epoch's losses at its end: no step waits for the host
+        CHK(hipMemcpy(ls.data(), dloss, ls.size() * sizeof(double), hipMemcpyDeviceToHost));
+        double es = 0.0;
+        for (double v : ls) es += v / batch;
+        if (epoch_loss) epoch_loss->push_back((float)(es / nsteps));
     }
     CHK(hipMemcpy(params.data(), dp, btl::MLP_PARAMS * sizeof(float), hipMemcpyDeviceToHost));
     return "";
@@ -257,16 +247,14 @@ std::string DegreeModel::predict(int n, const float *x, float delta, int *degree
     if (!(delta > 0.0f && delta < 1.0f)) return "delta must lie in (0, 1)";
     if (n == 0) return "";
     if (!has_scaling()) return "model has no feature scaling (train it or set it first)";
-    // in chunks, so the activation buffers stay small
+    // in chunks, so the buffers stay small
     const int chunk = std::min(n, 1 << 18);
     DevBufs db;
     float *dp = db.get<float>(btl::MLP_PARAMS), *dmu = db.get<float>(btl::MLP_IN),
           *dsc = db.get<float>(btl::MLP_IN), *dx = db.get<float>((size_t)chunk * btl::MLP_IN);
     int *dd = db.get<int>(chunk);
     float *dz = logits ? db.get<float>((size_t)chunk * btl::MLP_OUT) : nullptr;
-    btl::TrainBufs tb;
-    if (!dp || !dmu || !dsc || !dx || !dd || (logits && !dz) || !alloc_train(db, chunk, tb))
-        return "hipMalloc failed";
+    if (!dp || !dmu || !dsc || !dx || !dd || (logits && !dz)) return "hipMalloc failed";
     CHK(hipMemcpy(dp, params.data(), btl::MLP_PARAMS * sizeof(float), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dmu, mean, sizeof(mean), hipMemcpyHostToDevice));
     CHK(hipMemcpy(dsc, scale, sizeof(scale), hipMemcpyHostToDevice));
@@ -274,7 +262,7 @@ std::string DegreeModel::predict(int n, const float *x, float delta, int *degree
         const int m = std::min(chunk, n - o);
         CHK(hipMemcpy(dx, x + (size_t)o * btl::MLP_IN, (size_t)m * btl::MLP_IN * sizeof(float),
                       hipMemcpyHostToDevice));
-        CHK(btl::launch_mlp_infer(dp, dmu, dsc, m, dx, delta, dz, dd, tb, nullptr));
+        CHK(btl::launch_mlp_infer(dp, dmu, dsc, m, dx, delta, dz, dd, nullptr));
         if (degree) CHK(hipMemcpy(degree + o, dd, m * sizeof(int), hipMemcpyDeviceToHost));
         if (logits)
             CHK(hipMemcpy(logits + (size_t)o * btl::MLP_OUT, dz, (size_t)m * btl::MLP_OUT * sizeof(float),

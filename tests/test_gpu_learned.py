@@ -220,6 +220,28 @@ def test_mlp_gradient_and_logits_match_oracle(bt, oracle_mod):
     assert np.array_equal(d[clear], expect[clear])
 
 
+@pytest.mark.parametrize("n", [1, 15, 17, 31, 32, 33, 8192, 8192 + 33, 3 * 8192 + 1])
+def test_mlp_tiles_of_samples(bt, oracle_mod, n):
+    """Batches around a tile of 32 samples and around 256 tiles (one per
+    block of the gradient launch, whose blocks then take several): FP32 sums
+    of at most n terms, whose rounding grows as sqrt(n) 2^-24 (1e-5 at
+    24577; a sample whose hidden unit changes sign at rounding level moves
+    the gradient by about 1/n of its norm)."""
+    m, rng = random_model(bt, 4)
+    p, mu, sc = m.get_params()
+    x = rng.normal(0, 1, (n, 8)).astype(np.float32)
+    y = rng.integers(2, 14, n)
+    loss, g = m.gradient(x, y)
+    lo, go = oracle_mod.mlp_loss_grad(p.astype(np.float64), mu, sc, x, y)
+    assert abs(loss - lo) <= 1e-5 * abs(lo)
+    assert rel_l2(go, g) <= 1e-4
+    assert np.array_equal(m.gradient(x, y)[1], g)  # fixed order of every sum
+    d, z = m.predict(x, with_logits=True)
+    zo = oracle_mod.mlp_logits(p.astype(np.float64), mu, sc, x)
+    assert np.max(np.abs(z - zo)) <= 1e-4 * (1 + np.max(np.abs(zo)))
+    assert d.shape == (n,) and np.array_equal(m.predict(x), d)
+
+
 def test_training_lowers_loss_and_learns_a_rule(bt):
     rng = np.random.default_rng(8)
     x = rng.uniform(-1, 1, (40000, 8)).astype(np.float32)
