@@ -9,28 +9,87 @@
 #include <cfloat>
 #include <cmath>
 
+#include "bt_exp.h"
 #include "bt_learn.h"
+#include "bt_rsq.h"
 
 namespace btl {
 
 namespace {
 
 // ---------------------------------------------------------------------
-// Pair labels.
+// Pair labels.  One block of 4 waves per pair; degrees are tried in order.
+// A degree's heavy part is a sum over points (sources, or source grid points)
+// for each of a set of grid points; its work items are (grid point, share of
+// the points): G = label_split shares per grid point, so that the small grids
+// of the low degrees fill the block too, the shares added in order
+// afterwards.  FP64; 1/r by rsq64, exponentials from the table of bt_exp.h.
+// Instantiated per kind, kernel and singularity, so that a block holds only
+// the arrays its kind uses: 34 kB of LDS for a cluster-particle pair (4
+// blocks per CU), where one kernel for every kind held 128 kB (1 block, one
+// wave per SIMD) and took IEEE square roots and divisions and three integer
+// divisions per term.  16k cluster-particle pairs of a 300k Plummer sphere
+// (regularized Coulomb, tol 1e-7, 190k terms a pair): 18.5 -> 2.5 ms, of which
+// the terms' 17 FP64 instructions each take 1.7.
 // ---------------------------------------------------------------------
 constexpr int LTPB = 256;
 constexpr int NLMAX = LABEL_DMAX + 1;
 constexpr int PMAX = NLMAX * NLMAX * NLMAX;
 constexpr int LPT = LTPB / LABEL_NT;  // lanes per sampled target (8)
+constexpr int L_PC = 1, L_CP = 2;     // pair kinds (3: CC)
 
-// SK pair kernel: 1/r, exp(-kappa r)/r, 1/sqrt(r^2 + eps^2)
-__device__ __forceinline__ double green(int kernel, double p0, double dx, double dy, double dz)
+// Shares of the points per grid point of degree nl - 1: what leaves the
+// fewest of the block's threads and steps idle for 128 points (at least
+// 0.87 busy), within PMAX partial sums.
+__device__ __forceinline__ int label_split(int nl)
 {
-    const double r2 = dx * dx + dy * dy + dz * dz;
-    if (kernel == 3) return 1.0 / sqrt(r2 + p0 * p0);
-    const double r = sqrt(r2);
-    if (kernel == 2) return exp(-p0 * r) / r;
-    return 1.0 / r;
+    switch (nl) {
+        case 3: return 9;
+        case 4: return 8;
+        case 5: return 8;
+        case 6: return 7;
+        case 7: return 5;
+        case 8: return 2;
+        default: return 1;
+    }
+}
+
+// (k1, k2, k3) of grid point j = k1 + nl (k2 + nl k3); exact for j < 4096,
+// nl <= 13: the quotient's error j (ceil(2^16/nl) - 2^16/nl) / 2^16 is below
+// j / 2^16 < 1/nl
+__device__ __forceinline__ void grid_index(int j, int nl, int &k1, int &k2, int &k3)
+{
+    const unsigned m = (65536u + nl - 1) / nl;
+    const int r = (int)(((unsigned)j * m) >> 16);
+    k1 = j - r * nl;
+    k3 = (int)(((unsigned)r * m) >> 16);
+    k2 = r - k3 * nl;
+}
+
+// The pair's kernel from r^2 (1/r, e^{-kappa r}/r, 1/sqrt(r^2 + eps^2)), and
+// with subtraction the second term's, which multiplies the source weight
+// and, at the target, minus the target's charge (coulomb_ss_pc.c:47,
+// yukawa_ss_pc.c:46, regularized-coulomb_ss_pc.c, coulomb_ss_cp.c:54-55):
+// Coulomb e^{-r^2/k^2}/r, Yukawa the same kernel, regularized Coulomb
+// e^{-r^2/a^2}/sqrt(r^2 + eps^2)
+struct LabelKernel {
+    double eps2;
+    btk::ExpRate ek, eg;
+    const double *tab;
+};
+
+template <int KER, bool SS>
+__device__ __forceinline__ void green(const LabelKernel &K, double r2, double a, double b, double &v, double &vw)
+{
+    const double ir = btk::rsq64(KER == 3 ? r2 + K.eps2 : r2);
+    if constexpr (KER == 2) {
+        const double g = btk::exp_neg(r2 * ir, K.ek, K.tab) * ir;
+        v = fma(a, g, v);
+        if constexpr (SS) vw = fma(b, g, vw);
+    } else {
+        v = fma(a, ir, v);
+        if constexpr (SS) vw = fma(b, btk::exp_neg(r2, K.eg, K.tab) * ir, vw);
+    }
 }
 
 // Lagrange basis at Chebyshev points (barycentric form, second kind):
@@ -60,72 +119,72 @@ __device__ __forceinline__ double group_sum(double v)
     return v;
 }
 
-// Subtraction kernels: the second term's kernel, which multiplies the
-// source weight and, at the target, minus the target's charge
-// (coulomb_ss_pc.c:47, yukawa_ss_pc.c:46, regularized-coulomb_ss_pc.c,
-// coulomb_ss_cp.c:54-55): Coulomb e^{-r^2/k^2}/r, Yukawa e^{-kappa r}/r (the
-// same kernel), regularized Coulomb e^{-r^2/a^2}/sqrt(r^2 + eps^2);
-// p1 = 1/k^2 or 1/a^2.
-__device__ __forceinline__ double green_w(int kernel, double p0, double p1, double dx, double dy, double dz)
-{
-    if (kernel == 2) return green(kernel, p0, dx, dy, dz);
-    const double r2 = dx * dx + dy * dy + dz * dz;
-    return exp(-r2 * p1) * green(kernel, p0, dx, dy, dz);
-}
-
-__global__ __launch_bounds__(LTPB) void k_label(LabelArgs A)
+template <int KIND, int KER, bool SS>
+__global__ __launch_bounds__(LTPB) void k_label(LabelArgs A, LabelKernel K)
 {
     constexpr int NT = LABEL_NT, NS = LABEL_NS;
-    __shared__ double Ltx[NT], Lty[NT], Ltz[NT], Ltq[NT], Lex[NT], Lred[2 * NT];
-    __shared__ double Lsx[NS], Lsy[NS], Lsz[NS], Lsq[NS], Lsw[NS];
-    __shared__ double Lnt[3 * NLMAX], Lns[3 * NLMAX];
-    __shared__ double Bs[NS * 3 * NLMAX];
-    __shared__ double Bt[NT * 3 * NLMAX];
-    // grid values of the two terms (the second only with subtraction)
-    __shared__ double G1[PMAX], G2[PMAX], G1w[PMAX], G2w[PMAX];
-    __shared__ int Ldone;
-
-    const bool ss = A.ss != 0;
+    constexpr bool SRC = KIND != L_CP, TGT = KIND != L_PC;  // interpolated sides
+    constexpr bool EXPS = SS || KER == 2;
     const int pi = blockIdx.x, tid = threadIdx.x;
-    const int kind = A.kind[pi];
+    if (A.kind[pi] != KIND) return;  // another instantiation's (block-uniform)
+
+    __shared__ double4 Ls[NS];  // sources: x, y, z, first term's charge
+    __shared__ double Lsw[SS ? NS : 1];
+    __shared__ double Ltx[NT], Lty[NT], Ltz[NT], Ltq[NT], Lex[NT], Lred[2 * NT];
+    __shared__ double Lnt[3 * NLMAX], Lns[3 * NLMAX];
+    __shared__ double Bs[SRC ? NS * 3 * NLMAX : 1];
+    __shared__ double Bt[TGT ? NT * 3 * NLMAX : 1];
+    // grid values of the two terms (the second only with subtraction)
+    __shared__ double G1[SRC ? PMAX : 1], G1w[SRC && SS ? PMAX : 1];
+    // (CC: in the place of the source basis, which has been read by then)
+    __shared__ double G2s[TGT && !SRC ? (SS ? 2 : 1) * PMAX : 1];
+    static_assert(NS * 3 * NLMAX >= 2 * PMAX, "target grids fit the source basis");
+    double *const G2 = SRC ? Bs : G2s, *const G2w = G2 + PMAX;
+    __shared__ double Ltab[EXPS ? btk::EXP_TAB : 1];
+    if constexpr (EXPS) btk::exp_table(Ltab, tid);
+    K.tab = Ltab;
+
     const int tb0 = A.tbeg[pi], tc = A.tcnt[pi], sb0 = A.sbeg[pi], sc = A.scnt[pi];
     const int nt = min(tc, NT), ns = min(sc, NS);
     const double *tbox = A.tbox + 6 * (size_t)pi, *sbox = A.sbox + 6 * (size_t)pi;
     if (tid < nt) {
         const int i = tb0 + (int)(((long long)tid * tc) / nt);
         Ltx[tid] = A.tx[i]; Lty[tid] = A.ty[i]; Ltz[tid] = A.tz[i];
-        Ltq[tid] = ss ? A.tq[i] : 0.0;
+        Ltq[tid] = SS ? A.tq[i] : 0.0;
     }
     if (tid < ns) {
         const int s = sb0 + (int)(((long long)tid * sc) / ns);
-        Lsx[tid] = A.sx[s]; Lsy[tid] = A.sy[s]; Lsz[tid] = A.sz[s];
         // subtraction: the first term's charge is q w, the second's w
-        const double w = ss ? A.sw[s] : 1.0;
-        Lsq[tid] = ss ? A.sq[s] * w : A.sq[s];
-        Lsw[tid] = w;
+        double q = A.sq[s];
+        if constexpr (SS) {
+            const double w = A.sw[s];
+            Lsw[tid] = w;
+            q *= w;
+        }
+        Ls[tid] = make_double4(A.sx[s], A.sy[s], A.sz[s], q);
     }
-    if (tid == 0) Ldone = 0;
     __syncthreads();
 
     const int g = tid / LPT, l = tid % LPT;  // target of this lane group, lane in group
+    const double tx = g < nt ? Ltx[g] : 0.0, ty = g < nt ? Lty[g] : 0.0, tz = g < nt ? Ltz[g] : 0.0;
     // exact sums at the sampled targets
     {
         double v = 0.0, vw = 0.0;
         if (g < nt)
             for (int s = l; s < ns; s += LPT) {
-                const double dx = Ltx[g] - Lsx[s], dy = Lty[g] - Lsy[s], dz = Ltz[g] - Lsz[s];
-                v += Lsq[s] * green(A.kernel, A.p0, dx, dy, dz);
-                if (ss) vw += Lsw[s] * green_w(A.kernel, A.p0, A.p1, dx, dy, dz);
+                const double4 p = Ls[s];
+                const double dx = tx - p.x, dy = ty - p.y, dz = tz - p.z;
+                green<KER, SS>(K, fma(dz, dz, fma(dy, dy, dx * dx)), p.w, SS ? Lsw[s] : 0.0, v, vw);
             }
         v = group_sum(v);
-        if (ss) vw = group_sum(vw);
-        if (l == 0 && g < nt) Lex[g] = ss ? v - Ltq[g] * vw : v;
+        if constexpr (SS) vw = group_sum(vw);
+        if (l == 0 && g < nt) Lex[g] = SS ? v - Ltq[g] * vw : v;
     }
-    __syncthreads();
 
     int label = LABEL_DMAX + 1;
     for (int p = LABEL_DMIN; p <= LABEL_DMAX; p++) {
-        const int nl = p + 1, P = nl * nl * nl;
+        const int nl = p + 1, n2 = nl * nl, P = n2 * nl, G = label_split(nl);
+        __syncthreads();  // the previous degree's arrays have been read
         if (tid < 3 * nl) {
             const int d = tid / nl, k = tid % nl;
             const double u = (cos(k * M_PI / p) + 1.0) * 0.5;
@@ -133,112 +192,147 @@ __global__ __launch_bounds__(LTPB) void k_label(LabelArgs A)
             Lns[d * nl + k] = sbox[2 * d] + u * (sbox[2 * d + 1] - sbox[2 * d]);
         }
         __syncthreads();
-        if (kind != 2) {  // PC, CC: source-side basis
-            for (int idx = tid; idx < ns * 3; idx += LTPB) {
-                const int s = idx / 3, d = idx % 3;
-                const double c = d == 0 ? Lsx[s] : (d == 1 ? Lsy[s] : Lsz[s]);
-                lagrange_row(c, Lns + d * nl, nl, Bs + (s * 3 + d) * NLMAX);
+        if constexpr (SRC)
+            for (int i = tid; i < ns * 3; i += LTPB) {
+                const int s = i / 3, d = i % 3;
+                const double c = d == 0 ? Ls[s].x : (d == 1 ? Ls[s].y : Ls[s].z);
+                lagrange_row(c, Lns + d * nl, nl, Bs + i * NLMAX);
             }
-        }
-        if (kind != 1) {  // CP, CC: target-side basis
-            for (int idx = tid; idx < nt * 3; idx += LTPB) {
-                const int i = idx / 3, d = idx % 3;
-                const double c = d == 0 ? Ltx[i] : (d == 1 ? Lty[i] : Ltz[i]);
-                lagrange_row(c, Lnt + d * nl, nl, Bt + (i * 3 + d) * NLMAX);
+        if constexpr (TGT)
+            for (int i = tid; i < nt * 3; i += LTPB) {
+                const int t = i / 3, d = i % 3;
+                const double c = d == 0 ? Ltx[t] : (d == 1 ? Lty[t] : Ltz[t]);
+                lagrange_row(c, Lnt + d * nl, nl, Bt + i * NLMAX);
             }
-        }
-        __syncthreads();
-        if (kind != 2) {
+        // the shares' sums (X[g P + j]) added in order into X[j]
+        auto combine = [&](double *X, double *Xw) {
+            __syncthreads();
+            if (G > 1) {
+                for (int j = tid; j < P; j += LTPB) {
+                    double v = X[j], vw = SS ? Xw[j] : 0.0;
+                    for (int q = 1; q < G; q++) {
+                        v += X[q * P + j];
+                        if constexpr (SS) vw += Xw[q * P + j];
+                    }
+                    X[j] = v;
+                    if constexpr (SS) Xw[j] = vw;
+                }
+                __syncthreads();
+            }
+        };
+        if constexpr (SRC) {
+            __syncthreads();
             // modified charges of the source grid: Q_k = sum_s q_s l_k(y_s)
-            for (int j = tid; j < P; j += LTPB) {
-                const int k1 = j % nl, k2 = (j / nl) % nl, k3 = j / (nl * nl);
-                double q = 0.0, qw = 0.0;
-                for (int s = 0; s < ns; s++) {
-                    const double b = Bs[(s * 3) * NLMAX + k1] * Bs[(s * 3 + 1) * NLMAX + k2] *
-                                     Bs[(s * 3 + 2) * NLMAX + k3];
-                    q += Lsq[s] * b;
-                    if (ss) qw += Lsw[s] * b;
+            for (int it = tid; it < P * G; it += LTPB) {
+                const int q = it / P, j = it - q * P;
+                int k1, k2, k3;
+                grid_index(j, nl, k1, k2, k3);
+                double v = 0.0, vw = 0.0;
+#pragma unroll 2
+                for (int s = q; s < ns; s += G) {
+                    const double *r = Bs + 3 * s * NLMAX;
+                    const double b = r[k1] * r[NLMAX + k2] * r[2 * NLMAX + k3];
+                    v = fma(Ls[s].w, b, v);
+                    if constexpr (SS) vw = fma(Lsw[s], b, vw);
                 }
-                G1[j] = q;
-                G1w[j] = qw;
+                G1[it] = v;
+                if constexpr (SS) G1w[it] = vw;
             }
-            __syncthreads();
+            combine(G1, G1w);
         }
-        if (kind == 2) {
-            // target grid values from the sources
-            for (int j = tid; j < P; j += LTPB) {
-                const int k1 = j % nl, k2 = (j / nl) % nl, k3 = j / (nl * nl);
+        if constexpr (TGT) {
+            // target grid values, from the sources (CP) or the source grid (CC)
+            if constexpr (!SRC) __syncthreads();
+            for (int it = tid; it < P * G; it += LTPB) {
+                const int q = it / P, j = it - q * P;
+                int k1, k2, k3;
+                grid_index(j, nl, k1, k2, k3);
                 const double gx = Lnt[k1], gy = Lnt[nl + k2], gz = Lnt[2 * nl + k3];
                 double v = 0.0, vw = 0.0;
-                for (int s = 0; s < ns; s++) {
-                    const double dx = gx - Lsx[s], dy = gy - Lsy[s], dz = gz - Lsz[s];
-                    v += Lsq[s] * green(A.kernel, A.p0, dx, dy, dz);
-                    if (ss) vw += Lsw[s] * green_w(A.kernel, A.p0, A.p1, dx, dy, dz);
+                if constexpr (KIND == L_CP) {
+#pragma unroll 4
+                    for (int s = q; s < ns; s += G) {
+                        const double4 c = Ls[s];
+                        const double dx = gx - c.x, dy = gy - c.y, dz = gz - c.z;
+                        green<KER, SS>(K, fma(dz, dz, fma(dy, dy, dx * dx)), c.w, SS ? Lsw[s] : 0.0, v, vw);
+                    }
+                } else {
+                    // the source grid's pencils (m2, m3) of the share
+                    int m2 = q % nl, m3 = q / nl;
+                    for (int m = q; m < n2; m += G) {
+                        const double dy = gy - Lns[nl + m2], dz = gz - Lns[2 * nl + m3];
+                        const double dyz = fma(dz, dz, dy * dy);
+                        for (int m1 = 0; m1 < nl; m1++) {
+                            const double dx = gx - Lns[m1];
+                            green<KER, SS>(K, fma(dx, dx, dyz), G1[m * nl + m1], SS ? G1w[m * nl + m1] : 0.0, v, vw);
+                        }
+                        m2 += G;
+                        while (m2 >= nl) { m2 -= nl; m3++; }
+                    }
                 }
-                G2[j] = v;
-                G2w[j] = vw;
+                G2[it] = v;
+                if constexpr (SS) G2w[it] = vw;
             }
-            __syncthreads();
-        } else if (kind == 3) {
-            // target grid values from the source grid
-            for (int j = tid; j < P; j += LTPB) {
-                const int k1 = j % nl, k2 = (j / nl) % nl, k3 = j / (nl * nl);
-                const double gx = Lnt[k1], gy = Lnt[nl + k2], gz = Lnt[2 * nl + k3];
-                double v = 0.0, vw = 0.0;
-                for (int k = 0; k < P; k++) {
-                    const int m1 = k % nl, m2 = (k / nl) % nl, m3 = k / (nl * nl);
-                    const double dx = gx - Lns[m1], dy = gy - Lns[nl + m2], dz = gz - Lns[2 * nl + m3];
-                    v += G1[k] * green(A.kernel, A.p0, dx, dy, dz);
-                    if (ss) vw += G1w[k] * green_w(A.kernel, A.p0, A.p1, dx, dy, dz);
-                }
-                G2[j] = v;
-                G2w[j] = vw;
-            }
-            __syncthreads();
+            combine(G2, G2w);
         }
-        // approximation at the sampled targets
+        // approximation at the sampled targets: the group's lanes take the
+        // pencils (m2, m3) of the grid in turn
         double v = 0.0, vw = 0.0;
         if (g < nt) {
-            if (kind == 1) {
-                for (int k = l; k < P; k += LPT) {
-                    const int m1 = k % nl, m2 = (k / nl) % nl, m3 = k / (nl * nl);
-                    const double dx = Ltx[g] - Lns[m1], dy = Lty[g] - Lns[nl + m2], dz = Ltz[g] - Lns[2 * nl + m3];
-                    v += G1[k] * green(A.kernel, A.p0, dx, dy, dz);
-                    if (ss) vw += G1w[k] * green_w(A.kernel, A.p0, A.p1, dx, dy, dz);
+            int m2 = l % nl, m3 = l / nl;
+            const double *b = Bt + (TGT ? g * 3 * NLMAX : 0);
+            for (int m = l; m < n2; m += LPT) {
+                if constexpr (KIND == L_PC) {
+                    const double dy = ty - Lns[nl + m2], dz = tz - Lns[2 * nl + m3];
+                    const double dyz = fma(dz, dz, dy * dy);
+                    for (int m1 = 0; m1 < nl; m1++) {
+                        const double dx = tx - Lns[m1];
+                        green<KER, SS>(K, fma(dx, dx, dyz), G1[m * nl + m1], SS ? G1w[m * nl + m1] : 0.0, v, vw);
+                    }
+                } else {
+                    const double f = b[NLMAX + m2] * b[2 * NLMAX + m3];
+                    double x = 0.0, xw = 0.0;
+                    for (int m1 = 0; m1 < nl; m1++) {
+                        x = fma(b[m1], G2[m * nl + m1], x);
+                        if constexpr (SS) xw = fma(b[m1], G2w[m * nl + m1], xw);
+                    }
+                    v = fma(f, x, v);
+                    if constexpr (SS) vw = fma(f, xw, vw);
                 }
-            } else {
-                const double *b = Bt + (g * 3) * NLMAX;
-                for (int j = l; j < P; j += LPT) {
-                    const int k1 = j % nl, k2 = (j / nl) % nl, k3 = j / (nl * nl);
-                    const double bb = b[k1] * b[NLMAX + k2] * b[2 * NLMAX + k3];
-                    v += bb * G2[j];
-                    if (ss) vw += bb * G2w[j];
-                }
+                m2 += LPT;
+                while (m2 >= nl) { m2 -= nl; m3++; }
             }
         }
         v = group_sum(v);
-        if (ss) vw = group_sum(vw);
-        if (l == 0 && g < NT) {
-            const double e = g < nt ? (ss ? v - Ltq[g] * vw : v) - Lex[g] : 0.0;
+        if constexpr (SS) vw = group_sum(vw);
+        if (l == 0) {
+            const double e = g < nt ? (SS ? v - Ltq[g] * vw : v) - Lex[g] : 0.0;
             Lred[g] = e * e;
             Lred[NT + g] = g < nt ? Lex[g] * Lex[g] : 0.0;
         }
         __syncthreads();
-        if (tid == 0) {
-            double num = 0.0, den = 0.0;
-            for (int i = 0; i < NT; i++) { num += Lred[i]; den += Lred[NT + i]; }
-            const double err = den > 0.0 ? sqrt(num / den) : (num > 0.0 ? INFINITY : 0.0);
-            A.errors[(size_t)pi * LABEL_ND + (p - LABEL_DMIN)] = err;
-            if (err <= A.tol) Ldone = 1;
-        }
-        __syncthreads();
-        if (Ldone) { label = p; break; }
+        // every thread forms the same two sums
+        double num = 0.0, den = 0.0;
+        for (int i = 0; i < NT; i++) { num += Lred[i]; den += Lred[NT + i]; }
+        const double err = den > 0.0 ? sqrt(num / den) : (num > 0.0 ? INFINITY : 0.0);
+        if (tid == 0) A.errors[(size_t)pi * LABEL_ND + (p - LABEL_DMIN)] = err;
+        if (err <= A.tol) { label = p; break; }  // block-uniform
     }
     if (tid == 0) {
         A.labels[pi] = label;
         for (int p = label + 1; p <= LABEL_DMAX; p++)
             A.errors[(size_t)pi * LABEL_ND + (p - LABEL_DMIN)] = NAN;
     }
+}
+
+template <int KER, bool SS>
+hipError_t label_dispatch(const LabelArgs &a, const LabelKernel &k, hipStream_t st)
+{
+    // every kind over the whole list, each block keeping the pairs of its own
+    k_label<1, KER, SS><<<a.npairs, LTPB, 0, st>>>(a, k);
+    k_label<2, KER, SS><<<a.npairs, LTPB, 0, st>>>(a, k);
+    k_label<3, KER, SS><<<a.npairs, LTPB, 0, st>>>(a, k);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------
@@ -564,8 +658,16 @@ __global__ __launch_bounds__(4 * RPB) void k_mlp_adam(const float *part, int npa
 hipError_t launch_label(const LabelArgs &a, hipStream_t st)
 {
     if (a.npairs <= 0) return hipSuccess;
-    k_label<<<a.npairs, LTPB, 0, st>>>(a);
-    return hipGetLastError();
+    LabelKernel k{};
+    k.eps2 = a.p0 * a.p0;
+    k.ek = btk::exp_rate(a.p0);
+    k.eg = btk::exp_rate(a.p1);
+    switch (a.kernel) {
+        case 1: return a.ss ? label_dispatch<1, true>(a, k, st) : label_dispatch<1, false>(a, k, st);
+        case 2: return a.ss ? label_dispatch<2, true>(a, k, st) : label_dispatch<2, false>(a, k, st);
+        case 3: return a.ss ? label_dispatch<3, true>(a, k, st) : label_dispatch<3, false>(a, k, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_mlp_infer(const float *params, const float *mean, const float *scale, int n,

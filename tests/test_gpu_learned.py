@@ -115,6 +115,40 @@ def test_labels_match_oracle(bt, oracle_mod):
         assert np.array_equal(lg, lo) or border
 
 
+@pytest.mark.parametrize("nt,ns", [(1, 1), (2, 5), (31, 8), (32, 9), (33, 127), (64, 129)])
+@pytest.mark.parametrize("ss", [False, True])
+def test_label_shares_at_their_edges(bt, oracle_mod, nt, ns, ss):
+    """Every degree (an unreachable tolerance), with fewer sources than a
+    grid point has shares, around 32 sampled targets and 128 sampled sources;
+    each kind and kernel.  Bars as in test_labels_match_oracle: the potentials
+    are O(ns)."""
+    rng = np.random.default_rng(100 * nt + ns)
+    kinds = np.array([1, 2, 3])
+    T = np.concatenate([rng.uniform(-0.4, 0.4, (nt, 3)) + [0, 0, 3.0 * i] for i in range(3)])
+    S = np.concatenate([rng.uniform(-0.4, 0.4, (ns, 3)) + [1.9, 0.3, 3.0 * i] for i in range(3)])
+    box = lambda c: np.concatenate([np.ravel([[c[0] - 0.5, c[0] + 0.5], [c[1] - 0.5, c[1] + 0.5],
+                                              [c[2] - 0.5, c[2] + 0.5]])])
+    tbox = np.concatenate([box((0, 0, 3.0 * i)) for i in range(3)])
+    sbox = np.concatenate([box((1.9, 0.3, 3.0 * i)) for i in range(3)])
+    Q, tq, w = rng.uniform(-1, 1, 3 * ns), rng.uniform(-1, 1, 3 * nt), rng.uniform(0.5, 1.5, 3 * ns)
+    tb, tc = np.arange(3) * nt, np.full(3, nt)
+    sb, sc = np.arange(3) * ns, np.full(3, ns)
+    pairs = (kinds, tb, tc, sb, sc, tbox, sbox)
+    for kernel, kp in ((1, [0.5]), (2, [0.5]), (3, [0.3, 0.01])):
+        p0 = {1: 0.0, 2: kp[0], 3: kp[-1]}[kernel]
+        if ss:
+            p1 = 0.0 if kernel == 2 else 1.0 / kp[0] ** 2
+            lg, eg = bt.label_pairs_subtraction(*pairs, (*T.T, tq), (*S.T, Q, w), kernel, kp, 1e-30)
+            lo, eo = oracle_mod.label_pairs_ss(*pairs, *T.T, tq, *S.T, Q, w, kernel, p0, p1, 1e-30)
+        else:
+            lg, eg = bt.label_pairs(*pairs, tuple(T.T), (*S.T, Q), kernel, p0, 1e-30)
+            lo, eo = oracle_mod.label_pairs(*pairs, *T.T, *S.T, Q, kernel, p0, 1e-30)
+        assert np.all(lg == 13) and np.all(lo == 13)
+        # relative to the pair's exact potentials, which may cancel for a few
+        # random charges: 1e-12 where the oracle's own sums keep 4 digits more
+        assert np.allclose(eg, eo, rtol=1e-8, atol=1e-12), (kernel, np.abs(eg - eo).max())
+
+
 def test_subtraction_labels_match_oracle(bt, oracle_mod):
     """Labels of the subtraction kernels (both terms) against the oracle's
     restatement, which scipy's interpolation pins."""
