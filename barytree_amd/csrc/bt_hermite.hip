@@ -17,7 +17,9 @@
 
 #include <cfloat>
 
+#include "bt_exp.h"
 #include "bt_kernels.h"
+#include "bt_rsq.h"
 
 namespace btk {
 namespace {
@@ -144,115 +146,193 @@ __global__ __launch_bounds__(HTPB) void k_herm_anterp(HermAnterpArgs a)
 }
 
 // ---------------------------------------------------------------------
-// Particle-cluster far field: tile {key, first target, count} of up to HTPB
-// targets (one per thread) against the 8-plane clusters of its key, added to
-// the potential (coulomb_pc.c:66-135, yukawa_pc.c:61-140,
+// Particle-cluster far field: tile {key, first target, count} of up to
+// HERM_PC_TILE targets against the 8-plane clusters of its key, added to the
+// potential (coulomb_pc.c:66-135, yukawa_pc.c:61-140,
 // regularized-coulomb_pc.c:67-139, coulomb_ss_pc.c:63-163,
 // yukawa_ss_pc.c:61-167, regularized-coulomb_ss_pc.c:63-160).
+//
+// The launch issues FP64 instructions back to back, so the derivative
+// expansion is written for few of them: the linear, bilinear and trilinear
+// forms of the planes once each, then Horner in 1/r^2; and the points of a
+// cluster's pencil (k2, k3) share dy, dz, dy^2 + dz^2 and dy dz.  Coulomb: 21
+// instructions per pair and 5 per pencil, where the reference's expressions
+// compiled to 44.  A point's 8 planes are 64 bytes of LDS, read as four
+// 16-byte broadcasts for the thread's HPT = 2 targets.  Each of the
+// block's 4 waves holds the tile's 128 targets and takes every fourth
+// pencil; the waves' sums are added in wave order.  With 256 targets a block
+// and every wave its own 64 (the form before) N = 100k had 1.5 waves per
+// SIMD.  N = 500k, degree 5, 7.3e9 pairs: 13.6 -> 6.7 ms (7.8 with tiles of
+// 256 targets on pairs of waves); N = 100k 4.5 -> 2.1 ms; Yukawa with
+// subtraction, N = 100k, degree 4: 5.6 -> 3.5 ms.
 // ---------------------------------------------------------------------
-template <int KER, bool SS>
-__device__ __forceinline__ double herm_pc_pair(double dx, double dy, double dz, const double *q, const double *w,
-                                               double tq, const KParams &kp)
+constexpr int HPT = 2;                // targets per thread
+constexpr int HPTS = 256;             // points per LDS chunk (whole pencils)
+static_assert(HERM_PC_TILE == 64 * HPT && HTPB == 256, "a wave's targets, four waves");
+
+// the forms of planes c in the displacement: linear, bilinear, trilinear
+// (yz = dy dz)
+__device__ __forceinline__ void herm_forms(const double *c, double dx, double dy, double dz, double yz, double &lin,
+                                           double &bil, double &tri)
 {
+    lin = fma(c[3], dz, fma(c[2], dy, c[1] * dx));
+    bil = fma(dx, fma(c[6], dz, c[4] * dy), c[5] * yz);
+    tri = (c[7] * yz) * dx;
+}
+
+// One point's expansion: dyz2 = dy^2 + dz^2 (r2 = dx^2 + dyz2).  Coulomb and
+// regularized Coulomb planes 4..6 come multiplied by 3, plane 7 by 15.
+template <int KER, bool SS>
+__device__ __forceinline__ void herm_pc_pair(double dx, double dy, double dz, double dyz2, double yz, const double *q,
+                                             const double *w, double tq, const KParams &kp, const double *tab,
+                                             double &acc)
+{
+    double r2 = fma(dx, dx, dyz2);
     if constexpr (KER == HKS) {
         // derivative expansion of sin(k r)/r; coincident points are skipped
         // (sin-over-r_pc.c:68-155)
         const double k = kp.p0, k2 = k * k, k3 = k * k2;
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        if (!(r > DBL_MIN)) return 0.0;
+        const double r = sqrt(r2);
+        if (!(r > DBL_MIN)) return;
         const double rinv = 1.0 / r;
         const double r2inv = rinv * rinv, r3inv = rinv * r2inv, r4inv = r2inv * r2inv;
         const double r5inv = r3inv * r2inv, r6inv = r3inv * r3inv, r7inv = r4inv * r3inv;
         double sn, cs;
         sincos(k * r, &sn, &cs);
-        return sn * rinv * q[0] + (sn * r3inv - k * cs * r2inv) * (q[1] * dx + q[2] * dy + q[3] * dz) +
-               (sn * (3 * r5inv - k2 * r3inv) - 3 * k * cs * r4inv) * (q[4] * dx * dy + q[5] * dy * dz + q[6] * dx * dz) +
+        acc += sn * rinv * q[0] + (sn * r3inv - k * cs * r2inv) * (q[1] * dx + q[2] * dy + q[3] * dz) +
+               (sn * (3 * r5inv - k2 * r3inv) - 3 * k * cs * r4inv) *
+                   (q[4] * dx * dy + q[5] * dy * dz + q[6] * dx * dz) +
                (sn * (15 * r7inv - 6 * k2 * r5inv) + cs * (k3 * r4inv - 15 * k * r6inv)) * q[7] * dx * dy * dz;
     } else if constexpr (KER == HKY) {
-        const double k = kp.p0, k2 = k * k, k3 = k * k2;
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double rinv = rsqrt(r2), r = r2 * rinv, r3 = r2 * r;
-        const double r3inv = rinv * rinv * rinv, r5inv = r3inv * rinv * rinv, r7inv = r5inv * rinv * rinv;
-        double c[8];
+        // e^{-x} (c0 + (1+x) L/r^2 + (3+3x+x^2) B/r^4 + (15+15x+6x^2+x^3) T/r^6)/r, x = k r
+        const double ir = rsq64(r2), i2 = ir * ir, r = r2 * ir, x = kp.p0 * r;
+        double c[8], lin, bil, tri;
 #pragma unroll
-        for (int m = 0; m < 8; m++) c[m] = SS ? q[m] - w[m] * tq : q[m];
-        return exp(-k * r) *
-               (rinv * c[0] + r3inv * (1 + k * r) * (c[1] * dx + c[2] * dy + c[3] * dz) +
-                r5inv * (3 + 3 * k * r + k2 * r2) * (c[4] * dx * dy + c[5] * dy * dz + c[6] * dx * dz) +
-                r7inv * (15 + 15 * k * r + 6 * k2 * r2 + k3 * r3) * c[7] * dx * dy * dz);
+        for (int m = 0; m < 8; m++) c[m] = SS ? fma(-w[m], tq, q[m]) : q[m];
+        herm_forms(c, dx, dy, dz, yz, lin, bil, tri);
+        const double p3 = fma(x, fma(x, x + 6.0, 15.0), 15.0), p2 = fma(x, x + 3.0, 3.0);
+        double s = fma(i2 * p3, tri, p2 * bil);
+        s = fma(i2, s, fma(x, lin, lin));
+        s = fma(i2, s, c[0]);
+        acc = fma(exp_neg(r, kp.ek, tab) * ir, s, acc);
     } else {
-        // Coulomb and regularized Coulomb: derivative expansion of 1/r (r with
-        // eps^2 for the regularized kernel); subtraction adds the one of
-        // exp(-r^2/k^2)/r weighted by -tq
-        double r2 = dx * dx + dy * dy + dz * dz;
+        // Coulomb and regularized Coulomb: (q0 + L/r^2 + 3 B/r^4 + 15 T/r^6)/r
+        // (r with eps^2 for the regularized kernel); subtraction adds the
+        // expansion of e^{-r^2/k^2}/r weighted by -tq
         if constexpr (KER == HKR) r2 += kp.eps2;
-        const double rinv = rsqrt(r2);
-        const double r3inv = rinv * rinv * rinv, r5inv = r3inv * rinv * rinv, r7inv = r5inv * rinv * rinv;
-        double v = rinv * q[0] + r3inv * (q[1] * dx + q[2] * dy + q[3] * dz) +
-                   3 * r5inv * (q[4] * dx * dy + q[5] * dy * dz + q[6] * dx * dz) + 15 * r7inv * q[7] * dx * dy * dz;
+        const double ir = rsq64(r2), i2 = ir * ir;
+        const double lin = fma(q[3], dz, fma(q[2], dy, q[1] * dx));
+        const double u = fma(i2, q[7] * yz, fma(q[6], dz, q[4] * dy));
+        double s = fma(i2, fma(dx, u, q[5] * yz), lin);
+        s = fma(i2, s, q[0]);
         if constexpr (SS) {
-            const double rk2 = r2 * kp.inv_a2, rk4 = rk2 * rk2, rk6 = rk4 * rk2;
-            v -= tq * exp(-rk2) *
-                 (rinv * w[0] + r3inv * (1 + 2 * rk2) * (w[1] * dx + w[2] * dy + w[3] * dz) +
-                  r5inv * (3 + 4 * rk2 + 4 * rk4) * (w[4] * dx * dy + w[5] * dy * dz + w[6] * dx * dz) +
-                  r7inv * (15 + 18 * rk2 + 12 * rk4 + 8 * rk6) * w[7] * dx * dy * dz);
+            double lw, bw, tw;
+            herm_forms(w, dx, dy, dz, yz, lw, bw, tw);
+            const double x = r2 * kp.inv_a2;
+            const double p3 = fma(x, fma(x, fma(x, 8.0, 12.0), 18.0), 15.0);
+            const double p2 = fma(x, fma(x, 4.0, 4.0), 3.0), p1 = fma(x, 2.0, 1.0);
+            double sw = fma(i2 * p3, tw, p2 * bw);
+            sw = fma(i2, sw, p1 * lw);
+            sw = fma(i2, sw, w[0]);
+            s = fma(-tq * exp_neg(r2, kp.eg, tab), sw, s);
         }
-        return v;
+        acc = fma(ir, s, acc);
     }
 }
 
 template <int KER, bool SS>
 __global__ __launch_bounds__(HTPB) void k_herm_pc(HermPCArgs a)
 {
+    constexpr bool EXPS = KER == HKY || (SS && KER != HKS);
     const Tile tile = a.tiles[blockIdx.x];
     if (tile.z == 0) return;
     const int tid = threadIdx.x;
-    const int P = a.P;
-    __shared__ double Lx[HTPB], Ly[HTPB], Lz[HTPB];
-    __shared__ double Lq[8][HTPB];
-    __shared__ double Lw[SS ? 8 : 1][HTPB];
-    const int i = tile.y + (tid < tile.z ? tid : 0);
-    const double tx = a.tx[i], ty = a.ty[i], tz = a.tz[i];
-    const double tq = SS ? a.tq[i] : 0.0;
-    double acc = 0.0;
+    const int nl = a.nl, P = nl * nl * nl, n2 = nl * nl;
+    __shared__ alignas(16) double Lq[HPTS][8];
+    __shared__ alignas(16) double Lw[SS ? HPTS : 1][8];
+    __shared__ double Lt[3 * (MAX_DEGREE + 1)];  // the cluster's Chebyshev points
+    __shared__ double Ltab[EXPS ? EXP_TAB : 1];
+    __shared__ double Lr[4][HERM_PC_TILE];  // the waves' sums
+    if constexpr (EXPS) exp_table(Ltab, tid);
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    int ix[HPT];
+    double tx[HPT], ty[HPT], tz[HPT], tq[HPT], acc[HPT];
+#pragma unroll
+    for (int u = 0; u < HPT; u++) {
+        const int li = lane + 64 * u;
+        ix[u] = tile.y + (li < tile.z ? li : 0);
+        tx[u] = a.tx[ix[u]]; ty[u] = a.ty[ix[u]]; tz[u] = a.tz[ix[u]];
+        tq[u] = SS ? a.tq[ix[u]] : 0.0;
+        acc[u] = 0.0;
+    }
+    const int pens = HPTS / nl;  // pencils per chunk
     for (int c = a.clu_off[tile.x]; c < a.clu_off[tile.x + 1]; c++) {
         const size_t node = (size_t)a.clu_id[c];
         const double *cq = a.cq + node * 8 * P;
         const double *cw = SS ? a.cw + node * 8 * P : nullptr;
-        for (int off = 0; off < P; off += HTPB) {
-            const int n = min(HTPB, P - off);
-            __syncthreads();
+        for (int pb = 0; pb < n2; pb += pens) {
+            const int np = min(pens, n2 - pb), n = np * nl;
+            __syncthreads();  // the previous chunk has been read
+            if (tid < 3 * nl) Lt[tid] = a.tab[node * 3 * nl + tid];
             if (tid < n) {
-                const size_t g = node * P + off + tid;
-                Lx[tid] = a.cx[g]; Ly[tid] = a.cy[g]; Lz[tid] = a.cz[g];
+                const int j = tid;
 #pragma unroll
-                for (int m = 0; m < 8; m++) Lq[m][tid] = cq[m * P + off + tid];
-                if constexpr (SS) {
-#pragma unroll
-                    for (int m = 0; m < 8; m++) Lw[m][tid] = cw[m * P + off + tid];
+                for (int m = 0; m < 8; m++) {
+                    // 3 and 15 of the Coulomb expansion
+                    constexpr bool C = KER == HKC || KER == HKR;
+                    const double f = C && m == 7 ? 15.0 : (C && m >= 4 ? 3.0 : 1.0);
+                    Lq[j][m] = f * cq[m * P + pb * nl + j];
+                    if constexpr (SS) Lw[j][m] = cw[m * P + pb * nl + j];
                 }
             }
             __syncthreads();
-            for (int jj = 0; jj < n; jj++) {
-                double q[8], w[8];
+            int k2 = (pb + wv) % nl, k3 = (pb + wv) / nl;
+            for (int pen = wv; pen < np; pen += 4) {
+                double dy[HPT], dz[HPT], dyz2[HPT], yz[HPT];
 #pragma unroll
-                for (int m = 0; m < 8; m++) {
-                    q[m] = Lq[m][jj];
-                    w[m] = SS ? Lw[m][jj] : 0.0;
+                for (int u = 0; u < HPT; u++) {
+                    dy[u] = ty[u] - Lt[nl + k2];
+                    dz[u] = tz[u] - Lt[2 * nl + k3];
+                    dyz2[u] = fma(dz[u], dz[u], dy[u] * dy[u]);
+                    yz[u] = dy[u] * dz[u];
                 }
-                acc += herm_pc_pair<KER, SS>(tx - Lx[jj], ty - Ly[jj], tz - Lz[jj], q, w, tq, a.kp);
+                for (int k1 = 0; k1 < nl; k1++) {
+                    const int j = pen * nl + k1;
+                    const double x = Lt[k1];
+                    double q[8], w[8];
+#pragma unroll
+                    for (int m = 0; m < 8; m++) {
+                        q[m] = Lq[j][m];
+                        w[m] = SS ? Lw[SS ? j : 0][m] : 0.0;
+                    }
+#pragma unroll
+                    for (int u = 0; u < HPT; u++)
+                        herm_pc_pair<KER, SS>(tx[u] - x, dy[u], dz[u], dyz2[u], yz[u], q, w, tq[u], a.kp, Ltab, acc[u]);
+                }
+                k2 += 4;
+                while (k2 >= nl) { k2 -= nl; k3++; }
             }
         }
     }
-    if (tid < tile.z) a.pot[i] += acc;
+#pragma unroll
+    for (int u = 0; u < HPT; u++) Lr[wv][lane + 64 * u] = acc[u];
+    __syncthreads();
+    if (tid < tile.z) a.pot[tile.y + tid] += ((Lr[0][tid] + Lr[1][tid]) + Lr[2][tid]) + Lr[3][tid];
 }
 
 // ---------------------------------------------------------------------
 // Cluster-particle far field: tile {key, first grid point, count, node} of
-// up to HTPB grid points (one per thread) of a target node against the
-// source ranges of its key; the 8 plane sums go to the key's output row
-// (coulomb_cp.c:66-184, yukawa_cp.c:68-194, regularized-coulomb_cp.c:68-188,
-// sin-over-r_cp.c:68-198).
+// up to HTPB grid points of a target node against the source ranges of its
+// key; the 8 plane sums go to the key's output row (coulomb_cp.c:66-184,
+// yukawa_cp.c:68-194, regularized-coulomb_cp.c:68-188,
+// sin-over-r_cp.c:68-198).  A tile of at most HTPB/2 points leaves room for
+// G = HTPB / count shares of the sources: thread (share, point) takes every
+// G-th source and the shares' sums are added in share order, so the grids of
+// degrees 1 to 4 (8 to 125 points) fill the block.  Coulomb: 28 FP64
+// instructions per pair (the expressions as the reference writes them
+// compiled to about 34): the second derivatives' common factor is applied once,
+// and 3 and 15 after the sums.  N = 500k, degree 5: 10.7 -> 9.2 ms; N = 100k,
+// degree 3 (64 points): 3.1 -> 0.7 ms.
 // ---------------------------------------------------------------------
 template <int KER>
 __global__ __launch_bounds__(HTPB) void k_herm_cp(HermCPArgs a)
@@ -261,8 +341,14 @@ __global__ __launch_bounds__(HTPB) void k_herm_cp(HermCPArgs a)
     if (tile.z == 0) return;
     const int tid = threadIdx.x;
     const int nl = a.nl, P = nl * nl * nl;
-    __shared__ double Lx[HTPB], Ly[HTPB], Lz[HTPB], Lq[HTPB];
-    const int jl = tile.y + (tid < tile.z ? tid : 0);
+    __shared__ double4 Ls[HTPB];
+    __shared__ double Lr[HTPB];
+    __shared__ double Ltab[KER == HKY ? EXP_TAB : 1];
+    if constexpr (KER == HKY) exp_table(Ltab, tid);
+    const int G = HTPB / tile.z;  // shares of the sources (1 above HTPB/2 points)
+    const int share = tid / tile.z, lp = tid - share * tile.z;
+    const bool on = share < G;
+    const int jl = tile.y + lp;
     const int k1 = jl % nl, k2 = (jl / nl) % nl, k3 = jl / (nl * nl);
     const double *tab = a.tab + (size_t)tile.w * 3 * nl;
     const double cx = tab[k1], cy = tab[nl + k2], cz = tab[2 * nl + k3];
@@ -277,20 +363,23 @@ __global__ __launch_bounds__(HTPB) void k_herm_cp(HermCPArgs a)
             __syncthreads();
             if (tid < n) {
                 const int g = sg.x + off + tid;
-                Lx[tid] = a.sx[g]; Ly[tid] = a.sy[g]; Lz[tid] = a.sz[g]; Lq[tid] = a.sq[g];
+                Ls[tid] = make_double4(a.sx[g], a.sy[g], a.sz[g], a.sq[g]);
             }
             __syncthreads();
-            for (int jj = 0; jj < n; jj++) {
-                const double dx = Lx[jj] - cx, dy = Ly[jj] - cy, dz = Lz[jj] - cz;
+            if (!on) continue;
+            for (int jj = share; jj < n; jj += G) {
+                const double4 S = Ls[jj];
+                const double dx = S.x - cx, dy = S.y - cy, dz = S.z - cz;
+                double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
                 if constexpr (KER == HKS) {
                     const double k = a.kp.p0, k2 = k * k, k3 = k * k2;
-                    const double r = sqrt(dx * dx + dy * dy + dz * dz);
+                    const double r = sqrt(r2);
                     const double rinv = 1.0 / r;
                     const double r2inv = rinv * rinv, r3inv = rinv * r2inv, r4inv = r2inv * r2inv;
                     const double r5inv = r3inv * r2inv, r6inv = r3inv * r3inv, r7inv = r4inv * r3inv;
                     double sn, cs;
                     sincos(k * r, &sn, &cs);
-                    sn *= Lq[jj]; cs *= Lq[jj];
+                    sn *= S.w; cs *= S.w;
                     const double d1 = sn * r3inv - k * cs * r2inv;
                     const double d2 = sn * (3 * r5inv - k2 * r3inv) - 3 * k * cs * r4inv;
                     const double d3 = sn * (15 * r7inv - 6 * k2 * r5inv) + cs * (k3 * r4inv - 15 * k * r6inv);
@@ -298,39 +387,51 @@ __global__ __launch_bounds__(HTPB) void k_herm_cp(HermCPArgs a)
                     t[1] += d1 * dx; t[2] += d1 * dy; t[3] += d1 * dz;
                     t[4] += d2 * dx * dy; t[5] += d2 * dy * dz; t[6] += d2 * dx * dz;
                     t[7] += d3 * dx * dy * dz;
-                } else if constexpr (KER == HKY) {
-                    const double k = a.kp.p0, k2 = k * k, k3 = k * k2;
-                    const double r2 = dx * dx + dy * dy + dz * dz;
-                    const double rinv = rsqrt(r2), r = r2 * rinv, r3 = r2 * r;
-                    const double r2inv = rinv * rinv;
-                    const double rinvq = Lq[jj] * rinv * exp(-k * r);
-                    const double r3inv = rinvq * r2inv, r5inv = r3inv * r2inv, r7inv = r5inv * r2inv;
-                    const double d1 = r3inv * (1 + k * r);
-                    const double d2 = r5inv * (3 + 3 * k * r + k2 * r2);
-                    const double d3 = r7inv * (15 + 15 * k * r + 6 * k2 * r2 + k3 * r3);
-                    t[0] += rinvq;
-                    t[1] += d1 * dx; t[2] += d1 * dy; t[3] += d1 * dz;
-                    t[4] += d2 * dx * dy; t[5] += d2 * dy * dz; t[6] += d2 * dx * dz;
-                    t[7] += d3 * dx * dy * dz;
                 } else {
-                    double r2 = dx * dx + dy * dy + dz * dz;
                     if constexpr (KER == HKR) r2 += a.kp.eps2;
-                    const double rinv = rsqrt(r2);
-                    const double r2inv = rinv * rinv;
-                    const double rinvq = Lq[jj] * rinv;
-                    const double r3inv = rinvq * r2inv, r5inv = 3.0 * (r3inv * r2inv), r7inv = r3inv * r2inv * r2inv;
-                    t[0] += rinvq;
-                    t[1] += r3inv * dx; t[2] += r3inv * dy; t[3] += r3inv * dz;
-                    t[4] += r5inv * dx * dy; t[5] += r5inv * dy * dz; t[6] += r5inv * dx * dz;
-                    t[7] += r7inv * dx * dy * dz * 15.0;
+                    const double ir = rsq64(r2), i2 = ir * ir;
+                    // g q; the factors of the first, second and third
+                    // derivatives d1, d2, d3 (Coulomb: over 1, 3, 15)
+                    double g, d1, d2, d3;
+                    if constexpr (KER == HKY) {
+                        const double r = r2 * ir, x = a.kp.p0 * r;
+                        g = S.w * ir * exp_neg(r, a.kp.ek, Ltab);
+                        const double g3 = g * i2, g5 = g3 * i2;
+                        d1 = fma(g3, x, g3);
+                        d2 = g5 * fma(x, x + 3.0, 3.0);
+                        d3 = g5 * i2 * fma(x, fma(x, x + 6.0, 15.0), 15.0);
+                    } else {
+                        g = S.w * ir;
+                        d1 = g * i2;
+                        d2 = d1 * i2;
+                        d3 = 0.0;
+                    }
+                    t[0] += g;
+                    t[1] = fma(d1, dx, t[1]); t[2] = fma(d1, dy, t[2]); t[3] = fma(d1, dz, t[3]);
+                    const double d2y = d2 * dy, d2xy = d2y * dx;
+                    t[4] += d2xy;
+                    t[5] = fma(d2y, dz, t[5]);
+                    t[6] = fma(d2 * dx, dz, t[6]);
+                    t[7] = fma(KER == HKY ? d3 * dx * dy : d2xy * i2, dz, t[7]);
                 }
             }
         }
     }
-    if (tid < tile.z) {
-        double *o = a.rows + a.out_row[tile.x];
+    if constexpr (KER == HKC || KER == HKR) {
+        t[4] *= 3.0; t[5] *= 3.0; t[6] *= 3.0;
+        t[7] *= 15.0;
+    }
+    double *o = a.rows + a.out_row[tile.x];
 #pragma unroll
-        for (int m = 0; m < 8; m++) o[(size_t)m * P + jl] = t[m];
+    for (int m = 0; m < 8; m++) {
+        if (G > 1) {  // block-uniform
+            __syncthreads();
+            Lr[tid] = t[m];
+            __syncthreads();
+            if (share == 0)
+                for (int q = 1; q < G; q++) t[m] += Lr[q * tile.z + lp];
+        }
+        if (share == 0) o[(size_t)m * P + jl] = t[m];
     }
 }
 
@@ -449,6 +550,7 @@ hipError_t launch_herm_anterp(const HermAnterpArgs &a, hipStream_t st)
 hipError_t launch_herm_pc(const HermPCArgs &a, hipStream_t st)
 {
     if (a.ntiles <= 0) return hipSuccess;
+    if (a.nl < 2 || a.nl > MAX_DEGREE + 1) return hipErrorInvalidValue;
     dim3 g(a.ntiles), b(HTPB);
     const bool ss = a.singularity == 2;
 #define L(K, S) k_herm_pc<K, S><<<g, b, 0, st>>>(a)

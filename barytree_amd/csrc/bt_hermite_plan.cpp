@@ -25,7 +25,12 @@ namespace {
         if (e_ != hipSuccess) return std::string(#expr ": ") + hipGetErrorString(e_); \
     } while (0)
 
-constexpr int HERM_TILE = 256;  // targets (or grid points) per Hermite tile
+constexpr int HERM_TILE = 256;  // grid points (CP) or targets (downpass) per Hermite tile
+// upward pass: particles per part (multiples of the 64-particle chunk), so
+// that a system has about HERM_PARTS parts (blocks per 256 grid points); with
+// parts of 16384 the root of 20k particles was two blocks' work (1.08 ms of
+// a 1.45 ms execution at degree 2)
+constexpr int HERM_PARTS = 4096, HERM_PART_MIN = 256;
 constexpr int HERM_PLANES = 8;
 // sources per Hermite CP key: heavier keys are split (into rows of their
 // own), so that the launch has many blocks of similar work
@@ -44,13 +49,18 @@ void Plan::build_hermite_work()
 
     if (p.compute_type == C_PC) {
         // upward pass: every source node from its own particles, in parts
+        // (systems of a batch are split as they are alone)
         for (const System &sy : sys_) {
+            long long all = 0;
+            for (int i = 0; i < sy.stree.n; i++) all += sy.stree.numpar[i];
+            const int part = (int)std::min<long long>(
+                PART_MAX, std::max<long long>(HERM_PART_MIN, (all / HERM_PARTS + 63) / 64 * 64));
             for (int i = 0; i < sy.stree.n; i++) {
                 const int b = sy.soff + sy.stree.ibeg[i], e = sy.soff + sy.stree.iend[i];
-                for (int o = b; o < e; o += PART_MAX) {
+                for (int o = b; o < e; o += part) {
                     hp_node_.push_back(sy.snode_off + i);
                     hp_beg_.push_back(o);
-                    hp_end_.push_back(std::min(e, o + PART_MAX));
+                    hp_end_.push_back(std::min(e, o + part));
                 }
                 hp_off_.push_back((int)hp_node_.size());
             }
@@ -79,8 +89,9 @@ void Plan::build_hermite_work()
             hpc_.clu_off.push_back((int)hpc_.clu_id.size());
             hpc_.seg_off.push_back(0);
             hpc_.pairs += (long long)near_.tcnt[k] * P * (c1 - c0);
-            for (int o = 0; o < near_.tcnt[k]; o += HERM_TILE)
-                hpc_tiles_.push_back(btk::Tile{hk, near_.tbeg[k] + o, std::min(HERM_TILE, near_.tcnt[k] - o), 0});
+            const int tt = btk::HERM_PC_TILE;
+            for (int o = 0; o < near_.tcnt[k]; o += tt)
+                hpc_tiles_.push_back(btk::Tile{hk, near_.tbeg[k] + o, std::min(tt, near_.tcnt[k] - o), 0});
         }
         near_ = std::move(nn);
         make_queue_tiles(near_, tile_targets_, false, P, near_tiles_, near_qlen_);
@@ -139,7 +150,8 @@ std::string Plan::validate_hermite() const
                 return "hermite part";
         if (swtab_.size() != (size_t)nsnodes_ * 3 * (prm_.degree + 1)) return "hermite source weights";
         for (const btk::Tile &t : hpc_tiles_)
-            if (t.x < 0 || t.x >= (int)hpc_.key.size() || t.y < 0 || t.z <= 0 || t.y + t.z > M_)
+            if (t.x < 0 || t.x >= (int)hpc_.key.size() || t.y < 0 || t.z <= 0 || t.z > btk::HERM_PC_TILE ||
+                t.y + t.z > M_)
                 return "hermite PC tile";
         for (int c : hpc_.clu_id)
             if (c < 0 || c >= nsnodes_) return "hermite PC cluster";
@@ -195,7 +207,6 @@ std::string Plan::hermite_upward()
 {
     const Params &p = prm_;
     const bool ss = p.singularity == S_SUBTRACTION;
-    HIPCHK(btk::launch_cluster_points(nsnodes_, p.degree + 1, d_stab_, d_cx_, d_cy_, d_cz_, st_));
     btk::HermAnterpArgs a{};
     a.degree = p.degree; a.subtraction = ss; a.nparts = (int)hp_node_.size();
     a.part_node = d_hp_node_; a.part_beg = d_hp_beg_; a.part_end = d_hp_end_;
@@ -211,9 +222,9 @@ std::string Plan::hermite_upward()
 std::string Plan::hermite_pc()
 {
     btk::HermPCArgs a{};
-    a.kernel = prm_.kernel; a.singularity = prm_.singularity; a.ntiles = (int)hpc_tiles_.size(); a.P = prm_.P;
+    a.kernel = prm_.kernel; a.singularity = prm_.singularity; a.ntiles = (int)hpc_tiles_.size(); a.nl = prm_.degree + 1;
     a.tiles = d_hpc_tiles_; a.clu_off = d_hpc_clu_off_; a.clu_id = d_hpc_clu_id_;
-    a.cx = d_cx_; a.cy = d_cy_; a.cz = d_cz_; a.cq = d_cq_; a.cw = d_cw_;
+    a.tab = d_stab_; a.cq = d_cq_; a.cw = d_cw_;
     a.tx = d_tx_; a.ty = d_ty_; a.tz = d_tz_; a.tq = d_tq_;
     a.kp = kp_; a.pot = d_pot_;
     HIPCHK(btk::launch_herm_pc(a, st_));

@@ -194,13 +194,14 @@ struct HermAnterpArgs {
     double *Qp, *Wp;
 };
 hipError_t launch_herm_anterp(const HermAnterpArgs &a, hipStream_t st);
-// Particle-cluster far field: tile {key, first target, count} against the
-// clusters clu_id[clu_off[key] ..) of its key, added to pot.
+// Particle-cluster far field: tile {key, first target, count <= HERM_PC_TILE}
+// against the clusters clu_id[clu_off[key] ..) of its key, added to pot.
+constexpr int HERM_PC_TILE = 128;
 struct HermPCArgs {
-    int kernel, singularity, ntiles, P;
+    int kernel, singularity, ntiles, nl;
     const Tile *tiles;
     const int *clu_off, *clu_id;
-    const double *cx, *cy, *cz, *cq, *cw;
+    const double *tab, *cq, *cw;  // the clusters' Chebyshev points and planes
     const double *tx, *ty, *tz, *tq;
     KParams kp;
     double *pot;

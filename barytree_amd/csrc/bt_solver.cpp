@@ -1259,10 +1259,13 @@ std::string Plan::finish_create(const PlanInput &in, bool host_only, double t2)
     if (need_src_clusters) {
         if (!(r = up(&d_stab_, stab)).empty()) return r;
         const size_t np = (size_t)nsnodes_ * Pz;
-        d_cx_ = dalloc<double>(np); d_cy_ = dalloc<double>(np); d_cz_ = dalloc<double>(np);
+        if (!herm_) {  // the Hermite kernels take the points from the node tables
+            d_cx_ = dalloc<double>(np); d_cy_ = dalloc<double>(np); d_cz_ = dalloc<double>(np);
+            if (!d_cx_ || !d_cy_ || !d_cz_) return "hipMalloc failed (source cluster points)";
+        }
         d_cq_ = dalloc<double>(np * planes);
         if (ss) d_cw_ = dalloc<double>(np * planes);
-        if (!d_cx_ || !d_cy_ || !d_cz_ || !d_cq_ || (ss && !d_cw_)) return "hipMalloc failed (source clusters)";
+        if (!d_cq_ || (ss && !d_cw_)) return "hipMalloc failed (source clusters)";
         if (!(r = up(&d_sibeg_, g_sibeg_)).empty()) return r;
         if (!(r = up(&d_siend_, g_siend_)).empty()) return r;
         if (!(r = up(&d_sleaves_, g_sleaves_)).empty()) return r;

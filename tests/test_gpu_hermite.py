@@ -47,9 +47,37 @@ def test_hermite_degrees(bt, oracle_mod, ct, k, s, deg):
     assert rel_l2(ref, got) <= TOL_FP64
 
 
+@pytest.mark.parametrize("m", [1, 63, 65, 127, 128, 129, 257])
+def test_hermite_particle_cluster_tiles(bt, oracle_mod, m):
+    """Target batches around the 128 targets of a particle-cluster tile, at
+    degrees whose pencils (4, 9, 25, 49, 169) leave the four waves unequal
+    shares; degree 12 takes several chunks of pencils per cluster."""
+    rng = np.random.default_rng(m)
+    t = [rng.uniform(3.0, 3.4, m) for _ in range(3)] + [rng.uniform(-1, 1, m)]
+    _, src = uniform_cube(3000, 1, seed=77)
+    for k, s, deg, leaf in ((1, 1, 1, 60), (3, 2, 2, 120), (2, 2, 4, 600), (1, 2, 6, 1500), (2, 1, 12, 3000)):
+        args = (k, KP[k][s], s, 2, 1, 0.7, deg, leaf, 1000)
+        ref = oracle_mod.treecode(*t, *src, *args)
+        if deg < 12:
+            assert oracle_mod.last_stats()["num_pc"] > 0
+        assert rel_l2(ref, bt.solve(t, src, *args)) <= TOL_FP64, (k, s, deg)
+
+
+@pytest.mark.parametrize("deg", [1, 2, 3, 4, 5, 6])
+def test_hermite_cluster_particle_shares(bt, oracle_mod, deg):
+    """Grids of 8 to 125 points, whose blocks split the sources into 32 to 2
+    shares, and of 216 and 343, which do not; source batches smaller than the
+    number of shares included."""
+    t, src = uniform_cube(4000, 4000, seed=500 + deg)
+    for k, leaf in ((1, 20), (2, 300), (3, 80)):
+        args = (k, KP[k][1], 1, 2, 2, 0.7, deg, leaf, 400)
+        ref = oracle_mod.treecode(*t, *src, *args)
+        assert rel_l2(ref, bt.solve(t, src, *args)) <= TOL_FP64, (k, deg)
+
+
 def test_hermite_large_nodes_in_parts(bt, oracle_mod):
-    """A source root of 40000 particles: its upward pass runs in parts of
-    16384 particles summed in order."""
+    """A source root of 40000 particles: its upward pass runs in parts (of
+    256 particles here) summed in order."""
     t, src = uniform_cube(2000, 40000, seed=5)
     for s in (1, 2):
         args = (1, KP[1][s], s, 2, 1, 0.7, 2, 800, 800)
