@@ -124,6 +124,7 @@ struct InteractArgs {
     // recomputed from the coordinate differences
     const double4 *key_ctr;
     int skip_sym;            // pass over source ranges flagged SEG_SYM_BIT
+    int skip_clu;            // pass over the source clusters (launch_pc64 takes them)
     // mixed grid targets: r^2 from the expansion around the target node's
     // centre (valid for acceptance-separated sources, theta < 0.99)
     int grid_scaled;
@@ -138,6 +139,23 @@ hipError_t launch_interact(const InteractArgs &a, hipStream_t st);
 // targets.  a.precision 0: FP64 displacements; 1: the centred expansion
 // (grid_scaled), for acceptance-separated sources only.
 hipError_t launch_grid_pencil(const InteractArgs &a, hipStream_t st);
+
+// FP64 particle targets against source clusters of one degree (bt_pc.hip),
+// added to pot: tile {key, first target, count <= PC_TILE} against the
+// clusters clu_id[clu_off[key] ..); Coulomb, Yukawa, regularized Coulomb and
+// regularized Yukawa with either singularity, sin-over-r and the user kernel
+// with skipping.
+constexpr int PC_TILE = 128;
+struct PcArgs {
+    int kernel, singularity, ntiles, nl;
+    const Tile *tiles;
+    const int *clu_off, *clu_id;
+    const double *tab, *cq, *cw;  // the clusters' Chebyshev points (3 nl per node) and charges
+    const double *tx, *ty, *tz, *tq;
+    KParams kp;
+    double *pot;
+};
+hipError_t launch_pc64(const PcArgs &a, hipStream_t st);
 
 // Item launch of the near field's particle pairs (Coulomb and Yukawa with
 // either singularity, regularized Coulomb with skipping; FP64 or mixed

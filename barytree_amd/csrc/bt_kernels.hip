@@ -18,9 +18,8 @@
 #include <cstdint>
 #include <type_traits>
 
-#include "bt_exp.h"
 #include "bt_kernels.h"
-#include "bt_rsq.h"
+#include "bt_pair.h"
 
 namespace btk {
 
@@ -29,23 +28,6 @@ namespace {
 constexpr int TPB = 256;  // threads per block of the interaction kernels (4 waves)
 constexpr int GRID_TPT = 2;  // targets per thread of grid-target tiles
 constexpr int NQ = TILE_QUEUES;  // tile queues, one per XCD
-constexpr int KC = 1, KY = 2, KR = 3;
-
-
-// e^{-kappa r} and e^{-r^2 inv_a2}: the table form (TAB, bt_exp.h) or the
-// library's
-template <bool TAB>
-__device__ __forceinline__ double exp_kr(double r, const KParams &kp, const double *tab)
-{
-    if constexpr (TAB) return exp_neg(r, kp.ek, tab);
-    else return exp(-kp.p0 * r);
-}
-template <bool TAB>
-__device__ __forceinline__ double exp_r2(double r2, const KParams &kp, const double *tab)
-{
-    if constexpr (TAB) return exp_neg(r2, kp.eg, tab);
-    else return exp(-r2 * kp.inv_a2);
-}
 
 // ---------------------------------------------------------------------
 // The kernels beside the Coulomb family, FP64, one pair's term with the
@@ -65,9 +47,6 @@ __device__ __forceinline__ double exp_r2(double r2, const KParams &kp, const dou
 // division: atan and MQ jump at d = +-1/2, where the wrap must see the
 // reference's rounding of d.
 // ---------------------------------------------------------------------
-constexpr int KRY = KERNEL_REG_YUKAWA, KAT = KERNEL_ATAN, KSR = KERNEL_SIN_OVER_R, KMQ = KERNEL_MQ,
-              KRU = KERNEL_RBS_U, KRV = KERNEL_RBS_V, KUS = KERNEL_USER;
-
 __device__ __forceinline__ double wrap_half(double d)
 {
     if (d < -0.5) d += 1.0;
@@ -75,37 +54,21 @@ __device__ __forceinline__ double wrap_half(double d)
     return d;
 }
 
-template <int KER, bool SS, bool CHECK, bool TAB>
-__device__ __forceinline__ double other_term(double dx, double dy, double dz, double r2, double a, double b,
-                                             double tq, const KParams &kp, const double *tab)
+// atan, MQ and the RBS kernels (the others of these depend on r alone:
+// term_r2 of bt_pair.h)
+template <int KER>
+__device__ __forceinline__ double other_term(double dx, double dy, double dz, double a, const KParams &kp)
 {
-    if constexpr (KER == KRY) {
-        // r = 0 for coincident points, which this kernel does not skip
-        const double r = TAB ? r2 * rsq64(fmax(r2, 1e-300)) : sqrt(r2);
-        const double e = exp_kr<TAB>(r, kp, tab) * rsq64(r2 + kp.eps2);
-        return (SS ? fma(-tq, b, a) : a) * e;
-    } else if constexpr (KER == KAT) {
+    if constexpr (KER == KAT) {
         const double d = wrap_half(dz / kp.p0);
         return a * (1.0 / M_PI * atan(kp.c1 * tan(M_PI * d)) - d);
     } else if constexpr (KER == KMQ) {
         const double d = wrap_half(dz / kp.p0);
         return a * (0.5 * d * kp.c2 * rsq64(d * d + kp.c1) - d);
-    } else if constexpr (KER == KRU || KER == KRV) {
+    } else {
+        static_assert(KER == KRU || KER == KRV, "other_term: atan, MQ, RBS");
         const double r = fma(dy, dy, dx * dx) + kp.c1;
         return (KER == KRU ? 1.0 : -1.0) / (2.0 * M_PI) * a * (KER == KRU ? dy : dx) / r;
-    } else {  // KSR, KUS
-        const double ir = rsq64(r2);
-        double r = TAB ? r2 * ir : sqrt(r2), v;
-        if constexpr (KER == KSR) {
-            // the sine sees k times r's rounding: one Newton step makes r
-            // as good as the root (half an ulp)
-            if constexpr (TAB) r = fma(fma(-r, r, r2), 0.5 * ir, r);
-            v = (TAB ? sin_kr(r, kp.p0, kp.sn, tab) : sin(kp.p0 * r)) * ir;
-        } else {
-            v = exp_kr<TAB>(r, kp, tab) * ir;
-        }
-        if constexpr (CHECK) v = r > DBL_MIN ? v : 0.0;
-        return a * v;
     }
 }
 
@@ -125,31 +88,14 @@ __device__ __forceinline__ double other_term(double dx, double dy, double dz, do
 // can never trigger; cluster sources never need it (an accepted cluster is
 // separated from its targets).
 // ---------------------------------------------------------------------
-// TAB: exponentials from the table tab.
+// TAB: exponentials and sines from the table tab.
 template <int KER, bool SS, bool CHECK, bool TAB = false>
 __device__ __forceinline__ void pair_pot(double dx, double dy, double dz, double a, double b,
                                          double tq, const KParams &kp, double &acc,
                                          const double *tab = nullptr)
 {
-    const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
-    if constexpr (KER == KC) {
-        double ir = rsq64(r2);
-        if constexpr (CHECK) ir = r2 > (SS ? 0.0 : DBL_MIN) ? ir : 0.0;
-        if constexpr (!SS) acc = fma(a, ir, acc);
-        else acc = fma(fma(-tq * b, exp_r2<TAB>(r2, kp, tab), a), ir, acc);
-    } else if constexpr (KER == KY) {
-        const double ir = rsq64(r2);
-        double e = exp_kr<TAB>(r2 * ir, kp, tab) * ir;
-        if constexpr (CHECK) e = r2 > 0.0 ? e : 0.0;
-        if constexpr (!SS) acc = fma(a, e, acc);
-        else acc = fma(fma(-tq, b, a), e, acc);
-    } else if constexpr (KER == KR) {
-        const double ir = rsq64(r2 + kp.eps2);
-        if constexpr (!SS) acc = fma(a, ir, acc);
-        else acc = fma(fma(-tq * b, exp_r2<TAB>(r2, kp, tab), a), ir, acc);
-    } else {
-        acc += other_term<KER, SS, CHECK, TAB>(dx, dy, dz, r2, a, b, tq, kp, tab);
-    }
+    if constexpr (radial(KER)) pair_r2<KER, SS, CHECK, TAB>(fma(dz, dz, fma(dy, dy, dx * dx)), a, b, tq, kp, acc, tab);
+    else acc += other_term<KER>(dx, dy, dz, a, kp);
 }
 
 // Target-grid form (accumulates Q and, for subtraction, W):
@@ -188,8 +134,10 @@ __device__ __forceinline__ void pair_grid(double dx, double dy, double dz, doubl
     const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
     if constexpr (KER == KC || KER == KY || KER == KR) {
         grid_term<KER, SS, TAB>(r2, a, b, kp, q, w, tab);
+    } else if constexpr (radial(KER)) {
+        q += term_r2<KER, false, false, TAB>(r2, a, 0.0, 0.0, kp, tab);
     } else {
-        q += other_term<KER, false, false, TAB>(dx, dy, dz, r2, a, 0.0, 0.0, kp, tab);
+        q += other_term<KER>(dx, dy, dz, a, kp);
     }
 }
 
@@ -542,7 +490,7 @@ __device__ __forceinline__ void interact_tile(const InteractArgs &A, const Tile 
     const bool clu_check = SCALED && can_close && ctr.w < 0.0;
 
     // source clusters (PC in PC mode, CC in CC mode)
-    const int c0 = A.clu_off[key], c1 = A.clu_off[key + 1];
+    const int c0 = A.clu_off[key], c1 = A.skip_clu ? c0 : A.clu_off[key + 1];
     for (int c = c0; c < c1; ++c) {
         const int id = A.clu_id[c];
         int P = A.P;

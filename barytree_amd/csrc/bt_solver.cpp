@@ -627,6 +627,18 @@ void Plan::build_work()
     for (int node : grid_.key) node_rows_off_[node + 1]++;
     for (int n = 0; n < ntnodes_; n++) node_rows_off_[n + 1] += node_rows_off_[n];
     make_queue_tiles(near_, tile_targets_, false, P, near_tiles_, near_qlen_);
+    // cluster tiles, keys with the most clusters first (ties in key order)
+    pc_tiles_.clear();
+    if (p.approximation == A_LAGRANGE) {
+        std::vector<int> ks;
+        for (size_t k = 0; k < near_.key.size(); k++)
+            if (near_.clu_off[k + 1] > near_.clu_off[k]) ks.push_back((int)k);
+        auto load = [&](int k) { return near_.clu_off[k + 1] - near_.clu_off[k]; };
+        std::stable_sort(ks.begin(), ks.end(), [&](int a, int b) { return load(a) > load(b); });
+        for (int k : ks)
+            for (int o = 0; o < near_.tcnt[k]; o += btk::PC_TILE)
+                pc_tiles_.push_back(btk::Tile{k, near_.tbeg[k] + o, std::min(btk::PC_TILE, near_.tcnt[k] - o), 0});
+    }
     make_queue_tiles(grid_, GRID_TILE, true, P, grid_tiles_, grid_qlen_);
     make_pencil_tiles(grid_, P, false, pencil_tiles_);
 
@@ -755,6 +767,10 @@ std::string Plan::validate() const
     std::string e = chk_csr(near_, near_tiles_, false);
     if (!e.empty()) return "near " + e;
     if (near_ctr_.size() != 4 * near_.key.size()) return "near centres";
+    for (const btk::Tile &t : pc_tiles_)
+        if (t.x < 0 || t.x >= (int)near_.key.size() || t.y < 0 || t.z <= 0 || t.z > btk::PC_TILE ||
+            (long long)t.y + t.z > M_)
+            return "cluster tile";
     if (sym_) {
         if (sym_ctr_.size() != 4 * sym_items_.size() || sym_items_.size() > (size_t)INT32_MAX) return "sym items";
         for (const btk::SymItem &it : sym_items_) {
@@ -1322,6 +1338,7 @@ std::string Plan::finish_create(const PlanInput &in, bool host_only, double t2)
     };
     if (!(r = up_csr(near_, &d_nseg_off_, &d_nsegs_, &d_nclu_off_, &d_nclu_id_)).empty()) return r;
     if (!(r = up(&d_near_tiles_, near_tiles_)).empty()) return r;
+    if (!pc_tiles_.empty() && !(r = up(&d_pc_tiles_, pc_tiles_)).empty()) return r;
     if (!(r = up(&d_near_ctr_, near_ctr_)).empty()) return r;
     if (sym_) {
         if (!(r = up(&d_sym_items_, sym_items_)).empty()) return r;
@@ -1412,6 +1429,27 @@ std::string Plan::down_fixed()
     }
     d.mode = 1; d.tiles = d_leaf_tiles_; d.nblocks = (int)leaf_tiles_.size();
     HIPCHK(btk::launch_down(d, st_));
+    return "";
+}
+
+bool Plan::pc_run() const
+{
+    const Params &p = prm_;
+    const bool fp64 = p.precision != PREC_MIXED || !coulomb_family(p.kernel);
+    return fp64 && !pc_tiles_.empty() &&
+           (coulomb_family(p.kernel) || p.kernel == K_REG_YUKAWA || p.kernel == K_SIN_OVER_R || p.kernel == K_USER);
+}
+
+std::string Plan::launch_pc()
+{
+    btk::PcArgs a{};
+    a.kernel = prm_.kernel; a.singularity = prm_.singularity;
+    a.ntiles = (int)pc_tiles_.size(); a.nl = prm_.degree + 1;
+    a.tiles = d_pc_tiles_; a.clu_off = d_nclu_off_; a.clu_id = d_nclu_id_;
+    a.tab = d_stab_; a.cq = d_cq_; a.cw = d_cw_;
+    a.tx = d_tx_; a.ty = d_ty_; a.tz = d_tz_; a.tq = d_tq_;
+    a.kp = kp_; a.pot = d_pot_;
+    HIPCHK(btk::launch_pc64(a, st_));
     return "";
 }
 
@@ -1600,7 +1638,12 @@ std::string Plan::execute(bool timed)
         a.skip_sym = sym_ready() ? 1 : 0;
         std::copy(near_qlen_, near_qlen_ + NXCD, a.qlen);
         a.cursor = d_cursor_;
+        a.skip_clu = pc_run() ? 1 : 0;
         HIPCHK(btk::launch_interact(a, st_));
+        if (a.skip_clu) {
+            std::string r = launch_pc();
+            if (!r.empty()) return r;
+        }
         if (a.skip_sym) {
             std::string r = near_sym(!ov);
             if (!r.empty()) return r;

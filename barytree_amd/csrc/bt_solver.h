@@ -215,6 +215,11 @@ private:
     // the item launch runs in this execution's precision: always for a
     // symmetric plan, in mixed precision for one-sided items only
     bool items_run() const { return sym_ && sym_enabled_ && (sym_ok_ || prm_.precision == PREC_MIXED); }
+    // the near keys' clusters run in launch_pc64: Lagrange, FP64 arithmetic
+    // (the kernels beside the Coulomb family in either precision), kernels
+    // of r alone
+    bool pc_run() const;
+    std::string launch_pc();
     std::string upward_fixed();  // upward pass at the plan's degree
     std::string down_fixed();    // downpass at the plan's degree
     bool sym_ready();  // items_run(), and the slots allocated (at the first execution that uses them)
@@ -266,6 +271,10 @@ private:
     std::vector<System> sys_;
     WorkCSR near_, grid_;
     std::vector<btk::Tile> near_tiles_, grid_tiles_, leaf_tiles_;
+    // FP64 executions at the plan's degree take the near keys' clusters in a
+    // launch of their own (pc_run): tiles of the keys with clusters,
+    // heaviest first
+    std::vector<btk::Tile> pc_tiles_;
     // grid keys write rows of partial grid values (row of key k at
     // grid_row_[k]); node n sums rows [node_rows_off_[n], node_rows_off_[n+1])
     // per near key: centre of its target node and the r^2 below which the
@@ -372,6 +381,7 @@ private:
     double *d_up_Qe_ = nullptr, *d_up_We_ = nullptr;
     int *d_down_nodes_ = nullptr;
     btk::Tile *d_near_tiles_ = nullptr, *d_grid_tiles_ = nullptr, *d_leaf_tiles_ = nullptr;
+    btk::Tile *d_pc_tiles_ = nullptr;
     // grid_ keys, one tile each (the tensor-grid launch of mixed executions)
     std::vector<btk::Tile> pencil_tiles_;
     btk::Tile *d_pencil_tiles_ = nullptr;
