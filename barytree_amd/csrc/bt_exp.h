@@ -56,14 +56,17 @@ __device__ __forceinline__ void exp_table(double *tab, int tid)
 // has |a| <= 6.2e-3, so sin a to degree 5 is truncated below 1.1e-17
 // relative and cos a to degree 4 below 8e-17.  Within about 1.5 ulp of 1
 // besides the rounding of k r's own size.  Beyond sr.rmax (c r >= 2^50) the
-// library's sin; a NaN r gives NaN.
+// library's sin (GUARD; without it the caller keeps r below rmax); a NaN r
+// gives NaN.
 //
 // 12 FP64 instructions and one 16-byte table read.  The library's sin (with
 // its reduction for every magnitude) and the square root took most of a
 // pair: N = 200k particle-cluster, degree 5, 1.4e10 pairs 55.4 -> 26.1 ms.
+template <bool GUARD = true>
 __device__ __forceinline__ double sin_kr(double r, double k, const SinRate &sr, const double *tab)
 {
-    if (__builtin_expect(r >= sr.rmax, 0)) return sin(k * r);
+    if constexpr (GUARD)
+        if (__builtin_expect(r >= sr.rmax, 0)) return sin(k * r);
     constexpr double MAGIC = 0x1.8p52;
     constexpr double S1 = 0.01227184630308513, S3 = -3.080196845561248e-07, S5 = 2.3193606829202922e-12;  // (2 pi/512)^k / k!
     constexpr double C2 = -7.529910584327208e-05, C4 = 9.44992556799382e-10;

@@ -159,7 +159,8 @@ hipError_t launch_pc64(const PcArgs &a, hipStream_t st);
 
 // Item launch of the near field's particle pairs (Coulomb and Yukawa with
 // either singularity, regularized Coulomb with skipping; FP64 or mixed
-// precision): one system whose targets are its sources, or (one-sided items
+// precision; regularized Yukawa, sin-over-r and the user kernel with
+// skipping in FP64): one system whose targets are its sources, or (one-sided items
 // only) one system with other targets.  A two-sided item (cslot >= 0) is a pair
 // of distinct leaves A, B, each in the other's near list: every pair (a, b)
 // is evaluated once and gives both a's term from b and b's term from a.

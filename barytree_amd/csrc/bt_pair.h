@@ -43,8 +43,8 @@ __device__ __forceinline__ double exp_r2(double r2, const KParams &kp, const dou
 
 // Regularized Yukawa, sin-over-r and the user example: one pair's term
 // (r by r^2 rsq64(r^2) with TAB, about 1 ulp; r = 0 for coincident points,
-// which the regularized kernel does not skip).
-template <int KER, bool SS, bool CHECK, bool TAB>
+// which the regularized kernel does not skip).  GUARD as for sin_kr.
+template <int KER, bool SS, bool CHECK, bool TAB, bool GUARD = true>
 __device__ __forceinline__ double term_r2(double r2, double a, double b, double tq, const KParams &kp,
                                           const double *tab)
 {
@@ -60,7 +60,7 @@ __device__ __forceinline__ double term_r2(double r2, double a, double b, double 
             // the sine sees k times r's rounding: one Newton step makes r
             // as good as the root (half an ulp)
             if constexpr (TAB) r = fma(fma(-r, r, r2), 0.5 * ir, r);
-            v = (TAB ? sin_kr(r, kp.p0, kp.sn, tab) : sin(kp.p0 * r)) * ir;
+            v = (TAB ? sin_kr<GUARD>(r, kp.p0, kp.sn, tab) : sin(kp.p0 * r)) * ir;
         } else {
             v = exp_kr<TAB>(r, kp, tab) * ir;
         }

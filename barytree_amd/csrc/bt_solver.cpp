@@ -1167,19 +1167,23 @@ std::string Plan::finish_create(const PlanInput &in, bool host_only, double t2)
     }
 
     herm_ = prm.approximation == A_HERMITE;
-    // symmetric near field: one system (Coulomb or Yukawa, or regularized
-    // Coulomb with skipping; either approximation, which only concerns the
-    // far field) whose targets are its sources, particle for particle in
-    // tree order (the same order after both tree builds)
+    // symmetric near field: one system (Coulomb or Yukawa, or the other
+    // kernels of r alone with skipping; either approximation, which only
+    // concerns the far field) whose targets are its sources, particle for
+    // particle in tree order (the same order after both tree builds);
+    // analyses report it for the Coulomb family
+    const bool sym_kernel =
+        prm.kernel == K_COULOMB || prm.kernel == K_YUKAWA ||
+        (prm.singularity == S_SKIPPING &&
+         (prm.kernel == K_REG_COULOMB || prm.kernel == K_REG_YUKAWA || prm.kernel == K_SIN_OVER_R ||
+          prm.kernel == K_USER));
     sym_ok_ = false;
-    if (sys_.size() == 1 &&
-        (prm.kernel == K_COULOMB || prm.kernel == K_YUKAWA ||
-         (prm.kernel == K_REG_COULOMB && prm.singularity == S_SKIPPING))) {
+    if (sys_.size() == 1 && sym_kernel) {
         const System &y = sys_[0];
         if (dev_tree_) {
             // one tree and one set of arrays serve as sources and targets
             sym_ok_ = shared_;
-        } else {
+        } else if (coulomb_family(prm.kernel)) {
             auto same = [&](const HostVec<double> &u, const HostVec<double> &v) {
                 return std::memcmp(u.data(), v.data(), (size_t)y.M * sizeof(double)) == 0;
             };
@@ -1435,8 +1439,7 @@ std::string Plan::down_fixed()
 bool Plan::pc_run() const
 {
     const Params &p = prm_;
-    const bool fp64 = p.precision != PREC_MIXED || !coulomb_family(p.kernel);
-    return fp64 && !pc_tiles_.empty() &&
+    return fp64_arithmetic() && !pc_tiles_.empty() &&
            (coulomb_family(p.kernel) || p.kernel == K_REG_YUKAWA || p.kernel == K_SIN_OVER_R || p.kernel == K_USER);
 }
 
@@ -1479,7 +1482,7 @@ std::string Plan::launch_items()
     btk::SymArgs a{};
     a.kernel = prm_.kernel;
     a.singularity = prm_.singularity;
-    a.fp64 = prm_.precision == PREC_MIXED ? 0 : 1;
+    a.fp64 = fp64_arithmetic() ? 1 : 0;
     a.nitems = (int)sym_items_.size();
     a.items = d_sym_items_;
     a.ctr = reinterpret_cast<const double4 *>(d_sym_ctr_);

@@ -212,6 +212,9 @@ private:
     // (sym_ok_), one-sided items only otherwise (items_ok_); set by create
     void build_sym(const System &sy, const std::vector<int> &keys, const std::vector<std::vector<int>> &segs_of,
                    std::vector<std::vector<char>> &sym_of, bool symmetric);
+    // this execution's pairs are evaluated in FP64: the plain precision, and
+    // the kernels beside the Coulomb family in either
+    bool fp64_arithmetic() const { return prm_.precision != PREC_MIXED || !coulomb_family(prm_.kernel); }
     // the item launch runs in this execution's precision: always for a
     // symmetric plan, in mixed precision for one-sided items only
     bool items_run() const { return sym_ && sym_enabled_ && (sym_ok_ || prm_.precision == PREC_MIXED); }
@@ -282,7 +285,8 @@ private:
     // (negated: the key's clusters are checked too)
     std::vector<double> near_ctr_;
     // Item launch of the near field's particle pairs (Coulomb or Yukawa, or
-    // regularized Coulomb with skipping).  Symmetric plans (sym_ok_: one
+    // regularized Coulomb, regularized Yukawa, sin-over-r or the user kernel
+    // with skipping).  Symmetric plans (sym_ok_: one
     // system whose targets are its sources, the same particles in the same
     // tree order): pairs of near-field keys (A, B), each key's particle
     // range a source range of the other's near list, are evaluated once for

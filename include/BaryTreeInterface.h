@@ -127,8 +127,10 @@ typedef struct BaryTreeStats {
                                 symmetric near field delivers (either precision):
                                 a single system whose targets are its sources in
                                 the same tree order (Coulomb, Yukawa, or
-                                regularized Coulomb with skipping; Lagrange or
-                                Hermite); pairs of
+                                regularized Coulomb, regularized Yukawa,
+                                sin-over-r or the user kernel with skipping, the
+                                last three in FP64 and in plans, not in analyses;
+                                Lagrange or Hermite); pairs of
                                 two leaves in each other's near list are
                                 evaluated once for both particles, the rest once
                                 for their target; 0 otherwise or when switched

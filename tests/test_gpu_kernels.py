@@ -61,3 +61,29 @@ def test_other_kernels_reject_learned_degrees(bt):
     with bt.Plan(t, src, 8, [1.5], 1, 1, 1, 0.7, 3, 60, 60) as p:
         with pytest.raises(RuntimeError, match="per-pair degrees"):
             p.set_pair_degrees(np.full(p.num_pairs(), 3))
+
+
+@pytest.mark.parametrize("k", [4, 8, 12])
+@pytest.mark.parametrize("ct,leaf", [(1, 300), (2, 33), (3, 130), (1, 7)])
+def test_other_kernels_targets_equal_sources(bt, oracle_mod, k, ct, leaf):
+    """Targets equal to the sources: the near field evaluates each pair of
+    two leaves once for both particles.  Two particles at one point (the
+    regularized kernel does not skip them, the others do), one leaf pass with
+    a remainder, the one-directional form, and the mixed precision request,
+    which runs in FP64."""
+    rng = np.random.default_rng(10 * ct + k)
+    x, y, z, q = (rng.uniform(-1, 1, 5000) for _ in range(4))
+    x[40], y[40], z[40] = x[41], y[41], z[41]
+    t, src = (x.copy(), y.copy(), z.copy(), q.copy()), (x, y, z, q, np.ones(5000))
+    args = (k, KP_OTHER[k], 1, 1, ct, 0.7, 3, leaf, leaf)
+    ref = oracle_mod.treecode(*t, *src, *args)
+    with bt.Plan(t, src, *args) as p:
+        st = p.stats()
+        assert st["sym_ptwise"] > 0.5 * st["pp_ptwise"] and st["sym_evals"] < st["sym_ptwise"], st
+        got = p.execute()
+        assert np.array_equal(got, p.execute())
+        p.set_symmetric(False)
+        assert p.stats()["sym_ptwise"] == 0
+        one = p.execute()
+    assert rel_l2(ref, got) <= TOL_FP64 and rel_l2(ref, one) <= TOL_FP64
+    assert np.array_equal(got, bt.solve(t, src, *args, precision=bt.PRECISION_MIXED))
