@@ -91,6 +91,32 @@ void split_keys(const WorkCSR &in, long long max_src, int P, bool multi, WorkCSR
     }
 }
 
+// Most source points of a grid key: MAX_KEY_SOURCES where that gives the
+// launch (one block per key and chunk of its sources) GRID_BLOCKS blocks, else
+// chunks that give about four times as many, of 2^20 pairs or more (a row of
+// P sums per chunk is written and added up after it).  Cluster-particle
+// far fields with few target nodes: Coulomb with subtraction, FP64, N = 100k,
+// degree 9, 9.9-13.7 ms with chunks of 16384, 5.4 ms so; Yukawa, mixed, 65k
+// sources, 0.77 -> 0.33 ms (150 blocks for 256 CUs before).  Where the chunks
+// of 16384 fill the chip, finer ones only add rows to sum (cluster-cluster,
+// mixed, N = 300k, degree 4: 0.6 -> 1.2 ms).
+long long grid_key_sources(const WorkCSR &w, int P, bool multi)
+{
+    long long all = 0, blocks = 0;
+    double pairs = 0.0;
+    for (size_t k = 0; k < w.key.size(); k++) {
+        long long src = 0;
+        for (int c = w.clu_off[k]; c < w.clu_off[k + 1]; c++) src += cluster_points(w.clu_id[c], P, multi);
+        for (int s = w.seg_off[k]; s < w.seg_off[k + 1]; s++) src += w.seg_cnt[s];
+        all += src;
+        blocks += (src + MAX_KEY_SOURCES - 1) / MAX_KEY_SOURCES;
+        pairs += (double)src * w.tcnt[k];
+    }
+    if (blocks >= GRID_BLOCKS || pairs <= 0.0) return MAX_KEY_SOURCES;
+    const long long work = (long long)((1 << 20) * ((double)all / pairs));
+    return std::min(MAX_KEY_SOURCES, std::max({1024LL, work, all / (4 * GRID_BLOCKS)}));
+}
+
 void make_queue_tiles(const WorkCSR &w, int tile_t, bool grid, int P, std::vector<btk::Tile> &tiles,
                       int *qlen, bool multi)
 {
@@ -574,6 +600,12 @@ void Plan::build_work()
                 close_key(gw);
             }
         }
+        // heavy grid keys are split by sources; every key writes its own row
+        // (systems of a batch are split as they are alone)
+        if (!gw.key.empty()) {
+            const WorkCSR raw = std::move(gw);
+            split_keys(raw, grid_key_sources(raw, P, false), P, false, gw);
+        }
     };
     auto csr_start = [](WorkCSR &w) { w.seg_off.assign(1, 0); w.clu_off.assign(1, 0); };
     csr_start(near_);
@@ -612,11 +644,6 @@ void Plan::build_work()
         }
     }
 
-    // heavy grid keys are split by sources; every key writes its own row
-    {
-        WorkCSR raw = std::move(grid_);
-        split_keys(raw, MAX_KEY_SOURCES, P, false, grid_);
-    }
     grid_row_.assign(grid_.key.size(), 0);
     grid_rows_len_ = 0;
     for (size_t k = 0; k < grid_.key.size(); k++) {

@@ -22,8 +22,9 @@ namespace bt {
 constexpr int DOWN_TILE = 1024;  // targets per block of the leaf downpass
 constexpr int GRID_TILE = 512;   // grid points per block of grid-target tiles (2 per thread)
 constexpr int PART_MAX = 16384;  // particles per block of a source slot's charges
-constexpr long long MAX_KEY_SOURCES = 1 << 14;  // source points per grid key (heavier keys are split:
-                                                 // blocks enough to fill the GPU)
+constexpr long long MAX_KEY_SOURCES = 1 << 14;  // source points per grid key at most (heavier keys are
+                                                 // split, further in small plans: grid_key_sources)
+constexpr int GRID_BLOCKS = 512;                 // fewest blocks of a grid launch (2 per CU)
 constexpr int SMALL_TARGETS = 1 << 18;  // single-system plans below this many targets: 1 target per thread
 
 struct Timings {
@@ -99,6 +100,7 @@ void make_pencil_tiles(const WorkCSR &w, int P, bool multi, std::vector<btk::Til
 // max_src into consecutive chunks of its particle ranges and clusters; the
 // chunks are keys of their own with the same node and targets, in order.
 void split_keys(const WorkCSR &in, long long max_src, int P, bool multi, WorkCSR &out);
+long long grid_key_sources(const WorkCSR &w, int P, bool multi);
 
 struct PlanInput {
     int nsys = 1;

@@ -263,7 +263,7 @@ std::string Plan::set_pair_degrees(const int *deg)
             raw.clu_off.push_back((int)raw.clu_id.size());
         }
     }
-    split_keys(raw, MAX_KEY_SOURCES, 0, true, vfar_);
+    split_keys(raw, grid_key_sources(raw, 0, true), 0, true, vfar_);
     vfar_row_.assign(vfar_.key.size(), 0);
     vfar_rows_len_ = 0;
     for (size_t k = 0; k < vfar_.key.size(); k++) {

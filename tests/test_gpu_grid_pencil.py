@@ -92,3 +92,27 @@ def test_pencil_grids_fp64_mixed_degrees_in_one_launch(bt, oracle_mod, ct, k, s)
     err = rel_l2(ref, got)
     print(f"FP64 vs oracle {err:.2e}", flush=True)
     assert err <= 1e-12
+
+
+@pytest.mark.parametrize("ct,k,s", [(2, 1, 1), (2, 1, 2), (3, 3, 1)])
+def test_grids_with_few_target_nodes(bt, oracle_mod, ct, k, s):
+    """Few grid keys: their sources are cut into finer chunks, whose length
+    depends on the whole plan (degrees 2 and 12: limited by the pairs of a
+    chunk, or by its 1024 sources).  In a batch each system is cut as it is
+    alone: the same bits."""
+    rng = np.random.default_rng(ct + k)
+    for deg in (2, 12):
+        print(f"case ct={ct} kernel={k} singularity={s} degree={deg}", flush=True)
+        systems = [uniform_cube(n, m, seed=int(rng.integers(99))) for m, n in ((3000, 4000), (700, 20000))]
+        leaf = 110
+        args = (k, KP[k][s], s, 1, ct, 0.7, deg, leaf, leaf)
+        got = [bt.solve(t, src, *args, size_check=0.0) for t, src in systems]
+        for (t, src), g in zip(systems, got):
+            ref = oracle_mod.treecode(*t, *src, *args, size_check=0.0)
+            assert oracle_mod.last_stats()["num_cc"] + oracle_mod.last_stats()["num_cp"] > 0
+            assert rel_l2(ref, g) <= 1e-12
+        if k == s == 1:
+            with bt.Plan.batched(systems, *args[:7], max_source_leaf=leaf, max_target_leaf=leaf,
+                                 size_check=0.0) as p:
+                both = p.execute()
+            assert np.array_equal(both, np.concatenate(got))
