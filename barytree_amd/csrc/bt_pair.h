@@ -17,6 +17,9 @@ constexpr bool radial(int ker)
 }
 // the kernel's FP64 evaluation reads the table of exp_neg or of sin_kr
 constexpr bool exp_kernel(int ker, bool ss) { return ker == KY || ker == KRY || ker == KUS || (ss && ker != KSR); }
+// the subtraction's Gaussian e^{-r^2/a^2} as the product of e^{-dx^2/a^2} and
+// e^{-(dy^2+dz^2)/a^2}, which tensor grids share over their pencils
+constexpr bool separable_gauss(int ker, bool ss) { return ss && (ker == KC || ker == KR); }
 // doubles of that table (1 without one)
 constexpr int pair_table_len(int ker, bool ss) { return ker == KSR ? 2 * SIN_TAB : (exp_kernel(ker, ss) ? EXP_TAB : 1); }
 template <int KER, bool SS>

@@ -116,3 +116,22 @@ def test_grids_with_few_target_nodes(bt, oracle_mod, ct, k, s):
                                  size_check=0.0) as p:
                 both = p.execute()
             assert np.array_equal(both, np.concatenate(got))
+
+
+@pytest.mark.parametrize("ct", [1, 2, 3])
+@pytest.mark.parametrize("kappa", [0.01, 30.0])
+def test_gaussian_as_a_product_over_the_dimensions(bt, oracle_mod, ct, kappa):
+    """Subtraction with Gaussians whose factors underflow (kappa = 0.01:
+    exponents to 1e5) or stay near 1, on grids whose pencils fill the block
+    evenly and unevenly."""
+    t, src = uniform_cube(5000, 4000, seed=7)
+    for k, kp in ((1, [kappa]), (3, [0.05, kappa])):
+        if k == 3 and ct > 1:
+            continue
+        for deg in (1, 7, 9):
+            print(f"case ct={ct} kernel={k} kappa={kappa} degree={deg}", flush=True)
+            args = (k, kp, 2, 1, ct, 0.7, deg, 110, 110)
+            ref = oracle_mod.treecode(*t, *src, *args, size_check=0.0)
+            st = oracle_mod.last_stats()
+            assert st["num_cc"] + st["num_cp"] + st["num_pc"] > 0
+            assert rel_l2(ref, bt.solve(t, src, *args, size_check=0.0)) <= 1e-12
