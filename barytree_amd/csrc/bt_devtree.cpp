@@ -103,29 +103,33 @@ std::string device_build_trees(DevParticles &p, const std::vector<DevRoot> &root
     Grow<btk::TreeSeg> d_segs;
     Grow<double> d_part;
     Grow<int> d_low;
-    std::vector<btk::TreeChunk> chunks;
-    std::vector<btk::TreeSeg> segs;
+    // Two sets of a pass's host arrays: a set is used again two passes later,
+    // after the wait for the counts of the pass between, so a pass does not
+    // wait for its own copies and scatter.
+    std::vector<btk::TreeChunk> box_chunks, chunk_set[2];
+    std::vector<btk::TreeSeg> seg_set[2];
+    int set = 0;
     std::vector<double> part;
     std::vector<int> low;
 
     while (!cur.empty()) {
         // 1. exact bounding boxes of the level's nodes
-        chunks.clear();
-        for (size_t k = 0; k < cur.size(); k++) add_chunks(chunks, (int)k, all[cur[k]].b, all[cur[k]].e);
-        HIPCHK(d_chunks.fit(chunks.size()));
-        HIPCHK(d_part.fit(6 * chunks.size()));
-        HIPCHK(hipMemcpyAsync(d_chunks.p, chunks.data(), chunks.size() * sizeof(btk::TreeChunk),
+        box_chunks.clear();
+        for (size_t k = 0; k < cur.size(); k++) add_chunks(box_chunks, (int)k, all[cur[k]].b, all[cur[k]].e);
+        HIPCHK(d_chunks.fit(box_chunks.size()));
+        HIPCHK(d_part.fit(6 * box_chunks.size()));
+        HIPCHK(hipMemcpyAsync(d_chunks.p, box_chunks.data(), box_chunks.size() * sizeof(btk::TreeChunk),
                               hipMemcpyHostToDevice, st));
-        HIPCHK(btk::launch_tree_bbox((int)chunks.size(), d_chunks.p, p.x, p.y, p.z, d_part.p, st));
-        part.resize(6 * chunks.size());
+        HIPCHK(btk::launch_tree_bbox((int)box_chunks.size(), d_chunks.p, p.x, p.y, p.z, d_part.p, st));
+        part.resize(6 * box_chunks.size());
         HIPCHK(hipMemcpyAsync(part.data(), d_part.p, part.size() * sizeof(double), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         std::vector<int> first(cur.size(), -1);
-        for (size_t c = 0; c < chunks.size(); c++) {
-            NodeRec &r = all[cur[chunks[c].seg]].rec;
+        for (size_t c = 0; c < box_chunks.size(); c++) {
+            NodeRec &r = all[cur[box_chunks[c].seg]].rec;
             const double *v = &part[6 * c];
-            if (first[chunks[c].seg] < 0) {
-                first[chunks[c].seg] = (int)c;
+            if (first[box_chunks[c].seg] < 0) {
+                first[box_chunks[c].seg] = (int)c;
                 r.lo[0] = v[0]; r.hi[0] = v[1]; r.lo[1] = v[2]; r.hi[1] = v[3]; r.lo[2] = v[4]; r.hi[2] = v[5];
                 continue;
             }
@@ -153,6 +157,8 @@ std::string device_build_trees(DevParticles &p, const std::vector<DevRoot> &root
         // 3. one partition pass per split dimension (the r-th set dimension
         // of each node in pass r), copying every other particle through
         for (int pass = 0; pass < 3; pass++) {
+            std::vector<btk::TreeChunk> &chunks = chunk_set[set];
+            std::vector<btk::TreeSeg> &segs = seg_set[set];
             segs.clear();
             std::vector<std::pair<int, int>> owner;  // (split, range) of each split segment
             std::vector<int> sdim(splits.size(), -1);
@@ -210,8 +216,7 @@ std::string device_build_trees(DevParticles &p, const std::vector<DevRoot> &root
                                   hipMemcpyHostToDevice, st));
             HIPCHK(btk::launch_tree_scatter((int)chunks.size(), d_chunks.p, d_segs.p, p.x, p.y, p.z, p.idx, p.x2,
                                             p.y2, p.z2, p.idx2, st));
-            // the host vectors are reused in the next pass: let the copies finish
-            HIPCHK(hipStreamSynchronize(st));
+            set ^= 1;
             std::swap(p.x, p.x2); std::swap(p.y, p.y2); std::swap(p.z, p.z2); std::swap(p.idx, p.idx2);
             // the ranges after the pass, as the host builder arranges them:
             // range i keeps its lower part, range nr + i gets the upper part
@@ -239,7 +244,10 @@ std::string device_build_trees(DevParticles &p, const std::vector<DevRoot> &root
         for (const Split &s : splits) {
             int nonempty = 0;
             for (int i = 0; i < s.nr; i++) nonempty += s.rb[i] < s.re[i];
-            if (nonempty == 1) return COINCIDENT_ERROR;
+            if (nonempty == 1) {
+                HIPCHK(hipStreamSynchronize(st));  // the last pass
+                return COINCIDENT_ERROR;
+            }
             for (int i = 0; i < s.nr; i++) {
                 if (s.rb[i] >= s.re[i]) continue;
                 BNode c{};

@@ -52,43 +52,73 @@ long long cluster_points(int id, int P, bool multi)
     const long long nl = (id >> btk::DEG_SHIFT) + 1;
     return nl * nl * nl;
 }
+
+// keys, nodes or leaves above which their loops are shared by threads (a
+// parallel region costs a small plan more than it gives)
+constexpr int PAR_KEYS = 256;
+
+// source points of every key
+std::vector<long long> key_sources(const WorkCSR &w, int P, bool multi)
+{
+    const int nk = (int)w.key.size();
+    std::vector<long long> src(nk);
+#pragma omp parallel for schedule(static) if (nk > PAR_KEYS)
+    for (int k = 0; k < nk; k++) {
+        long long n = 0;
+        for (int s = w.seg_off[k]; s < w.seg_off[k + 1]; s++) n += w.seg_cnt[s];
+        if (!multi) n += (long long)(w.clu_off[k + 1] - w.clu_off[k]) * P;
+        else
+            for (int c = w.clu_off[k]; c < w.clu_off[k + 1]; c++) n += cluster_points(w.clu_id[c], P, multi);
+        src[k] = n;
+    }
+    return src;
+}
+
+// (-work, key), the heaviest key first and ties in key order
+void sort_keys(std::vector<std::pair<long long, int>> &ks)
+{
+    if (ks.size() > 64 * PAR_KEYS) __gnu_parallel::sort(ks.begin(), ks.end());
+    else std::sort(ks.begin(), ks.end());
+}
 }  // namespace
 
-void split_keys(const WorkCSR &in, long long max_src, int P, bool multi, WorkCSR &out)
+void split_keys(WorkCSR &&in, long long max_src, int P, bool multi, WorkCSR &out)
 {
+    const std::vector<long long> src = key_sources(in, P, multi);
+    if (std::none_of(src.begin(), src.end(), [&](long long n) { return n > max_src; })) {
+        out = std::move(in);
+        return;
+    }
+    // the lists stay as they are: only keys and offsets change
     out = WorkCSR();
     out.seg_off.push_back(0);
     out.clu_off.push_back(0);
     out.pairs = in.pairs;
-    auto open_key = [&](size_t k) {
-        out.key.push_back(in.key[k]); out.tbeg.push_back(in.tbeg[k]); out.tcnt.push_back(in.tcnt[k]);
-    };
-    auto close_key = [&]() {
-        out.seg_off.push_back((int)out.seg_beg.size());
-        out.clu_off.push_back((int)out.clu_id.size());
-    };
     for (size_t k = 0; k < in.key.size(); k++) {
-        open_key(k);
-        long long load = 0;
-        bool empty = true;
-        for (int c = in.clu_off[k]; c < in.clu_off[k + 1]; c++) {
-            const long long w = cluster_points(in.clu_id[c], P, multi);
-            if (!empty && load + w > max_src) { close_key(); open_key(k); load = 0; }
-            out.clu_id.push_back(in.clu_id[c]);
-            load += w;
-            empty = false;
+        // the key's chunk up to range s1 and cluster c1
+        auto chunk = [&](int s1, int c1) {
+            out.key.push_back(in.key[k]); out.tbeg.push_back(in.tbeg[k]); out.tcnt.push_back(in.tcnt[k]);
+            out.seg_off.push_back(s1);
+            out.clu_off.push_back(c1);
+        };
+        if (src[k] > max_src) {
+            long long load = 0;
+            bool empty = true;
+            auto add = [&](long long w, int s1, int c1) {
+                if (!empty && load + w > max_src) { chunk(s1, c1); load = 0; }
+                load += w;
+                empty = false;
+            };
+            for (int c = in.clu_off[k]; c < in.clu_off[k + 1]; c++)
+                add(cluster_points(in.clu_id[c], P, multi), in.seg_off[k], c);
+            for (int s = in.seg_off[k]; s < in.seg_off[k + 1]; s++) add(in.seg_cnt[s], s, in.clu_off[k + 1]);
         }
-        for (int s = in.seg_off[k]; s < in.seg_off[k + 1]; s++) {
-            const long long w = in.seg_cnt[s];
-            if (!empty && load + w > max_src) { close_key(); open_key(k); load = 0; }
-            out.seg_beg.push_back(in.seg_beg[s]);
-            out.seg_cnt.push_back(in.seg_cnt[s]);
-            out.seg_chk.push_back(in.seg_chk[s]);
-            load += w;
-            empty = false;
-        }
-        close_key();
+        chunk(in.seg_off[k + 1], in.clu_off[k + 1]);
     }
+    out.seg_beg = std::move(in.seg_beg);
+    out.seg_cnt = std::move(in.seg_cnt);
+    out.seg_chk = std::move(in.seg_chk);
+    out.clu_id = std::move(in.clu_id);
 }
 
 // Most source points of a grid key: MAX_KEY_SOURCES where that gives the
@@ -102,15 +132,13 @@ void split_keys(const WorkCSR &in, long long max_src, int P, bool multi, WorkCSR
 // mixed, N = 300k, degree 4: 0.6 -> 1.2 ms).
 long long grid_key_sources(const WorkCSR &w, int P, bool multi)
 {
+    const std::vector<long long> src = key_sources(w, P, multi);
     long long all = 0, blocks = 0;
     double pairs = 0.0;
-    for (size_t k = 0; k < w.key.size(); k++) {
-        long long src = 0;
-        for (int c = w.clu_off[k]; c < w.clu_off[k + 1]; c++) src += cluster_points(w.clu_id[c], P, multi);
-        for (int s = w.seg_off[k]; s < w.seg_off[k + 1]; s++) src += w.seg_cnt[s];
-        all += src;
-        blocks += (src + MAX_KEY_SOURCES - 1) / MAX_KEY_SOURCES;
-        pairs += (double)src * w.tcnt[k];
+    for (size_t k = 0; k < src.size(); k++) {
+        all += src[k];
+        blocks += (src[k] + MAX_KEY_SOURCES - 1) / MAX_KEY_SOURCES;
+        pairs += (double)src[k] * w.tcnt[k];
     }
     if (blocks >= GRID_BLOCKS || pairs <= 0.0) return MAX_KEY_SOURCES;
     const long long work = (long long)((1 << 20) * ((double)all / pairs));
@@ -120,53 +148,43 @@ long long grid_key_sources(const WorkCSR &w, int P, bool multi)
 void make_queue_tiles(const WorkCSR &w, int tile_t, bool grid, int P, std::vector<btk::Tile> &tiles,
                       int *qlen, bool multi)
 {
-    struct Group { long long work; std::vector<btk::Tile> t; };
-    std::vector<Group> groups;
-    for (size_t k = 0; k < w.key.size(); k++) {
-        long long src = 0;
-        for (int s = w.seg_off[k]; s < w.seg_off[k + 1]; s++) src += w.seg_cnt[s];
-        for (int c = w.clu_off[k]; c < w.clu_off[k + 1]; c++) src += cluster_points(w.clu_id[c], P, multi);
-        Group g{0, {}};
-        for (int o = 0; o < w.tcnt[k]; o += tile_t) {
-            btk::Tile t;
-            t.x = (int)k;
-            t.y = w.tbeg[k] + o;
-            t.z = std::min(tile_t, w.tcnt[k] - o);
-            t.w = grid ? w.key[k] : 0;
-            g.work += (src + 1) * t.z;
-            g.t.push_back(t);
-        }
-        if (!g.t.empty()) groups.push_back(std::move(g));
+    const std::vector<long long> src = key_sources(w, P, multi);
+    std::vector<std::pair<long long, int>> ks;
+    ks.reserve(src.size());
+    for (size_t k = 0; k < src.size(); k++)
+        if (w.tcnt[k] > 0) ks.push_back({-(src[k] + 1) * w.tcnt[k], (int)k});
+    sort_keys(ks);
+    // each key's queue and first place in it
+    std::vector<std::pair<int, int>> at(ks.size());
+    long long load[NXCD] = {};
+    std::fill(qlen, qlen + NXCD, 0);
+    for (size_t i = 0; i < ks.size(); i++) {
+        const int x = (int)(std::min_element(load, load + NXCD) - load);
+        load[x] -= ks[i].first;
+        at[i] = {x, qlen[x]};
+        qlen[x] += (w.tcnt[ks[i].second] + tile_t - 1) / tile_t;
     }
-    std::stable_sort(groups.begin(), groups.end(),
-                     [](const Group &a, const Group &b) { return a.work > b.work; });
-    std::vector<std::vector<btk::Tile>> lists(NXCD);
-    std::vector<long long> load(NXCD, 0);
-    for (const Group &g : groups) {
-        int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        load[x] += g.work;
-        lists[x].insert(lists[x].end(), g.t.begin(), g.t.end());
+    tiles.assign((size_t)*std::max_element(qlen, qlen + NXCD) * NXCD, btk::Tile{0, 0, 0, 0});
+    for (size_t i = 0; i < ks.size(); i++) {
+        const int k = ks[i].second;
+        size_t j = at[i].second;
+        for (int o = 0; o < w.tcnt[k]; o += tile_t)
+            tiles[j++ * NXCD + at[i].first] =
+                btk::Tile{k, w.tbeg[k] + o, std::min(tile_t, w.tcnt[k] - o), grid ? w.key[k] : 0};
     }
-    size_t L = 0;
-    for (auto &l : lists) L = std::max(L, l.size());
-    tiles.assign(L * NXCD, btk::Tile{0, 0, 0, 0});
-    for (int x = 0; x < NXCD; x++)
-        for (size_t j = 0; j < lists[x].size(); j++) tiles[j * NXCD + x] = lists[x][j];
-    for (int x = 0; x < NXCD; x++) qlen[x] = (int)lists[x].size();
 }
 
 void make_pencil_tiles(const WorkCSR &w, int P, bool multi, std::vector<btk::Tile> &tiles)
 {
-    std::vector<std::pair<long long, btk::Tile>> ks;
-    for (size_t k = 0; k < w.key.size(); k++) {
-        long long src = 0;
-        for (int s = w.seg_off[k]; s < w.seg_off[k + 1]; s++) src += w.seg_cnt[s];
-        for (int c = w.clu_off[k]; c < w.clu_off[k + 1]; c++) src += cluster_points(w.clu_id[c], P, multi);
-        ks.push_back({(src + 1) * w.tcnt[k], btk::Tile{(int)k, 0, w.tcnt[k], w.key[k]}});
+    const std::vector<long long> src = key_sources(w, P, multi);
+    std::vector<std::pair<long long, int>> ks(src.size());
+    for (size_t k = 0; k < src.size(); k++) ks[k] = {-(src[k] + 1) * w.tcnt[k], (int)k};
+    sort_keys(ks);
+    tiles.resize(ks.size());
+    for (size_t i = 0; i < ks.size(); i++) {
+        const int k = ks[i].second;
+        tiles[i] = btk::Tile{k, 0, w.tcnt[k], w.key[k]};
     }
-    std::stable_sort(ks.begin(), ks.end(), [](const auto &a, const auto &b) { return a.first > b.first; });
-    tiles.clear();
-    for (const auto &k : ks) tiles.push_back(k.second);
 }
 
 Plan::~Plan() { free_all(); }
@@ -258,16 +276,14 @@ bool Plan::pencil_grids() const
 // particle range is another key's range, while that key lists this key's
 // range, makes a symmetric pair: one two-sided item.  Every other source
 // node (one that does not list the key back, and the key's own range) makes
-// a one-sided item.  Every range is flagged SEG_SYM in sym_of (parallel to
-// segs_of): the near launch leaves the particle pairs to the items.  The
-// item's centre c is the centre of the two boxes' joint box and R the
-// largest distance from c to either box: r^2 is formed as in the near keys
-// (|t-c|^2 + |s-c|^2 - 2 (t-c).(s-c), rounding error below
+// a one-sided item.  The near launch leaves every particle pair to the items
+// (SEG_SYM).  The item's centre c is the centre of the two boxes' joint box
+// and R the largest distance from c to either box: r^2 is formed as in the
+// near keys (|t-c|^2 + |s-c|^2 - 2 (t-c).(s-c), rounding error below
 // 6e-15 (|t-c|^2 + |s-c|^2)), so pairs below 2e-7 R^2 are recomputed from
 // differences when the boxes come within that distance.
 void Plan::build_sym(const System &sy, const std::vector<int> &keys,
-                     const std::vector<std::vector<int>> &segs_of, std::vector<std::vector<char>> &sym_of,
-                     bool symmetric)
+                     const std::vector<std::vector<int>> &segs_of, bool symmetric)
 {
     const Tree &st = sy.stree, &tt = sy.ttree;
     sym_items_.clear(); sym_ctr_.clear(); sym_red_tiles_.clear();
@@ -281,8 +297,9 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
         std::vector<std::array<long long, 2>> key_range(nk);  // (beg << 32 | cnt, key index)
         for (int k = 0; k < nk; k++)
             key_range[k] = {((long long)tt.ibeg[keys[k]] << 32) | (unsigned)tt.numpar[keys[k]], (long long)k};
-        std::sort(key_range.begin(), key_range.end());
-#pragma omp parallel for schedule(static)
+        // (leaves come in particle order)
+        if (!std::is_sorted(key_range.begin(), key_range.end())) std::sort(key_range.begin(), key_range.end());
+#pragma omp parallel for schedule(static) if (nk > PAR_KEYS)
         for (int s = 0; s < st.n; s++) {
             const long long r = ((long long)st.ibeg[s] << 32) | (unsigned)st.numpar[s];
             auto it = std::lower_bound(key_range.begin(), key_range.end(), std::array<long long, 2>{r, -1});
@@ -292,7 +309,7 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     // per key: the keys among its source ranges, sorted (does ks list k back?)
     std::vector<std::vector<int>> nbr(nk);
     if (symmetric) {
-#pragma omp parallel for schedule(dynamic, 64)
+#pragma omp parallel for schedule(dynamic, 64) if (nk > PAR_KEYS)
         for (int k = 0; k < nk; k++) {
             for (int s : segs_of[keys[k]])
                 if (key_of_node[s] >= 0) nbr[k].push_back(key_of_node[s]);
@@ -304,12 +321,10 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     // candidates in key order, each key's ranges in list order
     struct Cand { int k, kb, s; };
     std::vector<int> first(nk + 1, 0);
-#pragma omp parallel for schedule(dynamic, 64)
+#pragma omp parallel for schedule(dynamic, 64) if (nk > PAR_KEYS)
     for (int k = 0; k < nk; k++) {
-        const int t = keys[k];
-        sym_of[t].assign(segs_of[t].size(), 1);
         int c = 0;
-        for (int s : segs_of[t]) {
+        for (int s : segs_of[keys[k]]) {
             const int ks = key_of_node[s];
             const bool two = ks >= 0 && ks != k && has(ks, k);
             c += (!two || k < ks) ? 1 : 0;
@@ -318,7 +333,7 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     }
     for (int k = 0; k < nk; k++) first[k + 1] += first[k];
     std::vector<Cand> cand(first[nk]);
-#pragma omp parallel for schedule(dynamic, 64)
+#pragma omp parallel for schedule(dynamic, 64) if (nk > PAR_KEYS)
     for (int k = 0; k < nk; k++) {
         int c = first[k];
         for (int s : segs_of[keys[k]]) {
@@ -333,14 +348,14 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     const size_t nc = cand.size();
     {
         std::vector<std::pair<long long, int>> order(nc);
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for schedule(static) if (nc > PAR_KEYS)
         for (size_t i = 0; i < nc; i++) {
             const Cand &c = cand[i];
             order[i] = {-(long long)tt.numpar[keys[c.k]] * st.numpar[c.s] * (c.kb >= 0 ? 2 : 1), (int)i};
         }
-        __gnu_parallel::sort(order.begin(), order.end());
+        sort_keys(order);
         std::vector<Cand> sorted(nc);
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for schedule(static) if (nc > PAR_KEYS)
         for (size_t i = 0; i < nc; i++) sorted[i] = cand[order[i].second];
         cand.swap(sorted);
     }
@@ -363,7 +378,7 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     sym_items_.resize(nc);
     sym_ctr_.resize(4 * nc);
     long long pairs = 0, evals = 0;
-#pragma omp parallel for schedule(static) reduction(+ : pairs, evals)
+#pragma omp parallel for schedule(static) reduction(+ : pairs, evals) if (nc > PAR_KEYS)
     for (size_t i = 0; i < nc; i++) {
         const Cand &c = cand[i];
         const int t = keys[c.k], s = c.s;
@@ -391,72 +406,85 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     sym_pairs_ = pairs;
     sym_evals_ = evals;
     // per key, the bases of its slots in candidate order
-    std::vector<std::vector<long long>> lists(nk);
-    for (size_t i = 0; i < nc; i++) {
-        const Cand &c = cand[i];
-        const btk::SymItem &it = sym_items_[i];
-        lists[c.k].push_back(it.rslot - it.a_beg);
-        if (c.kb >= 0) lists[c.kb].push_back(it.cslot - it.b_beg);
+    sym_red_off_.assign(nk + 1, 0);
+    for (const Cand &c : cand) {
+        sym_red_off_[c.k + 1]++;
+        if (c.kb >= 0) sym_red_off_[c.kb + 1]++;
+    }
+    for (int k = 0; k < nk; k++) sym_red_off_[k + 1] += sym_red_off_[k];
+    sym_red_base_.resize(sym_red_off_[nk]);
+    {
+        std::vector<int> at(sym_red_off_.begin(), sym_red_off_.end() - 1);
+        for (size_t i = 0; i < nc; i++) {
+            const btk::SymItem &it = sym_items_[i];
+            sym_red_base_[at[cand[i].k]++] = it.rslot - it.a_beg;
+            if (cand[i].kb >= 0) sym_red_base_[at[cand[i].kb]++] = it.cslot - it.b_beg;
+        }
+    }
+    for (int k = 0; k < nk; k++) {
+        if (sym_red_off_[k] == sym_red_off_[k + 1]) continue;
+        const int t = keys[k];
+        for (int o = 0; o < tt.numpar[t]; o += btk::TPB_SYM_REDUCE)
+            sym_red_tiles_.push_back(btk::Tile{k, sy.toff + tt.ibeg[t] + o,
+                                               std::min(btk::TPB_SYM_REDUCE, tt.numpar[t] - o), 0});
     }
     // Launch order.  Workgroups are dealt round-robin over the 8 XCDs, so
     // block b runs on XCD b % 8.  A block streams its B leaf once per pass
     // over A; items that share a B leaf go to one XCD back to back, so their
     // passes re-read B from that XCD's L2 rather than from HBM.  Groups
-    // (heaviest first; ties by first particle of B) go to the least loaded
-    // XCD; the queues are interleaved (block 8j + x: item j of XCD x) and
-    // padded with empty items.  Slots and sums do not depend on the order.
+    // (heaviest first; ties by B's node) go to the least loaded XCD; the
+    // queues are interleaved (block 8j + x: item j of XCD x) and padded with
+    // empty items.  Slots and sums do not depend on the order.
     {
-        std::vector<std::pair<int, int>> by_b(nc);  // (first particle of B, item)
-        for (size_t i = 0; i < nc; i++) by_b[i] = {sym_items_[i].b_beg, (int)i};
-        __gnu_parallel::sort(by_b.begin(), by_b.end());
-        struct Group { long long w; size_t beg, end; };
-        std::vector<Group> groups;
-        for (size_t i = 0; i < nc;) {
-            size_t e = i;
-            long long w = 0;
-            while (e < nc && by_b[e].first == by_b[i].first) w += work(cand[by_b[e++].second]);
-            groups.push_back({w, i, e});
-            i = e;
+        // the items of every source node, in candidate order
+        std::vector<int> beg(st.n + 1, 0), by_s(nc);
+        std::vector<std::pair<long long, int>> groups;  // (-work, source node)
+        {
+            std::vector<long long> load(st.n, 0);
+            for (const Cand &c : cand) {
+                beg[c.s + 1]++;
+                load[c.s] += work(c);
+            }
+            for (int s = 0; s < st.n; s++) {
+                if (beg[s + 1] > 0) groups.push_back({-load[s], s});
+                beg[s + 1] += beg[s];
+            }
+            std::vector<int> at(beg.begin(), beg.end() - 1);
+            for (size_t i = 0; i < nc; i++) by_s[at[cand[i].s]++] = (int)i;
         }
-        std::stable_sort(groups.begin(), groups.end(), [](const Group &a, const Group &b) { return a.w > b.w; });
-        std::vector<std::vector<int>> q(NXCD);
+        sort_keys(groups);
+        const int ng = (int)groups.size();
+        std::vector<std::pair<int, int>> at(ng);  // a group's queue and first place in it
         long long load[NXCD] = {};
-        for (const Group &g : groups) {
-            const int x = (int)(std::min_element(load, load + NXCD) - load);
-            load[x] += g.w;
-            for (size_t e = g.beg; e < g.end; e++) q[x].push_back(by_b[e].second);
+        int len[NXCD] = {};
+        for (int g = 0; g < ng; g++) {
+            const int x = (int)(std::min_element(load, load + NXCD) - load), s = groups[g].second;
+            load[x] -= groups[g].first;
+            at[g] = {x, len[x]};
+            len[x] += beg[s + 1] - beg[s];
         }
-        size_t qmax = 0;
-        for (const auto &v : q) qmax = std::max(qmax, v.size());
-        std::vector<btk::SymItem> items(qmax * NXCD, btk::SymItem{0, 0, 0, 0, 0, 0});
-        std::vector<double> ctr(4 * qmax * NXCD, 0.0);
-        for (int x = 0; x < NXCD; x++) {
-            const int len = (int)q[x].size();
-#pragma omp parallel for schedule(static)
-            for (int j = 0; j < len; j++) {
-                const size_t slot = (size_t)j * NXCD + x;
-                items[slot] = sym_items_[q[x][j]];
-                std::copy(sym_ctr_.begin() + 4 * (size_t)q[x][j], sym_ctr_.begin() + 4 * (size_t)q[x][j] + 4,
-                          ctr.begin() + 4 * slot);
+        const size_t slots = (size_t)*std::max_element(len, len + NXCD) * NXCD;
+        std::vector<btk::SymItem> items(slots, btk::SymItem{0, 0, 0, 0, 0, 0});
+        std::vector<double> ctr(4 * slots, 0.0);
+#pragma omp parallel for schedule(dynamic, 64) if (ng > PAR_KEYS)
+        for (int g = 0; g < ng; g++) {
+            const int s = groups[g].second;
+            size_t slot = (size_t)at[g].second * NXCD + at[g].first;
+            for (int e = beg[s]; e < beg[s + 1]; e++, slot += NXCD) {
+                items[slot] = sym_items_[by_s[e]];
+                std::copy_n(sym_ctr_.begin() + 4 * (size_t)by_s[e], 4, ctr.begin() + 4 * slot);
             }
         }
         sym_items_.swap(items);
         sym_ctr_.swap(ctr);
     }
-    sym_red_off_.assign(1, 0);
-    for (size_t k = 0; k < keys.size(); k++) {
-        const int t = keys[k];
-        sym_red_base_.insert(sym_red_base_.end(), lists[k].begin(), lists[k].end());
-        sym_red_off_.push_back((int)sym_red_base_.size());
-        if (lists[k].empty()) continue;
-        for (int o = 0; o < tt.numpar[t]; o += btk::TPB_SYM_REDUCE)
-            sym_red_tiles_.push_back(btk::Tile{(int)k, sy.toff + tt.ibeg[t] + o,
-                                               std::min(btk::TPB_SYM_REDUCE, tt.numpar[t] - o), 0});
-    }
     sym_ = !sym_items_.empty();
 }
 
-// Flattens the lists of every system into two global CSR work descriptions:
+// Flattens the lists of every system into two global CSR work descriptions
+// (sizes first, then filled by several threads in plans of many keys: N = 4M,
+// 36k leaves, lists and work 71 -> 32 ms; N = 1k 0.11 -> 0.02 ms, without the
+// parallel regions):
 //   near_ : target leaves (particle targets) <- source particle ranges + source clusters
 //   grid_ : target nodes (grid targets)      <- source particle ranges + source clusters
 // with particle indices and node ids offset to the concatenated numbering.
@@ -464,18 +492,24 @@ void Plan::build_work()
 {
     const Params &p = prm_;
     const int P = p.P;
-    auto add_key = [](WorkCSR &w, int key, int tbeg, int tcnt) {
-        w.key.push_back(key); w.tbeg.push_back(tbeg); w.tcnt.push_back(tcnt);
+    // keys ts (target nodes) with their clusters (clus_of, may be null) and
+    // source nodes (segs_of), both indexed by target node: the sizes and
+    // offsets of w's lists
+    using Jagged = std::vector<std::vector<int>>;
+    auto size_keys = [](WorkCSR &w, const std::vector<int> &ts, const Jagged *clus_of, const Jagged &segs_of) {
+        const size_t nk = ts.size();
+        for (auto *v : {&w.key, &w.tbeg, &w.tcnt}) v->resize(nk);
+        w.seg_off.assign(nk + 1, 0);
+        w.clu_off.assign(nk + 1, 0);
+        for (size_t k = 0; k < nk; k++) {
+            w.seg_off[k + 1] = w.seg_off[k] + (int)segs_of[ts[k]].size();
+            w.clu_off[k + 1] = w.clu_off[k] + (clus_of ? (int)(*clus_of)[ts[k]].size() : 0);
+        }
+        w.seg_beg.resize(w.seg_off[nk]);
+        w.seg_cnt.resize(w.seg_off[nk]);
+        w.seg_chk.resize(w.seg_off[nk]);
+        w.clu_id.resize(w.clu_off[nk]);
     };
-    auto close_key = [](WorkCSR &w) {
-        w.seg_off.push_back((int)w.seg_beg.size());
-        w.clu_off.push_back((int)w.clu_id.size());
-    };
-    auto add_seg = [](WorkCSR &w, int b, int c, long long nt, int flags = 0) {
-        w.seg_beg.push_back(b); w.seg_cnt.push_back(c); w.seg_chk.push_back((char)flags);
-        w.pairs += nt * c;
-    };
-    auto add_clu = [P](WorkCSR &w, int id, long long nt) { w.clu_id.push_back(id); w.pairs += nt * P; };
     near_ = WorkCSR();
     grid_ = WorkCSR();
     near_ctr_.clear();
@@ -520,91 +554,117 @@ void Plan::build_work()
                    tt.ymin[t] - st.ymax[s] <= g && st.ymin[s] - tt.ymax[t] <= g &&
                    tt.zmin[t] - st.zmax[s] <= g && st.zmin[s] - tt.zmax[t] <= g;
         };
-        // one near key: target node t (particles [tbeg, tbeg + tcnt) of the
-        // concatenation) <- source clusters clus and source particle nodes segs
-        auto near_key = [&](int t, int tbeg, int tcnt, const std::vector<int> &clus,
-                            const std::vector<int> &segs, const std::vector<char> *sym = nullptr) {
-            const double cx = tt.xmid[t], cy = tt.ymid[t], cz = tt.zmid[t];
-            const double rt2 = far2(cx, cy, cz, tt, t);
-            double R2 = rt2;
-            for (int s : segs) R2 = std::max(R2, far2(cx, cy, cz, st, s));
-            bool clu_check = false;
-            for (int c : clus) {
-                const double f2 = far2(cx, cy, cz, st, c);
-                if (rt2 + f2 > 1e7 * gap2(t, c)) { clu_check = true; R2 = std::max(R2, f2); }
+        // near keys: target nodes ts <- source clusters clus_of and source
+        // particle nodes segs_of
+        auto near_keys = [&](const std::vector<int> &ts, const Jagged *clus_of, const Jagged &segs_of) {
+            const int nk = (int)ts.size();
+            size_keys(nw, ts, clus_of, segs_of);
+            nctr.resize(4 * (size_t)nk);
+            long long pairs = 0;
+#pragma omp parallel for schedule(dynamic, 64) reduction(+ : pairs) if (nk > PAR_KEYS)
+            for (int k = 0; k < nk; k++) {
+                const int t = ts[k];
+                const std::vector<int> &segs = segs_of[t];
+                const double cx = tt.xmid[t], cy = tt.ymid[t], cz = tt.zmid[t];
+                const double rt2 = far2(cx, cy, cz, tt, t);
+                double R2 = rt2;
+                for (int s : segs) R2 = std::max(R2, far2(cx, cy, cz, st, s));
+                bool clu_check = false;
+                const long long nt = tt.numpar[t];
+                if (clus_of) {
+                    int *id = nw.clu_id.data() + nw.clu_off[k];
+                    for (int c : (*clus_of)[t]) {
+                        const double f2 = far2(cx, cy, cz, st, c);
+                        if (rt2 + f2 > 1e7 * gap2(t, c)) { clu_check = true; R2 = std::max(R2, f2); }
+                        *id++ = sn + c;
+                        pairs += nt * P;
+                    }
+                }
+                const double thresh = std::max(2e-7 * R2, 1e-300);
+                const double gclose = std::max(1e-150, std::sqrt(thresh));
+                nw.key[k] = tn + t; nw.tbeg[k] = to + tt.ibeg[t]; nw.tcnt[k] = tt.numpar[t];
+                int i = nw.seg_off[k];
+                for (int s : segs) {
+                    nw.seg_beg[i] = so + st.ibeg[s];
+                    nw.seg_cnt[i] = st.numpar[s];
+                    nw.seg_chk[i++] = (char)((within(t, s, 1e-150) ? SEG_COINCIDE : 0) |
+                                             (within(t, s, gclose) ? SEG_CLOSE : 0) | (items ? SEG_SYM : 0));
+                    pairs += nt * st.numpar[s];
+                }
+                double *c = nctr.data() + 4 * (size_t)k;
+                c[0] = cx; c[1] = cy; c[2] = cz; c[3] = clu_check ? -thresh : thresh;
             }
-            const double thresh = std::max(2e-7 * R2, 1e-300);
-            const double gclose = std::max(1e-150, std::sqrt(thresh));
-            const long long nt = tcnt;
-            add_key(nw, tn + t, tbeg, tcnt);
-            for (int c : clus) add_clu(nw, sn + c, nt);
-            for (size_t i = 0; i < segs.size(); i++) {
-                const int s = segs[i];
-                add_seg(nw, so + st.ibeg[s], st.numpar[s], nt,
-                        (within(t, s, 1e-150) ? SEG_COINCIDE : 0) | (within(t, s, gclose) ? SEG_CLOSE : 0) |
-                            (sym && (*sym)[i] ? SEG_SYM : 0));
+            nw.pairs = pairs;
+        };
+        // grid keys: the target nodes with source clusters (clus_of, may be
+        // null) or source particle nodes (segs_of)
+        auto grid_keys = [&](const Jagged *clus_of, const Jagged &segs_of) {
+            std::vector<int> ts;
+            for (int t = 0; t < tt.n; t++)
+                if (!segs_of[t].empty() || (clus_of && !(*clus_of)[t].empty())) ts.push_back(t);
+            const int nk = (int)ts.size();
+            size_keys(gw, ts, clus_of, segs_of);
+            long long pairs = 0;
+#pragma omp parallel for schedule(dynamic, 64) reduction(+ : pairs) if (nk > PAR_KEYS)
+            for (int k = 0; k < nk; k++) {
+                const int t = ts[k];
+                gw.key[k] = tn + t; gw.tbeg[k] = 0; gw.tcnt[k] = P;
+                if (clus_of) {
+                    int *id = gw.clu_id.data() + gw.clu_off[k];
+                    for (int c : (*clus_of)[t]) {
+                        *id++ = sn + c;
+                        pairs += (long long)P * P;
+                    }
+                }
+                int i = gw.seg_off[k];
+                for (int s : segs_of[t]) {
+                    gw.seg_beg[i] = so + st.ibeg[s];
+                    gw.seg_cnt[i] = st.numpar[s];
+                    gw.seg_chk[i++] = 0;
+                    pairs += (long long)P * st.numpar[s];
+                }
             }
-            close_key(nw);
-            nctr.push_back(cx); nctr.push_back(cy); nctr.push_back(cz);
-            nctr.push_back(clu_check ? -thresh : thresh);
+            gw.pairs = pairs;
         };
         if (p.compute_type == C_PC) {
             // keys: target batches; pc list -> clusters, pp list -> source leaves
-            std::vector<std::vector<char>> sym_of(tt.n);
-            if (items) {
-                std::vector<int> keys(tt.n);
-                for (int b = 0; b < tt.n; b++) keys[b] = b;
-                build_sym(sy, keys, L.pp, sym_of, sym_ok_);
-            }
-            for (int b = 0; b < tt.n; b++)
-                near_key(b, to + tt.ibeg[b], tt.numpar[b], L.approx[b], L.pp[b], items ? &sym_of[b] : nullptr);
+            std::vector<int> keys(tt.n);
+            for (int b = 0; b < tt.n; b++) keys[b] = b;
+            if (items) build_sym(sy, keys, L.pp, sym_ok_);
+            near_keys(keys, &L.approx, L.pp);
         } else if (p.compute_type == C_CP) {
             // lists keyed by source batch; invert to target-node keys
-            std::vector<std::vector<int>> pp_of(tt.n), cp_of(tt.n);
+            Jagged pp_of(tt.n), cp_of(tt.n);
             for (int b = 0; b < st.n; b++) {
                 for (int t : L.pp[b]) pp_of[t].push_back(b);
                 for (int t : L.approx[b]) cp_of[t].push_back(b);
             }
-            const std::vector<int> none;
-            std::vector<std::vector<char>> sym_of(tt.n);
-            if (items) build_sym(sy, tt.leaves, pp_of, sym_of, sym_ok_);
-            for (int leaf : tt.leaves)
-                near_key(leaf, to + tt.ibeg[leaf], tt.numpar[leaf], none, pp_of[leaf],
-                         items ? &sym_of[leaf] : nullptr);
-            for (int t = 0; t < tt.n; t++) {
-                if (cp_of[t].empty()) continue;
-                add_key(gw, tn + t, 0, P);
-                for (int b : cp_of[t]) add_seg(gw, so + st.ibeg[b], st.numpar[b], P);
-                close_key(gw);
-            }
+            if (items) build_sym(sy, tt.leaves, pp_of, sym_ok_);
+            near_keys(tt.leaves, nullptr, pp_of);
+            grid_keys(nullptr, cp_of);
         } else {
             // CC: a target leaf gets the PP and source-approx (PC) lists of
             // itself and of every ancestor; grids get CC and target-approx (CP)
-            std::vector<std::vector<int>> clus_of(tt.n), segs_of(tt.n);
-            for (int leaf : tt.leaves) {
+            Jagged clus_of(tt.n), segs_of(tt.n);
+            const int nl = (int)tt.leaves.size();
+#pragma omp parallel for schedule(dynamic, 64) if (nl > PAR_KEYS)
+            for (int l = 0; l < nl; l++) {
+                const int leaf = tt.leaves[l];
                 for (int a = leaf; a >= 0; a = tt.parent[a]) {
                     clus_of[leaf].insert(clus_of[leaf].end(), L.cc_pc[a].begin(), L.cc_pc[a].end());
                     segs_of[leaf].insert(segs_of[leaf].end(), L.pp[a].begin(), L.pp[a].end());
                 }
             }
-            std::vector<std::vector<char>> sym_of(tt.n);
-            if (items) build_sym(sy, tt.leaves, segs_of, sym_of, sym_ok_);
-            for (int leaf : tt.leaves)
-                near_key(leaf, to + tt.ibeg[leaf], tt.numpar[leaf], clus_of[leaf], segs_of[leaf],
-                         items ? &sym_of[leaf] : nullptr);
-            for (int t = 0; t < tt.n; t++) {
-                if (L.approx[t].empty() && L.cc_cp[t].empty()) continue;
-                add_key(gw, tn + t, 0, P);
-                for (int c : L.approx[t]) add_clu(gw, sn + c, P);
-                for (int s : L.cc_cp[t]) add_seg(gw, so + st.ibeg[s], st.numpar[s], P);
-                close_key(gw);
-            }
+            if (items) build_sym(sy, tt.leaves, segs_of, sym_ok_);
+            near_keys(tt.leaves, &clus_of, segs_of);
+            grid_keys(&L.approx, L.cc_cp);
         }
         // heavy grid keys are split by sources; every key writes its own row
         // (systems of a batch are split as they are alone)
         if (!gw.key.empty()) {
-            const WorkCSR raw = std::move(gw);
-            split_keys(raw, grid_key_sources(raw, P, false), P, false, gw);
+            WorkCSR raw = std::move(gw);
+            const long long max_src = grid_key_sources(raw, P, false);
+            split_keys(std::move(raw), max_src, P, false, gw);
         }
     };
     auto csr_start = [](WorkCSR &w) { w.seg_off.assign(1, 0); w.clu_off.assign(1, 0); };

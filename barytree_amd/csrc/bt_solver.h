@@ -99,7 +99,7 @@ void make_pencil_tiles(const WorkCSR &w, int P, bool multi, std::vector<btk::Til
 // Splits every key whose sources (particles plus cluster points) exceed
 // max_src into consecutive chunks of its particle ranges and clusters; the
 // chunks are keys of their own with the same node and targets, in order.
-void split_keys(const WorkCSR &in, long long max_src, int P, bool multi, WorkCSR &out);
+void split_keys(WorkCSR &&in, long long max_src, int P, bool multi, WorkCSR &out);
 long long grid_key_sources(const WorkCSR &w, int P, bool multi);
 
 struct PlanInput {
@@ -212,8 +212,8 @@ private:
     // the item launch's items, slots and reduction lists (one system):
     // two-sided and one-sided items when its targets are its sources
     // (sym_ok_), one-sided items only otherwise (items_ok_); set by create
-    void build_sym(const System &sy, const std::vector<int> &keys, const std::vector<std::vector<int>> &segs_of,
-                   std::vector<std::vector<char>> &sym_of, bool symmetric);
+    void build_sym(const System &sy, const std::vector<int> &keys,
+                   const std::vector<std::vector<int>> &segs_of, bool symmetric);
     // this execution's pairs are evaluated in FP64: the plain precision, and
     // the kernels beside the Coulomb family in either
     bool fp64_arithmetic() const { return prm_.precision != PREC_MIXED || !coulomb_family(prm_.kernel); }

@@ -45,17 +45,23 @@ void Plan::enumerate_pairs()
     for (int sy = 0; sy < (int)sys_.size(); sy++) {
         const System &y = sys_[sy];
         const Lists &L = y.L;
-        if (prm_.compute_type == C_PC) {
-            for (int b = 0; b < y.ttree.n; b++)
-                for (int c : L.approx[b]) pairs_.push_back({sy, FAR_PC, b, c});
-        } else if (prm_.compute_type == C_CP) {
-            for (int b = 0; b < y.stree.n; b++)
-                for (int t : L.approx[b]) pairs_.push_back({sy, FAR_CP, t, b});
-        } else {
-            for (int t = 0; t < y.ttree.n; t++) {
-                for (int s : L.approx[t]) pairs_.push_back({sy, FAR_CC, t, s});
-                for (int s : L.cc_pc[t]) pairs_.push_back({sy, FAR_PC, t, s});
-                for (int s : L.cc_cp[t]) pairs_.push_back({sy, FAR_CP, t, s});
+        const int ct = prm_.compute_type;
+        const int n = ct == C_CP ? y.stree.n : y.ttree.n;
+        std::vector<size_t> at(n + 1, pairs_.size());  // a list's first pair
+        for (int k = 0; k < n; k++)
+            at[k + 1] = at[k] + L.approx[k].size() + (ct == C_CC ? L.cc_pc[k].size() + L.cc_cp[k].size() : 0);
+        pairs_.resize(at[n]);
+#pragma omp parallel for schedule(static) if (at[n] - at[0] > 20000)
+        for (int k = 0; k < n; k++) {
+            FarPair *o = pairs_.data() + at[k];
+            if (ct == C_PC) {
+                for (int c : L.approx[k]) *o++ = {sy, FAR_PC, k, c};
+            } else if (ct == C_CP) {
+                for (int t : L.approx[k]) *o++ = {sy, FAR_CP, t, k};
+            } else {
+                for (int s : L.approx[k]) *o++ = {sy, FAR_CC, k, s};
+                for (int s : L.cc_pc[k]) *o++ = {sy, FAR_PC, k, s};
+                for (int s : L.cc_cp[k]) *o++ = {sy, FAR_CP, k, s};
             }
         }
     }
@@ -263,7 +269,8 @@ std::string Plan::set_pair_degrees(const int *deg)
             raw.clu_off.push_back((int)raw.clu_id.size());
         }
     }
-    split_keys(raw, grid_key_sources(raw, 0, true), 0, true, vfar_);
+    const long long max_src = grid_key_sources(raw, 0, true);
+    split_keys(std::move(raw), max_src, 0, true, vfar_);
     vfar_row_.assign(vfar_.key.size(), 0);
     vfar_rows_len_ = 0;
     for (size_t k = 0; k < vfar_.key.size(); k++) {

@@ -68,6 +68,23 @@ def test_host_lists_match_oracle(bt, oracle_mod, ct, n, m, deg, msl, mtl, theta)
     assert a["pp_ptwise"] + a["pc_replaced"] + a["cp_replaced"] + a["cc_replaced"] == n * m
 
 
+@pytest.mark.parametrize("ct", [1, 2, 3])
+@pytest.mark.parametrize("n,m", [(12000, 12000), (20000, 300), (300, 20000)])
+def test_host_lists_of_many_nodes_match_oracle(bt, oracle_mod, ct, n, m):
+    """Trees above 1024 nodes (their lists are walked by several threads),
+    one on each side or both; clustered, so subtrees end at all depths."""
+    rng = np.random.default_rng(n + ct)
+    t, s = uniform_cube(n, m, seed=n + ct)
+    for a in (t, s):
+        for d in range(3):
+            a[d] = np.sign(a[d]) * np.abs(a[d]) ** rng.uniform(2.0, 4.0)
+    a = bt.analyze(t, s, 1, [0.5], 1, 1, ct, 0.7, 1, 6, 6)
+    oracle_mod.treecode(*t, *s, 1, [0.5], 1, 1, ct, 0.7, 1, 6, 6)
+    o = oracle_mod.last_stats()
+    assert {k: a[k] for k in KEYS} == {k: o[k] for k in KEYS}
+    assert a["pp_ptwise"] + a["pc_replaced"] + a["cp_replaced"] + a["cc_replaced"] == n * m
+
+
 @pytest.mark.parametrize("ct,k,s", hermite_combos())
 def test_hermite_host_work_matches_oracle(bt, oracle_mod, ct, k, s):
     """Hermite plans build (and check) their work lists on the host; the
