@@ -53,9 +53,11 @@ long long cluster_points(int id, int P, bool multi)
     return nl * nl * nl;
 }
 
-// keys, nodes or leaves above which their loops are shared by threads (a
-// parallel region costs a small plan more than it gives)
-constexpr int PAR_KEYS = 256;
+// keys, nodes or leaves above which their loops are shared by threads, and 16
+// or 32 times as many items above which loops and sorts over them are (N = 1k,
+// 8 leaves: 0.11 ms of 0.95 in parallel regions; N = 10k, 145 leaves: 3.4 ms
+// with all of them parallel, 2.9 so, 4.0 with lines four to eight times higher)
+constexpr int PAR_KEYS = 64;
 
 // source points of every key
 std::vector<long long> key_sources(const WorkCSR &w, int P, bool multi)
@@ -77,7 +79,7 @@ std::vector<long long> key_sources(const WorkCSR &w, int P, bool multi)
 // (-work, key), the heaviest key first and ties in key order
 void sort_keys(std::vector<std::pair<long long, int>> &ks)
 {
-    if (ks.size() > 64 * PAR_KEYS) __gnu_parallel::sort(ks.begin(), ks.end());
+    if (ks.size() > 32 * PAR_KEYS) __gnu_parallel::sort(ks.begin(), ks.end());
     else std::sort(ks.begin(), ks.end());
 }
 }  // namespace
@@ -348,14 +350,14 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     const size_t nc = cand.size();
     {
         std::vector<std::pair<long long, int>> order(nc);
-#pragma omp parallel for schedule(static) if (nc > PAR_KEYS)
+#pragma omp parallel for schedule(static) if (nc > 16 * PAR_KEYS)
         for (size_t i = 0; i < nc; i++) {
             const Cand &c = cand[i];
             order[i] = {-(long long)tt.numpar[keys[c.k]] * st.numpar[c.s] * (c.kb >= 0 ? 2 : 1), (int)i};
         }
         sort_keys(order);
         std::vector<Cand> sorted(nc);
-#pragma omp parallel for schedule(static) if (nc > PAR_KEYS)
+#pragma omp parallel for schedule(static) if (nc > 16 * PAR_KEYS)
         for (size_t i = 0; i < nc; i++) sorted[i] = cand[order[i].second];
         cand.swap(sorted);
     }
@@ -378,7 +380,7 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
     sym_items_.resize(nc);
     sym_ctr_.resize(4 * nc);
     long long pairs = 0, evals = 0;
-#pragma omp parallel for schedule(static) reduction(+ : pairs, evals) if (nc > PAR_KEYS)
+#pragma omp parallel for schedule(static) reduction(+ : pairs, evals) if (nc > 16 * PAR_KEYS)
     for (size_t i = 0; i < nc; i++) {
         const Cand &c = cand[i];
         const int t = keys[c.k], s = c.s;
@@ -483,7 +485,7 @@ void Plan::build_sym(const System &sy, const std::vector<int> &keys,
 
 // Flattens the lists of every system into two global CSR work descriptions
 // (sizes first, then filled by several threads in plans of many keys: N = 4M,
-// 36k leaves, lists and work 71 -> 32 ms; N = 1k 0.11 -> 0.02 ms, without the
+// clustered, lists and work 71 -> 32 ms; N = 1k 0.11 -> 0.02 ms, without the
 // parallel regions):
 //   near_ : target leaves (particle targets) <- source particle ranges + source clusters
 //   grid_ : target nodes (grid targets)      <- source particle ranges + source clusters
