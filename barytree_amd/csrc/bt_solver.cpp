@@ -55,7 +55,7 @@ long long cluster_points(int id, int P, bool multi)
 
 // keys, nodes or leaves above which their loops are shared by threads, and 16
 // or 32 times as many items above which loops and sorts over them are (N = 1k,
-// 8 leaves: 0.11 ms of 0.95 in parallel regions; N = 10k, 145 leaves: 3.4 ms
+// 16 leaves: 0.11 ms of 0.95 in parallel regions; N = 10k, 251 leaves: 3.4 ms
 // with all of them parallel, 2.9 so, 4.0 with lines four to eight times higher)
 constexpr int PAR_KEYS = 64;
 
@@ -1711,8 +1711,17 @@ std::string Plan::execute(bool timed)
     // 2. near field and particle-cluster far field into the potential.  The
     // potential starts as NaN (all bytes 0xFF): the near-field tiles write
     // every target once, so a target that no tile covered would show NaN,
-    // never a value left from an earlier execution.
-    HIPCHK(hipMemsetAsync(d_pot_, 0xFF, (size_t)M_ * sizeof(double), st_));
+    // never a value left from an earlier execution.  It starts as zero where
+    // the items of a mixed cluster-particle execution take all of the near
+    // launch's work: its blocks (two waves per SIMD) took the far field's
+    // place beside the items to walk lists and store zeros (N = 65k, GPU
+    // 0.83 -> 0.76 ms; N = 100k, degree 11, 2.74 -> 2.30; N = 4M Plummer, 237
+    // -> 233).  Elsewhere the launch stays: without it the far field starts
+    // earlier beside the items, which is slower (FP64 Yukawa cluster-cluster,
+    // N = 1M, 79.3 -> 81.3 ms; mixed, N = 16M, 1245 -> 1250).
+    const bool items = sym_ready();
+    const bool near = !items || fp64_arithmetic() || p.compute_type != C_CP;
+    HIPCHK(hipMemsetAsync(d_pot_, near ? 0xFF : 0, (size_t)M_ * sizeof(double), st_));
     btk::InteractArgs ia{};
     ia.kernel = p.kernel; ia.singularity = p.singularity; ia.precision = p.precision;
     ia.tpt = tpt_;
@@ -1727,11 +1736,11 @@ std::string Plan::execute(bool timed)
         a.seg_off = d_nseg_off_; a.segs = d_nsegs_; a.clu_off = d_nclu_off_; a.clu_id = d_nclu_id_;
         a.out1 = d_pot_;
         if (p.precision == PREC_MIXED) a.key_ctr = reinterpret_cast<const double4 *>(d_near_ctr_);
-        a.skip_sym = sym_ready() ? 1 : 0;
+        a.skip_sym = items ? 1 : 0;
         std::copy(near_qlen_, near_qlen_ + NXCD, a.qlen);
         a.cursor = d_cursor_;
         a.skip_clu = pc_run() ? 1 : 0;
-        HIPCHK(btk::launch_interact(a, st_));
+        if (near) HIPCHK(btk::launch_interact(a, st_));
         if (a.skip_clu) {
             std::string r = launch_pc();
             if (!r.empty()) return r;

@@ -673,18 +673,21 @@ std::string Plan::execute_var(bool timed)
     }
 
     // 2. near field and the source slots of every degree into the potential
-    //    (NaN first: every target is written by exactly one key)
-    HIPCHK(hipMemsetAsync(d_pot_, 0xFF, (size_t)M_ * sizeof(double), st_));
+    //    (NaN first: every target is written by exactly one key; zero where
+    //    the items leave nothing to the near launch, as in execute)
+    const bool items = sym_ready();
+    const bool near = !items || fp64_arithmetic() || p.compute_type != C_CP;
+    HIPCHK(hipMemsetAsync(d_pot_, near ? 0xFF : 0, (size_t)M_ * sizeof(double), st_));
     {
         btk::InteractArgs a = ia;
         a.grid_targets = 0; a.ntiles = (int)vnear_tiles_.size(); a.tiles = d_vn_tiles_;
         a.seg_off = d_nseg_off_; a.segs = d_nsegs_; a.clu_off = d_vn_clu_off_; a.clu_id = d_vn_clu_id_;
         a.out1 = d_pot_;
         if (p.precision == PREC_MIXED) a.key_ctr = reinterpret_cast<const double4 *>(d_near_ctr_);
-        a.skip_sym = sym_ready() ? 1 : 0;
+        a.skip_sym = items ? 1 : 0;
         std::copy(vnear_qlen_, vnear_qlen_ + NQ, a.qlen);
         a.cursor = d_cursor_;
-        HIPCHK(btk::launch_interact(a, st_));
+        if (near) HIPCHK(btk::launch_interact(a, st_));
         if (a.skip_sym) {
             std::string r = near_sym(!ov);
             if (!r.empty()) return r;
