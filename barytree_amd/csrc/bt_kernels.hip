@@ -1269,7 +1269,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_near_sym64(SymArgs A)
     const bool check = ctr.w < 0.0;
     // no pair of the item is further apart than 2 R (ctr.w = 2e-7 R^2), so the
     // sine's range check and the library's sine behind it (36 bytes of spills)
-    // are left to items beyond its range; the dummies lie 3 R from the centre
+    // are left to items beyond its range
     const double R = KER == KSR ? sqrt(fabs(ctr.w) * 5.0e6) : 0.0;
     const bool guard = KER == KSR && !(8.0 * R < A.kp.sn.rmax);
     constexpr int NG = 64 / G;
@@ -1306,22 +1306,22 @@ __global__ __launch_bounds__(64 * NW, 4) void k_near_sym64(SymArgs A)
         for (int off = 0; off < it.b_cnt; off += NT) {
             const int n = min(NT, it.b_cnt - off);
             __syncthreads();  // the previous chunk's LDS has been read
-            if (tid < n) {
-                const int g = it.b_beg + off + tid;
-                const double q = A.q[g];
+            {
+                // past the chunk's n sources: its first source again, with
+                // zero charge and weight (the column sums are never stored).
+                // A dummy's term is zero times a value that a source of the
+                // item gives as well; a far point's e^{-k r} of a rate k < 0
+                // overflows, and zero times infinity is NaN.
+                const bool v = tid < n;
+                const int g = it.b_beg + off + (v ? tid : 0);
+                const double q = v ? A.q[g] : 0.0;
                 if constexpr (SS) {
-                    const double w = A.w[g];
+                    const double w = v ? A.w[g] : 0.0;
                     Ls[tid] = make_double4(A.x[g], A.y[g], A.z[g], q * w);
                     Lw[tid] = make_double2(w, q);
                 } else {
                     Ls[tid] = make_double4(A.x[g], A.y[g], A.z[g], q);
                 }
-            } else {
-                // dummies: zero charge and weight, away from every target
-                // (their column sums are never stored)
-                if constexpr (KER == KSR) Ls[tid] = make_double4(ctr.x + 3.0 * R, ctr.y, ctr.z, 0.0);
-                else Ls[tid] = make_double4(1.0e100, 1.0e100, 1.0e100, 0.0);
-                if constexpr (SS) Lw[tid] = make_double2(0.0, 0.0);
             }
             __syncthreads();
             const int steps = (n + NG - 1) / NG;

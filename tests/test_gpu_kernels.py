@@ -87,3 +87,36 @@ def test_other_kernels_targets_equal_sources(bt, oracle_mod, k, ct, leaf):
         one = p.execute()
     assert rel_l2(ref, got) <= TOL_FP64 and rel_l2(ref, one) <= TOL_FP64
     assert np.array_equal(got, bt.solve(t, src, *args, precision=bt.PRECISION_MIXED))
+
+
+@pytest.mark.parametrize("k,s", [(2, 1), (2, 2), (4, 1), (12, 1)])
+@pytest.mark.parametrize("ct,leaf", [(1, 300), (2, 33), (3, 130), (1, 7)])
+def test_growing_exponentials_targets_equal_sources(bt, oracle_mod, k, s, ct, leaf):
+    """A negative rate (e^{|k| r}) with targets equal to the sources, in
+    leaves whose counts are not multiples of 8: the places that fill the last
+    step of a leaf must not bring an overflow in (zero times infinity)."""
+    print(f"case k={k} s={s} ct={ct} leaf={leaf}", flush=True)
+    rng = np.random.default_rng(ct + 10 * k)
+    x, y, z, q = (rng.uniform(-1, 1, 3001) for _ in range(4))
+    src = (x, y, z, q, rng.uniform(0.5, 1.5, 3001))
+    t = tuple(a.copy() for a in src[:4])
+    for rate in (-0.5, -20.0):
+        args = (k, [rate, 0.1] if k == 4 else [rate], s, 1, ct, 0.7, 3, leaf, leaf)
+        got = bt.solve(t, src, *args)
+        assert bt.last_stats()["sym_ptwise"] > 0
+        assert rel_l2(oracle_mod.treecode(*t, *src, *args), got) <= TOL_FP64, rate
+
+
+@pytest.mark.parametrize("k,kp", [(8, [1.5]), (1, [0.5]), (2, [0.5]), (12, [0.5])])
+def test_leaves_smaller_than_their_coordinates_spacing(bt, oracle_mod, k, kp):
+    """Leaves far from the origin whose extent lies below the spacing of
+    doubles at one of their coordinates: a place that fills a leaf's last step
+    must not fall on a particle there."""
+    y = np.array([-1.0, 0.0, 1.0, 400.0, 401.0, 402.0, 407.0]) * 1e-12
+    x, z = np.full(7, 1.0e6), np.zeros(7)
+    src = (x, y, z, np.arange(1.0, 8.0), np.ones(7))
+    t = tuple(a.copy() for a in src[:4])
+    args = (k, kp, 1, 1, 1, 0.7, 3, 2, 2)
+    got = bt.solve(t, src, *args)
+    assert bt.last_stats()["sym_ptwise"] > 0
+    assert rel_l2(oracle_mod.treecode(*t, *src, *args), got) <= TOL_FP64
