@@ -314,7 +314,9 @@ __global__ __launch_bounds__(LTPB) void k_label(LabelArgs A, LabelKernel K)
         // every thread forms the same two sums
         double num = 0.0, den = 0.0;
         for (int i = 0; i < NT; i++) { num += Lred[i]; den += Lred[NT + i]; }
-        const double err = den > 0.0 ? sqrt(num / den) : (num > 0.0 ? INFINITY : 0.0);
+        // a sampled point on another's place makes the sums NaN (rsq64(0)):
+        // the error is NaN then, which no tolerance accepts
+        const double err = num == 0.0 && den == 0.0 ? 0.0 : sqrt(num / den);
         if (tid == 0) A.errors[(size_t)pi * LABEL_ND + (p - LABEL_DMIN)] = err;
         if (err <= A.tol) { label = p; break; }  // block-uniform
     }

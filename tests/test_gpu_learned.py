@@ -149,6 +149,45 @@ def test_label_shares_at_their_edges(bt, oracle_mod, nt, ns, ss):
         assert np.allclose(eg, eo, rtol=1e-8, atol=1e-12), (kernel, np.abs(eg - eo).max())
 
 
+@pytest.mark.parametrize("kind", [1, 2, 3])
+@pytest.mark.parametrize("ss", [False, True])
+def test_labels_of_a_pair_with_coincident_points(bt, oracle_mod, kind, ss):
+    """A sampled target on a sampled source: the exact sum is infinite, no
+    degree reaches any tolerance (13) and no error is finite, as the oracle has
+    it; the other pair of the call is labelled as it is alone.  Potentials
+    that are exactly zero (no charges) have error 0."""
+    rng = np.random.default_rng(kind)
+    n = 40
+    T = rng.uniform(-0.4, 0.4, (2 * n, 3))
+    S = rng.uniform(-0.4, 0.4, (2 * n, 3)) + [1.9, 0.3, 0.0]
+    T[n:] += [0, 0, 5.0]
+    S[n:] += [0, 0, 5.0]
+    T[3] = S[5]
+    box = lambda p: [v for d in range(3) for v in (p[:, d].min(), p[:, d].max())]
+    pairs = (np.array([kind, kind]), [0, n], [n, n], [0, n], [n, n],
+             np.array(box(T[:n]) + box(T[n:])), np.array(box(S[:n]) + box(S[n:])))
+    q, tq, w = rng.uniform(0.1, 1, 2 * n), rng.uniform(-1, 1, 2 * n), rng.uniform(0.5, 1.5, 2 * n)
+    tq[3] = -0.5  # both terms of the same sign: infinite, not NaN, in the oracle
+    for kernel, kp in ((1, [0.5]), (2, [0.5])):
+        for charges in (q, 0.0 * q):
+            if ss:
+                lab, err = bt.label_pairs_subtraction(*pairs, (*T.T, 0.0 * tq if charges is not q else tq),
+                                                      (*S.T, charges, w), kernel, kp, 1e-4)
+            else:
+                lab, err = bt.label_pairs(*pairs, tuple(T.T), (*S.T, charges), kernel, kp[0], 1e-4)
+            print(kernel, lab, err[0, :3], err[1, :3], flush=True)
+            assert lab[0] == 13 and not np.any(np.isfinite(err[0]))
+            if charges is q:
+                assert 2 <= lab[1] < 13 and err[1, lab[1] - 2] <= 1e-4
+            else:
+                assert lab[1] == 2 and err[1, 0] == 0.0
+            if charges is q:
+                lo, eo = (oracle_mod.label_pairs_ss(*pairs, *T.T, tq, *S.T, q, w, kernel, 0.0 if kernel == 1 else kp[0],
+                                                    0.0 if kernel == 2 else 1 / kp[0] ** 2, 1e-4) if ss else
+                          oracle_mod.label_pairs(*pairs, *T.T, *S.T, q, kernel, kp[0], 1e-4))
+                assert np.array_equal(lo, lab) and not np.any(np.isfinite(eo[0]))
+
+
 def test_subtraction_labels_match_oracle(bt, oracle_mod):
     """Labels of the subtraction kernels (both terms) against the oracle's
     restatement, which scipy's interpolation pins."""
