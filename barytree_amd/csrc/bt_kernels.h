@@ -41,9 +41,10 @@ struct ExpRate { double c, umax; };
 // k = 0: e^0 = 1 for every u; k beyond the range of c (an infinite rate,
 // a = 0): the largest that keeps c finite, where e^{-k u} is 0 for every
 // u > 1e-287.  k < 0 (a growing exponential): u is clamped where e^{|k| u}
-// has overflowed.
+// has overflowed.  A NaN rate gives NaN for every u.
 inline ExpRate exp_rate(long double k)
 {
+    if (std::isnan(k)) return {(double)k, (double)k};
     const long double lim = 1e290L;
     k = std::max(-lim, std::min(lim, k));
     ExpRate r;

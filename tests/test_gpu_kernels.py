@@ -120,3 +120,15 @@ def test_leaves_smaller_than_their_coordinates_spacing(bt, oracle_mod, k, kp):
     got = bt.solve(t, src, *args)
     assert bt.last_stats()["sym_ptwise"] > 0
     assert rel_l2(oracle_mod.treecode(*t, *src, *args), got) <= TOL_FP64
+
+
+@pytest.mark.parametrize("k", [2, 4, 8, 12])
+@pytest.mark.parametrize("same", [False, True])
+def test_a_nan_rate_gives_nan(bt, k, same):
+    """A kernel parameter that is not a number is not taken for a finite
+    rate: every potential is NaN."""
+    t, src = uniform_cube(700, 600, seed=k)
+    if same:
+        t = [a.copy() for a in src[:4]]
+    got = bt.solve(t, src, k, [np.nan, 0.1] if k == 4 else [np.nan], 1, 1, 1, 0.7, 3, 100, 100)
+    assert np.all(np.isnan(got))

@@ -99,3 +99,11 @@ def test_sin_table_form_is_within_two_ulp_of_one(k):
         ref = np.sin((np.float64(k) * x))
         assert np.all(np.abs(y - ref) <= 4 * ULP1 + np.abs(a) * 2.0 ** -52)
     assert np.all(np.isnan(probe.sin_kr(1.5, np.array([np.nan]))))
+
+
+def test_table_forms_of_a_nan_rate_are_nan():
+    """A rate that is not a number gives NaN, as the library's functions do."""
+    from barytree_amd import probe
+    x = np.array([0.0, 1e-3, 1.0, 1e300, np.inf])
+    assert np.all(np.isnan(probe.exp_neg(np.nan, x)))
+    assert np.all(np.isnan(probe.sin_kr(np.nan, x)))
