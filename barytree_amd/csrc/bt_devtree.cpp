@@ -55,6 +55,14 @@ template <class T> struct Grow {
     }
 };
 
+// Waits for the stream when it goes out of scope: declared after the host
+// arrays of asynchronous copies, it keeps them alive until the copies are
+// done, whichever way the build returns.
+struct StreamWait {
+    hipStream_t st;
+    ~StreamWait() { (void)hipStreamSynchronize(st); }
+};
+
 // A node found by the level-by-level build.
 struct BNode {
     int b, e, level, root;
@@ -111,6 +119,7 @@ std::string device_build_trees(DevParticles &p, const std::vector<DevRoot> &root
     int set = 0;
     std::vector<double> part;
     std::vector<int> low;
+    StreamWait copies_done{st};
 
     while (!cur.empty()) {
         // 1. exact bounding boxes of the level's nodes
@@ -244,10 +253,7 @@ std::string device_build_trees(DevParticles &p, const std::vector<DevRoot> &root
         for (const Split &s : splits) {
             int nonempty = 0;
             for (int i = 0; i < s.nr; i++) nonempty += s.rb[i] < s.re[i];
-            if (nonempty == 1) {
-                HIPCHK(hipStreamSynchronize(st));  // the last pass
-                return COINCIDENT_ERROR;
-            }
+            if (nonempty == 1) return COINCIDENT_ERROR;
             for (int i = 0; i < s.nr; i++) {
                 if (s.rb[i] >= s.re[i]) continue;
                 BNode c{};

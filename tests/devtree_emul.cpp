@@ -14,6 +14,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <tuple>
 #include <vector>
 
@@ -41,13 +42,42 @@ hipError_t hipFree(void *p)
     std::free(p);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+// Asynchronous copies act at once but count as in flight, by their host
+// address, until the next synchronisation; operator delete counts the blocks
+// that are released with a copy of theirs in flight.
+constexpr int MAX_IN_FLIGHT = 4096;
+static const void *g_in_flight[MAX_IN_FLIGHT];
+static int g_num_in_flight = 0;
+static long long g_freed_in_flight = 0;
+static long long g_fail_scatter = -1;  // scatter launches before one fails (emul_error_returns); < 0: none
+void *operator new(size_t n)
+{
+    void *p = std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept
+{
+    for (int k = 0; p && k < g_num_in_flight; k++) g_freed_in_flight += g_in_flight[k] == p;
+    std::free(p);
+}
+void operator delete(void *p, size_t) noexcept { operator delete(p); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind kind, hipStream_t)
 {
     std::memmove(d, s, n);
+    if (g_num_in_flight < MAX_IN_FLIGHT) g_in_flight[g_num_in_flight++] = kind == hipMemcpyHostToDevice ? s : d;
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    g_num_in_flight = 0;
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize()
+{
+    g_num_in_flight = 0;
+    return hipSuccess;
+}
 hipError_t hipGetDevice(int *d)
 {
     *d = 0;
@@ -99,6 +129,7 @@ hipError_t launch_tree_scatter(int nchunks, const TreeChunk *chunks, const TreeS
                                const double *y, const double *z, const int *idx, double *ox, double *oy,
                                double *oz, int *oidx, hipStream_t)
 {
+    if (g_fail_scatter >= 0 && g_fail_scatter-- == 0) return hipErrorLaunchFailure;
     for (int c = 0; c < nchunks; c++) {
         const TreeChunk k = chunks[c];
         const TreeSeg s = segs[k.seg];
@@ -225,6 +256,31 @@ extern "C" int emul_compare(int n, const double *x, const double *y, const doubl
     }
     *nnodes_out = total;
     return 0;
+}
+
+// Builds the tree of n particles with the scatter of partition pass `pass`
+// failing (pass < 0: none fails).  Returns the number of host blocks released
+// while a copy from or to them was in flight, or -1 when the build's outcome
+// is not the expected one.
+extern "C" long long emul_error_returns(int n, const double *x, const double *y, const double *z, int maxpar, int pass)
+{
+    using namespace bt;
+    DevParticles p;
+    p.n = n;
+    std::vector<double> X(x, x + n), Y(y, y + n), Z(z, z + n), X2(n), Y2(n), Z2(n);
+    std::vector<int> I(n), I2(n);
+    p.x = X.data(); p.y = Y.data(); p.z = Z.data(); p.idx = I.data();
+    p.x2 = X2.data(); p.y2 = Y2.data(); p.z2 = Z2.data(); p.idx2 = I2.data();
+    btk::launch_iota(n, p.idx, nullptr);
+    std::vector<std::vector<NodeRec>> recs;
+    std::vector<int> depth;
+    g_num_in_flight = 0;
+    g_freed_in_flight = 0;
+    g_fail_scatter = pass;
+    const std::string e = device_build_trees(p, {DevRoot{0, n, maxpar}}, false, nullptr, recs, depth);
+    g_fail_scatter = -1;
+    if ((pass >= 0 && e.empty()) || g_num_in_flight != 0) return -1;
+    return g_freed_in_flight;
 }
 
 // The device-memory cache (bt_devmem.cpp) on the emulated allocator: reuse

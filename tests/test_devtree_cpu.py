@@ -130,6 +130,27 @@ def test_many_systems(emul, leaves_only):
     assert rc == 0 and nn >= len(sizes)
 
 
+@pytest.mark.parametrize("fail", [-1, 0, 1, 2, 3, 5])
+def test_host_arrays_outlive_their_copies(emul, fail):
+    """No host array is released with an asynchronous copy of it in flight:
+    when the build ends, and when the scatter of its first or a later
+    partition pass fails."""
+    rng = np.random.default_rng(6)
+    x, y, z = rng.uniform(-1, 1, (3, 3000))
+    dp = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))  # noqa: E731
+    emul.emul_error_returns.restype = ctypes.c_longlong
+    assert emul.emul_error_returns(ctypes.c_int(3000), dp(x), dp(y), dp(z), ctypes.c_int(40), ctypes.c_int(fail)) == 0
+
+
+def test_refused_input_leaves_no_copy_in_flight(emul):
+    """The same for coincident particles, which end the build after a pass."""
+    x, y, z = np.repeat(np.array([[0.0, 0.0, 1.0], [0.0, 0.0, 0.5], [0.0, 0.0, 0.25]]), 50, axis=1)
+    dp = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))  # noqa: E731
+    x, y, z = (np.ascontiguousarray(a) for a in (x, y, z))
+    emul.emul_error_returns.restype = ctypes.c_longlong
+    assert emul.emul_error_returns(ctypes.c_int(150), dp(x), dp(y), dp(z), ctypes.c_int(20), ctypes.c_int(-1)) == 0
+
+
 def test_device_memory_cache_on_the_emulated_allocator(emul):
     """bt_devmem.cpp: released blocks are reused for close sizes only,
     the limit trims the largest cached blocks first and frees a release
