@@ -29,8 +29,16 @@ constexpr int HERM_TILE = 256;  // grid points (CP) or targets (downpass) per He
 // upward pass: particles per part (multiples of the 64-particle chunk), so
 // that a system has about HERM_PARTS parts (blocks per 256 grid points); with
 // parts of 16384 the root of 20k particles was two blocks' work (1.08 ms of
-// a 1.45 ms execution at degree 2)
+// a 1.45 ms execution at degree 2).  A part owns a row of 8 P values.  The
+// systems of a batch are cut as they are alone (the same sums in the same
+// order), so their parts run in groups of whole systems that use the same
+// rows one after the other: a plan's rows take HERM_ROW_BYTES at most (twice
+// that with subtraction), or what its largest system or one row per node
+// needs (256 systems of 64k particles at degree 12: 3 GB, where a row for
+// every part would take 36).  Smaller groups leave the chip idle at their
+// ends: 4096 rows cost 6% of the upward pass of 64 systems of 40k at degree 7.
 constexpr int HERM_PARTS = 4096, HERM_PART_MIN = 256;
+constexpr size_t HERM_ROW_BYTES = size_t(1) << 30;
 constexpr int HERM_PLANES = 8;
 // sources per Hermite CP key: heavier keys are split (into rows of their
 // own), so that the launch has many blocks of similar work
@@ -41,7 +49,9 @@ void Plan::build_hermite_work()
 {
     const Params &p = prm_;
     const int P = p.P;
-    hp_node_.clear(); hp_beg_.clear(); hp_end_.clear(); hp_off_.assign(1, 0);
+    hp_node_.clear(); hp_beg_.clear(); hp_end_.clear(); hp_off_.clear();
+    hp_groups_.clear();
+    hp_rows_ = 0;
     hpc_ = WorkCSR();
     hpc_tiles_.clear(); hcp_tiles_.clear(); hdown_tiles_.clear();
     swtab_.clear(); twtab_.clear();
@@ -50,6 +60,7 @@ void Plan::build_hermite_work()
     if (p.compute_type == C_PC) {
         // upward pass: every source node from its own particles, in parts
         // (systems of a batch are split as they are alone)
+        std::vector<int> sys_part = {0};  // first part of every system
         for (const System &sy : sys_) {
             long long all = 0;
             for (int i = 0; i < sy.stree.n; i++) all += sy.stree.numpar[i];
@@ -62,10 +73,29 @@ void Plan::build_hermite_work()
                     hp_beg_.push_back(o);
                     hp_end_.push_back(std::min(e, o + part));
                 }
-                hp_off_.push_back((int)hp_node_.size());
             }
+            sys_part.push_back((int)hp_node_.size());
             hermite_weight_table(sy.stree, p.degree, tab);
             swtab_.insert(swtab_.end(), tab.begin(), tab.end());
+        }
+        // groups of systems within the rows
+        const int ns = (int)sys_.size();
+        hp_rows_ = std::max(nsnodes_, (int)(HERM_ROW_BYTES / (sizeof(double) * HERM_PLANES * P)));
+        for (int s = 0; s < ns; s++) hp_rows_ = std::max(hp_rows_, sys_part[s + 1] - sys_part[s]);
+        hp_rows_ = std::min(hp_rows_, sys_part[ns]);
+        for (int s = 0; s < ns;) {
+            int e = s + 1;
+            while (e < ns && sys_part[e + 1] - sys_part[s] <= hp_rows_) e++;
+            const int n0 = sys_[s].snode_off, n1 = e < ns ? sys_[e].snode_off : nsnodes_;
+            hp_groups_.push_back({sys_part[s], sys_part[e], n0, n1, (int)hp_off_.size()});
+            // each node's rows, counted from the group's first
+            int k = sys_part[s];
+            for (int n = n0; n < n1; n++) {
+                hp_off_.push_back(k - sys_part[s]);
+                while (k < sys_part[e] && hp_node_[k] == n) k++;
+            }
+            hp_off_.push_back(k - sys_part[s]);
+            s = e;
         }
         // the near keys' clusters move to the Hermite PC launch
         WorkCSR nn;
@@ -143,11 +173,24 @@ std::string Plan::validate_hermite() const
 {
     const long long P = prm_.P;
     if (prm_.compute_type == C_PC) {
-        if ((int)hp_off_.size() != nsnodes_ + 1) return "hermite parts per node";
         for (size_t b = 0; b < hp_node_.size(); b++)
             if (hp_node_[b] < 0 || hp_node_[b] >= nsnodes_ || hp_beg_[b] < 0 || hp_end_[b] > N_ ||
                 hp_beg_[b] >= hp_end_[b])
                 return "hermite part";
+        // the groups hold every part and node once, in order, within the rows
+        int part = 0, node = 0;
+        size_t off = 0;
+        for (const HermGroup &g : hp_groups_) {
+            if (g.part0 != part || g.node0 != node || g.off0 != (int)off || g.part1 - g.part0 > hp_rows_ ||
+                g.node1 <= g.node0 || off + (g.node1 - g.node0) >= hp_off_.size() || hp_off_[off] != 0 ||
+                hp_off_[off + (g.node1 - g.node0)] != g.part1 - g.part0)
+                return "hermite part group";
+            for (int n = g.node0; n < g.node1; n++)
+                if (hp_off_[off + n - g.node0] >= hp_off_[off + n - g.node0 + 1]) return "hermite parts per node";
+            part = g.part1; node = g.node1;
+            off += g.node1 - g.node0 + 1;
+        }
+        if (part != (int)hp_node_.size() || node != nsnodes_ || off != hp_off_.size()) return "hermite part groups";
         if (swtab_.size() != (size_t)nsnodes_ * 3 * (prm_.degree + 1)) return "hermite source weights";
         for (const btk::Tile &t : hpc_tiles_)
             if (t.x < 0 || t.x >= (int)hpc_.key.size() || t.y < 0 || t.z <= 0 || t.z > btk::HERM_PC_TILE ||
@@ -187,7 +230,7 @@ std::string Plan::upload_hermite()
         if (!(r = up(&d_hp_end_, hp_end_)).empty()) return r;
         if (!(r = up(&d_hp_off_, hp_off_)).empty()) return r;
         if (!(r = up(&d_swtab_, swtab_)).empty()) return r;
-        const size_t rows = std::max<size_t>(hp_node_.size(), 1) * HERM_PLANES * P;
+        const size_t rows = (size_t)hp_rows_ * HERM_PLANES * P;
         d_Qp_ = dalloc<double>(rows);
         if (ss) d_Wp_ = dalloc<double>(rows);
         if (!d_Qp_ || (ss && !d_Wp_)) return "hipMalloc failed (hermite parts)";
@@ -208,14 +251,19 @@ std::string Plan::hermite_upward()
     const Params &p = prm_;
     const bool ss = p.singularity == S_SUBTRACTION;
     btk::HermAnterpArgs a{};
-    a.degree = p.degree; a.subtraction = ss; a.nparts = (int)hp_node_.size();
-    a.part_node = d_hp_node_; a.part_beg = d_hp_beg_; a.part_end = d_hp_end_;
+    a.degree = p.degree; a.subtraction = ss;
     a.tab = d_stab_; a.wtab = d_swtab_;
     a.px = d_sx_; a.py = d_sy_; a.pz = d_sz_; a.pq = d_sq_; a.pw = d_sw_;
     a.Qp = d_Qp_; a.Wp = d_Wp_;
-    HIPCHK(btk::launch_herm_anterp(a, st_));
-    HIPCHK(btk::launch_sum_parts(nsnodes_, HERM_PLANES * p.P, d_hp_off_, d_Qp_, d_Wp_, d_cq_, ss ? d_cw_ : nullptr,
-                                 st_));
+    const int row = HERM_PLANES * p.P;
+    for (const HermGroup &g : hp_groups_) {
+        a.nparts = g.part1 - g.part0;
+        a.part_node = d_hp_node_ + g.part0; a.part_beg = d_hp_beg_ + g.part0; a.part_end = d_hp_end_ + g.part0;
+        HIPCHK(btk::launch_herm_anterp(a, st_));
+        const size_t o = (size_t)g.node0 * row;
+        HIPCHK(btk::launch_sum_parts(g.node1 - g.node0, row, d_hp_off_ + g.off0, d_Qp_, d_Wp_, d_cq_ + o,
+                                     ss ? d_cw_ + o : nullptr, st_));
+    }
     return "";
 }
 

@@ -411,12 +411,18 @@ private:
     int *d_node_rows_off_ = nullptr;
     double *d_Qrows_ = nullptr, *d_Wrows_ = nullptr;
     // Hermite: 8 planes per grid point.  Upward pass from every source
-    // node's particles in parts (node n: parts [hp_off_[n], hp_off_[n+1]));
+    // node's particles in parts, whose rows are then added per node.  Groups
+    // of systems (parts [part0, part1), nodes [node0, node1)) take the rows in
+    // turn, hp_rows_ of them; hp_off_[off0 + n - node0] is the first row of
+    // the group's node n, and one more entry ends the group;
     // PC: the near keys' clusters in their own launch (hpc_, hpc_tiles_);
     // CP: grid tiles of 256 points (hcp_tiles_), rows of 8P values; the
     // downpass of every target node with rows (hdown_tiles_)
     bool herm_ = false;
+    struct HermGroup { int part0, part1, node0, node1, off0; };
     std::vector<int> hp_node_, hp_beg_, hp_end_, hp_off_;
+    std::vector<HermGroup> hp_groups_;
+    int hp_rows_ = 0;
     WorkCSR hpc_;
     std::vector<btk::Tile> hpc_tiles_, hcp_tiles_, hdown_tiles_;
     std::vector<double> swtab_, twtab_;

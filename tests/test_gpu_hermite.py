@@ -143,6 +143,31 @@ def test_hermite_batched_equals_single_solves(bt):
             assert np.array_equal(r, g)
 
 
+@pytest.mark.parametrize("sing", [1, 2])
+def test_hermite_batch_upward_rows_are_bounded(bt, sing):
+    """A batch whose nodes have more parts than the plan holds rows for: its
+    systems take the rows in turn, each system comes out as it does alone, and
+    the rows take 1 GiB (2 with subtraction) where a row for each of the about
+    15000 parts takes 2.1 GB (4.2)."""
+    sizes = [20000, 17001, 300, 20000, 19000, 12345, 20000] * 12
+    systems = [uniform_cube(n, 200, seed=i) for i, n in enumerate(sizes)]
+    P, leaf = 2197, 2500
+    args = (1, [0.5], sing, 2, 1, 0.7, 12)
+    pick = [0, 2, 5, 41, 83]
+    ref = [bt.solve(*systems[i], *args, leaf, leaf) for i in pick]
+    bt.empty_device_cache()
+    got = bt.solve_batched(systems, *args, max_source_leaf=leaf, max_target_leaf=leaf,
+                           schedule=bt.Schedule.make({}, 2, 1))
+    for i, r in zip(pick, ref):
+        assert np.array_equal(r, got[i]), i
+    two = 2 if sing == 2 else 1
+    nodes = bt.last_stats()["source_nodes"]
+    used = bt.empty_device_cache()
+    print(f"{nodes} nodes, {used / 1e9:.2f} GB", flush=True)
+    # the nodes' charges, the rows, and particles, lists and tables (under 0.2 GB)
+    assert used <= two * (8 * 8 * P * nodes + 2 ** 30) + 2e8
+
+
 def test_hermite_mixed_precision(bt, oracle_mod):
     """Mixed precision: the near field in FP32 pairs, the Hermite far field
     stays FP64."""
