@@ -130,7 +130,7 @@ void Plan::build_hermite_work()
         // its node and follow it, so each node's keys stay consecutive
         {
             WorkCSR raw = std::move(grid_);
-            split_keys(std::move(raw), HERM_KEY_SOURCES, P, false, grid_);
+            split_keys(std::move(raw), {HERM_KEY_SOURCES}, {}, P, false, grid_);
         }
         node_rows_off_.assign(ntnodes_ + 1, 0);
         for (int node : grid_.key) node_rows_off_[node + 1]++;

@@ -84,10 +84,14 @@ void sort_keys(std::vector<std::pair<long long, int>> &ks)
 }
 }  // namespace
 
-void split_keys(WorkCSR &&in, long long max_src, int P, bool multi, WorkCSR &out)
+void split_keys(WorkCSR &&in, const std::vector<long long> &max_src, const std::vector<int> &sys, int P, bool multi,
+                WorkCSR &out)
 {
     const std::vector<long long> src = key_sources(in, P, multi);
-    if (std::none_of(src.begin(), src.end(), [&](long long n) { return n > max_src; })) {
+    auto limit = [&](size_t k) { return max_src[sys.empty() ? 0 : sys[k]]; };
+    bool any = false;
+    for (size_t k = 0; k < src.size() && !any; k++) any = src[k] > limit(k);
+    if (!any) {
         out = std::move(in);
         return;
     }
@@ -103,11 +107,12 @@ void split_keys(WorkCSR &&in, long long max_src, int P, bool multi, WorkCSR &out
             out.seg_off.push_back(s1);
             out.clu_off.push_back(c1);
         };
-        if (src[k] > max_src) {
+        const long long most = limit(k);
+        if (src[k] > most) {
             long long load = 0;
             bool empty = true;
             auto add = [&](long long w, int s1, int c1) {
-                if (!empty && load + w > max_src) { chunk(s1, c1); load = 0; }
+                if (!empty && load + w > most) { chunk(s1, c1); load = 0; }
                 load += w;
                 empty = false;
             };
@@ -123,28 +128,36 @@ void split_keys(WorkCSR &&in, long long max_src, int P, bool multi, WorkCSR &out
     out.clu_id = std::move(in.clu_id);
 }
 
-// Most source points of a grid key: MAX_KEY_SOURCES where that gives the
-// launch (one block per key and chunk of its sources) GRID_BLOCKS blocks, else
-// chunks that give about four times as many, of 2^20 pairs or more (a row of
-// P sums per chunk is written and added up after it).  Cluster-particle
-// far fields with few target nodes: Coulomb with subtraction, FP64, N = 100k,
-// degree 9, 9.9-13.7 ms with chunks of 16384, 5.4 ms so; Yukawa, mixed, 65k
-// sources, 0.77 -> 0.33 ms (150 blocks for 256 CUs before).  Where the chunks
-// of 16384 fill the chip, finer ones only add rows to sum (cluster-cluster,
-// mixed, N = 300k, degree 4: 0.6 -> 1.2 ms).
-long long grid_key_sources(const WorkCSR &w, int P, bool multi)
+// Most source points of a grid key, for every system (sys: each key's; empty:
+// one system): MAX_KEY_SOURCES where that gives the launch (one block per key
+// and chunk of its sources) GRID_BLOCKS blocks, else chunks that give about
+// four times as many, of 2^20 pairs or more (a row of P sums per chunk is
+// written and added up after it).  Cluster-particle far fields with few target
+// nodes: Coulomb with subtraction, FP64, N = 100k, degree 9, 9.9-13.7 ms with
+// chunks of 16384, 5.4 ms so; Yukawa, mixed, 65k sources, 0.77 -> 0.33 ms (150
+// blocks for 256 CUs before).  Where the chunks of 16384 fill the chip, finer
+// ones only add rows to sum (cluster-cluster, mixed, N = 300k, degree 4: 0.6
+// -> 1.2 ms).  A system of a batch is cut as it is alone, so its sums have the
+// same order.
+std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int> &sys, int nsys, int P, bool multi)
 {
     const std::vector<long long> src = key_sources(w, P, multi);
-    long long all = 0, blocks = 0;
-    double pairs = 0.0;
+    struct Load { long long all = 0, blocks = 0; double pairs = 0.0; };
+    std::vector<Load> load(nsys);
     for (size_t k = 0; k < src.size(); k++) {
-        all += src[k];
-        blocks += (src[k] + MAX_KEY_SOURCES - 1) / MAX_KEY_SOURCES;
-        pairs += (double)src[k] * w.tcnt[k];
+        Load &l = load[sys.empty() ? 0 : sys[k]];
+        l.all += src[k];
+        l.blocks += (src[k] + MAX_KEY_SOURCES - 1) / MAX_KEY_SOURCES;
+        l.pairs += (double)src[k] * w.tcnt[k];
     }
-    if (blocks >= GRID_BLOCKS || pairs <= 0.0) return MAX_KEY_SOURCES;
-    const long long work = (long long)((1 << 20) * ((double)all / pairs));
-    return std::min(MAX_KEY_SOURCES, std::max({1024LL, work, all / (4 * GRID_BLOCKS)}));
+    std::vector<long long> most(nsys, MAX_KEY_SOURCES);
+    for (int s = 0; s < nsys; s++) {
+        const Load &l = load[s];
+        if (l.blocks >= GRID_BLOCKS || l.pairs <= 0.0) continue;
+        const long long work = (long long)((1 << 20) * ((double)l.all / l.pairs));
+        most[s] = std::min(MAX_KEY_SOURCES, std::max({1024LL, work, l.all / (4 * GRID_BLOCKS)}));
+    }
+    return most;
 }
 
 void make_queue_tiles(const WorkCSR &w, int tile_t, bool grid, int P, std::vector<btk::Tile> &tiles,
@@ -665,8 +678,8 @@ void Plan::build_work()
         // (systems of a batch are split as they are alone)
         if (!gw.key.empty()) {
             WorkCSR raw = std::move(gw);
-            const long long max_src = grid_key_sources(raw, P, false);
-            split_keys(std::move(raw), max_src, P, false, gw);
+            const std::vector<long long> most = grid_key_sources(raw, {}, 1, P, false);
+            split_keys(std::move(raw), most, {}, P, false, gw);
         }
     };
     auto csr_start = [](WorkCSR &w) { w.seg_off.assign(1, 0); w.clu_off.assign(1, 0); };

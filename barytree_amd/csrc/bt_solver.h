@@ -96,11 +96,13 @@ void make_queue_tiles(const WorkCSR &w, int tile_targets, bool grid, int P,
 // cluster ids carry their degree as in make_queue_tiles.
 void make_pencil_tiles(const WorkCSR &w, int P, bool multi, std::vector<btk::Tile> &tiles);
 
-// Splits every key whose sources (particles plus cluster points) exceed
-// max_src into consecutive chunks of its particle ranges and clusters; the
-// chunks are keys of their own with the same node and targets, in order.
-void split_keys(WorkCSR &&in, long long max_src, int P, bool multi, WorkCSR &out);
-long long grid_key_sources(const WorkCSR &w, int P, bool multi);
+// Splits every key whose sources (particles plus cluster points) exceed its
+// system's max_src (sys: each key's system; empty: one system) into
+// consecutive chunks of its particle ranges and clusters; the chunks are keys
+// of their own with the same node and targets, in order.
+void split_keys(WorkCSR &&in, const std::vector<long long> &max_src, const std::vector<int> &sys, int P, bool multi,
+                WorkCSR &out);
+std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int> &sys, int nsys, int P, bool multi);
 
 struct PlanInput {
     int nsys = 1;

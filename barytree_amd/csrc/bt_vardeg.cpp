@@ -252,11 +252,13 @@ std::string Plan::set_pair_degrees(const int *deg)
     // far: every target slot, degree by degree, split by sources; rows of
     // partial grid values, summed per slot after the launch
     WorkCSR raw;
+    std::vector<int> raw_sys;  // each key's system
     raw.seg_off.push_back(0); raw.clu_off.push_back(0);
     for (int p = 1; p <= MAXDEG; p++) {
         const int T = (int)slot_node[p].size();
         for (int sl = 0; sl < T; sl++) {
             raw.key.push_back(multi_id(p, sl));
+            raw_sys.push_back(slot_sys[p][sl]);
             raw.tbeg.push_back(0);
             raw.tcnt.push_back(dw_[p].P);
             for (size_t j = 0; j < tseg[p][sl].size(); j++) {
@@ -269,8 +271,8 @@ std::string Plan::set_pair_degrees(const int *deg)
             raw.clu_off.push_back((int)raw.clu_id.size());
         }
     }
-    const long long max_src = grid_key_sources(raw, 0, true);
-    split_keys(std::move(raw), max_src, 0, true, vfar_);
+    const std::vector<long long> most = grid_key_sources(raw, raw_sys, (int)sys_.size(), 0, true);
+    split_keys(std::move(raw), most, raw_sys, 0, true, vfar_);
     vfar_row_.assign(vfar_.key.size(), 0);
     vfar_rows_len_ = 0;
     for (size_t k = 0; k < vfar_.key.size(); k++) {

@@ -60,6 +60,30 @@ def test_pair_degrees_below_and_above_the_plan_degree(bt, oracle_mod, ct, k, s):
         assert rel_l2(ref, got) <= 1e-12
 
 
+@pytest.mark.parametrize("ct,s", [(2, 1), (2, 2), (3, 1)])
+def test_pair_degrees_of_a_batch_equal_single_plans(bt, ct, s):
+    """Systems of a batch with per-pair degrees come out as they do alone,
+    bit for bit: the far field's sources are cut by each system's own work,
+    which differs between these (low degrees, high degrees, few particles)."""
+    print(f"case ct={ct} s={s}", flush=True)
+    systems = [uniform_cube(n, m, seed=40 + i) for i, (m, n) in enumerate(((3000, 20000), (2500, 12000), (600, 700)))]
+    args = (1, [0.5], s, 1, ct, 0.7, 3)
+    plan = bt.Plan.batched(systems, *args, max_source_leaf=100, max_target_leaf=100, size_check=0.0,
+                           schedule=bt.Schedule.make({}, 1, 0))
+    try:
+        _, system = plan.pair_info()
+        rng = np.random.default_rng(3)
+        deg = np.where(system == 1, rng.integers(8, 11, len(system)), rng.integers(2, 4, len(system)))
+        plan.set_pair_degrees(deg)
+        out, off = plan.execute(), plan.offsets
+    finally:
+        plan.close()
+    for i, (t, src) in enumerate(systems):
+        with bt.Plan(t, src, *args, 100, 100, size_check=0.0) as p:
+            p.set_pair_degrees(deg[system == i])
+            assert np.array_equal(p.execute(), out[off[i]:off[i + 1]]), i
+
+
 @pytest.mark.parametrize("ct,k,s", supported_combos())
 def test_random_pair_degrees_match_oracle(bt, oracle_mod, ct, k, s):
     print(f"case ct={ct} k={k} s={s}", flush=True)
