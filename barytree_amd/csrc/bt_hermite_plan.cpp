@@ -126,7 +126,7 @@ void Plan::build_hermite_work()
         near_ = std::move(nn);
         make_queue_tiles(near_, tile_targets_, false, P, near_tiles_, near_qlen_);
     } else if (p.compute_type == C_CP) {
-        // grid keys split finer than the Lagrange ones; chunks of a key keep
+        // grid keys of at most HERM_KEY_SOURCES sources; chunks of a key keep
         // its node and follow it, so each node's keys stay consecutive
         {
             WorkCSR raw = std::move(grid_);

@@ -13,6 +13,7 @@
 #include <cstdint>
 #include <cstring>
 #include <map>
+#include <numeric>
 #include <parallel/algorithm>
 
 namespace bt {
@@ -138,8 +139,13 @@ void split_keys(WorkCSR &&in, const std::vector<long long> &max_src, const std::
 // blocks for 256 CUs before).  Where the chunks of 16384 fill the chip, finer
 // ones only add rows to sum (cluster-cluster, mixed, N = 300k, degree 4: 0.6
 // -> 1.2 ms).  A system of a batch is cut as it is alone, so its sums have the
-// same order.
-std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int> &sys, int nsys, int P, bool multi)
+// same order; against chunks of 16384 for all, the far fields of batches of 32
+// to 1000 systems took as long or less (32 systems of 20k, cluster-cluster
+// with subtraction, degree 10, 3.85 -> 1.33 ms; 256 of 30k, cluster-particle,
+// degree 12, 29.2 -> 23.9 ms; Hermite equal).  rows: the values of all rows,
+// about.
+std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int> &sys, int nsys, int P, bool multi,
+                                        double &rows)
 {
     const std::vector<long long> src = key_sources(w, P, multi);
     struct Load { long long all = 0, blocks = 0; double pairs = 0.0; };
@@ -157,8 +163,20 @@ std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int>
         const long long work = (long long)((1 << 20) * ((double)l.all / l.pairs));
         most[s] = std::min(MAX_KEY_SOURCES, std::max({1024LL, work, l.all / (4 * GRID_BLOCKS)}));
     }
+    rows = 0.0;
+    for (size_t k = 0; k < src.size(); k++) {
+        const long long m = most[sys.empty() ? 0 : sys[k]];
+        rows += (double)((src[k] + m - 1) / m) * w.tcnt[k];
+    }
     return most;
 }
+
+// Large batches: rows beyond GRID_ROW_BYTES are not taken for finer chunks.
+// Every system is then cut at MAX_KEY_SOURCES (256 systems of 64k particles,
+// Hermite, degree 12: about 90 GB of rows otherwise, 14 so), which leaves it
+// enough blocks by the number of systems; only there may a system's sums
+// have another order than alone.
+bool rows_fit(double rows, int planes, bool ss) { return rows * 8.0 * planes * (ss ? 2 : 1) <= GRID_ROW_BYTES; }
 
 void make_queue_tiles(const WorkCSR &w, int tile_t, bool grid, int P, std::vector<btk::Tile> &tiles,
                       int *qlen, bool multi)
@@ -674,20 +692,36 @@ void Plan::build_work()
             near_keys(tt.leaves, &clus_of, segs_of);
             grid_keys(&L.approx, L.cc_cp);
         }
-        // heavy grid keys are split by sources; every key writes its own row
-        // (systems of a batch are split as they are alone)
-        if (!gw.key.empty()) {
-            WorkCSR raw = std::move(gw);
-            const std::vector<long long> most = grid_key_sources(raw, {}, 1, P, false);
-            split_keys(std::move(raw), most, {}, P, false, gw);
-        }
     };
     auto csr_start = [](WorkCSR &w) { w.seg_off.assign(1, 0); w.clu_off.assign(1, 0); };
     csr_start(near_);
     csr_start(grid_);
     const int ns = (int)sys_.size();
+    // heavy grid keys are split by sources; every key writes its own row
+    // (systems of a batch are split as they are alone)
+    const int planes = p.approximation == A_HERMITE ? 8 : 1;
+    auto split = [&](std::vector<WorkCSR> &gws) {
+        const int n = (int)gws.size();
+        std::vector<std::vector<long long>> most(n);
+        std::vector<double> rows(n);
+#pragma omp parallel for schedule(dynamic) if (n > 1)
+        for (int s = 0; s < n; s++) most[s] = grid_key_sources(gws[s], {}, 1, P, false, rows[s]);
+        const bool fine = rows_fit(std::accumulate(rows.begin(), rows.end(), 0.0), planes,
+                                   p.singularity == S_SUBTRACTION);
+#pragma omp parallel for schedule(dynamic) if (n > 1)
+        for (int s = 0; s < n; s++) {
+            if (gws[s].key.empty()) continue;
+            if (!fine) most[s] = {MAX_KEY_SOURCES};
+            WorkCSR raw = std::move(gws[s]);
+            split_keys(std::move(raw), most[s], {}, P, false, gws[s]);
+        }
+    };
     if (ns == 1) {
-        per_system(sys_[0], near_, grid_, near_ctr_);
+        std::vector<WorkCSR> gw(1);
+        csr_start(gw[0]);
+        per_system(sys_[0], near_, gw[0], near_ctr_);
+        split(gw);
+        grid_ = std::move(gw[0]);
     } else {
         // systems in parallel (the symmetric near field needs a single
         // system), then concatenated in system order
@@ -699,6 +733,7 @@ void Plan::build_work()
             csr_start(gws[s]);
             per_system(sys_[s], nws[s], gws[s], ctrs[s]);
         }
+        split(gws);
         auto append = [](WorkCSR &w, const WorkCSR &f) {
             const int so = (int)w.seg_beg.size(), co = (int)w.clu_id.size();
             w.key.insert(w.key.end(), f.key.begin(), f.key.end());

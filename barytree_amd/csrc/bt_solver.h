@@ -25,6 +25,7 @@ constexpr int PART_MAX = 16384;  // particles per block of a source slot's charg
 constexpr long long MAX_KEY_SOURCES = 1 << 14;  // source points per grid key at most (heavier keys are
                                                  // split, further in small plans: grid_key_sources)
 constexpr int GRID_BLOCKS = 512;                 // fewest blocks of a grid launch (2 per CU)
+constexpr double GRID_ROW_BYTES = 8.0 * (1 << 30);  // rows of partial grid values that finer chunks may take
 constexpr int SMALL_TARGETS = 1 << 18;  // single-system plans below this many targets: 1 target per thread
 
 struct Timings {
@@ -102,7 +103,9 @@ void make_pencil_tiles(const WorkCSR &w, int P, bool multi, std::vector<btk::Til
 // of their own with the same node and targets, in order.
 void split_keys(WorkCSR &&in, const std::vector<long long> &max_src, const std::vector<int> &sys, int P, bool multi,
                 WorkCSR &out);
-std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int> &sys, int nsys, int P, bool multi);
+std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int> &sys, int nsys, int P, bool multi,
+                                        double &rows);
+bool rows_fit(double rows, int planes, bool ss);
 
 struct PlanInput {
     int nsys = 1;

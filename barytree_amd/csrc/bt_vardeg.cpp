@@ -271,7 +271,9 @@ std::string Plan::set_pair_degrees(const int *deg)
             raw.clu_off.push_back((int)raw.clu_id.size());
         }
     }
-    const std::vector<long long> most = grid_key_sources(raw, raw_sys, (int)sys_.size(), 0, true);
+    double rows = 0.0;
+    std::vector<long long> most = grid_key_sources(raw, raw_sys, (int)sys_.size(), 0, true, rows);
+    if (!rows_fit(rows, 1, ss)) most.assign(most.size(), MAX_KEY_SOURCES);
     split_keys(std::move(raw), most, raw_sys, 0, true, vfar_);
     vfar_row_.assign(vfar_.key.size(), 0);
     vfar_rows_len_ = 0;

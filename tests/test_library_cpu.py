@@ -85,6 +85,24 @@ def test_host_lists_of_many_nodes_match_oracle(bt, oracle_mod, ct, n, m):
     assert a["pp_ptwise"] + a["pc_replaced"] + a["cp_replaced"] + a["cc_replaced"] == n * m
 
 
+def test_rows_of_large_batches_stay_bounded(bt):
+    """A system's grid keys are cut as finely in a batch as alone, while the
+    rows of partial sums (8 planes of 13^3 values here) take less than 8 GiB;
+    a batch that would take more is cut at 16384 sources a key."""
+    P, leaf = 2197, 400
+    args = (1, [0.5], 1, 2, 2, 0.7, 12)
+    systems = [uniform_cube(16000, 16000, seed=i) for i in range(4)]
+    alone = sum(bt.analyze(t, s, *args, leaf, leaf, size_check=0.0)["far_tiles"] for t, s in systems)
+    for copies in (1, 40):
+        a = bt.analyze_batched(systems * copies, *args, max_source_leaf=leaf, max_target_leaf=leaf,
+                               schedule=bt.Schedule.make({}, 2, 0), size_check=0.0)
+        rows = a["far_tiles"] / 5 * 8 * 8 * P  # bytes; 5 tiles of 512 points a key, queues padded to one length
+        if copies == 1:
+            assert 0.9 * alone <= a["far_tiles"] <= alone + 8 * 5 * 4
+        else:
+            assert alone / 5 * 8 * 8 * P * copies > 10e9 and rows < 2 * 2 ** 30, rows
+
+
 @pytest.mark.parametrize("ct,k,s", hermite_combos())
 def test_hermite_host_work_matches_oracle(bt, oracle_mod, ct, k, s):
     """Hermite plans build (and check) their work lists on the host; the
