@@ -863,6 +863,34 @@ void Plan::build_work()
     }
 }
 
+// The items give every near pair to its target: each near key's targets have
+// one slot for every source range of the key (red_off), the slots stand for
+// as many pairs as the ranges hold, and the reduction covers the targets of
+// every key with ranges once, in order.  Mixed cluster-particle executions
+// start the potential at zero and launch nothing that stores every target, so
+// a target without its items would pass for the far field alone.
+std::string check_items(const WorkCSR &near, const std::vector<int> &red_off, const std::vector<btk::Tile> &red_tiles,
+                        long long pairs)
+{
+    const int nk = (int)near.key.size();
+    if ((int)red_off.size() != nk + 1) return "sym keys";
+    long long need = 0;
+    size_t tile = 0;
+    for (int k = 0; k < nk; k++) {
+        if (red_off[k + 1] - red_off[k] != near.seg_off[k + 1] - near.seg_off[k]) return "sym slots of a key";
+        for (int s = near.seg_off[k]; s < near.seg_off[k + 1]; s++) need += (long long)near.tcnt[k] * near.seg_cnt[s];
+        if (red_off[k + 1] == red_off[k]) continue;
+        int at = near.tbeg[k];
+        for (; tile < red_tiles.size() && red_tiles[tile].x == k; tile++) {
+            if (red_tiles[tile].y != at) return "sym tiles of a key";
+            at += red_tiles[tile].z;
+        }
+        if (at != near.tbeg[k] + near.tcnt[k]) return "sym tiles of a key";
+    }
+    if (tile != red_tiles.size()) return "sym tiles";
+    return need == pairs ? "" : "sym pairs";
+}
+
 // Every index a kernel will dereference is checked here, on the host,
 // before anything is launched.
 std::string Plan::validate() const
@@ -931,6 +959,7 @@ std::string Plan::validate() const
                 if (sym_red_base_[k] + t.y < 0 || sym_red_base_[k] + t.y + t.z > sym_slots_len_)
                     return "sym slot base";
         }
+        if (!(e = check_items(near_, sym_red_off_, sym_red_tiles_, sym_pairs_)).empty()) return e;
     }
     if (!(e = chk_csr(grid_, grid_tiles_, true)).empty()) return "far " + e;
     if (pencil_tiles_.size() != grid_.key.size()) return "pencil tiles";

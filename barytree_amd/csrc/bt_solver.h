@@ -106,6 +106,9 @@ void split_keys(WorkCSR &&in, const std::vector<long long> &max_src, const std::
 std::vector<long long> grid_key_sources(const WorkCSR &w, const std::vector<int> &sys, int nsys, int P, bool multi,
                                         double &rows);
 bool rows_fit(double rows, int planes, bool ss);
+// "" if the near field's items cover its pairs and targets
+std::string check_items(const WorkCSR &near, const std::vector<int> &red_off, const std::vector<btk::Tile> &red_tiles,
+                        long long pairs);
 
 struct PlanInput {
     int nsys = 1;
