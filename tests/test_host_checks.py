@@ -1,6 +1,7 @@
 """Host parts of the library that the C ABI does not show
-(tests/host_checks.cpp): the check that the near field's items cover every
-pair and target."""
+(tests/host_checks.cpp): the interaction lists, entry by entry in order,
+against the reference's walks in one thread, and the check that the near
+field's items cover every pair and target."""
 import ctypes
 import os
 import subprocess
@@ -24,6 +25,23 @@ def checks(tmp_path_factory):
                     f"-I{rocm}/include", os.path.join(ROOT, "tests", "host_checks.cpp"), lib,
                     f"-Wl,-rpath,{os.path.dirname(lib)}", "-o", out], check=True, capture_output=True)
     return ctypes.CDLL(out)
+
+
+@pytest.mark.parametrize("cc", [0, 1])
+@pytest.mark.parametrize("n,m", [(9000, 9000), (20000, 300), (300, 20000)])
+@pytest.mark.parametrize("degree", [1, 3])
+def test_lists_have_the_order_of_one_walk(checks, cc, n, m, degree):
+    """Trees above 1024 nodes, whose lists several threads write: sums run
+    over the lists and pairs are numbered by them, so the order counts."""
+    rng = np.random.default_rng(n + m)
+    dp = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))  # noqa: E731
+    pts = [np.sign(u) * np.abs(u) ** rng.uniform(2.0, 4.0)
+           for u in (rng.uniform(-1, 1, k) for k in (n, n, n, m, m, m))]
+    keys = ctypes.c_int(0)
+    bad = checks.check_lists(ctypes.c_int(cc), ctypes.c_int(n), *map(dp, pts[:3]), ctypes.c_int(m), *map(dp, pts[3:]),
+                             ctypes.c_double(0.7), ctypes.c_int(degree), ctypes.c_int(6), ctypes.byref(keys))
+    assert bad == 0
+    assert m < 9000 or keys.value > 1024
 
 
 def test_items_cover_check(checks):
