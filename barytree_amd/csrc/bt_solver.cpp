@@ -1025,6 +1025,7 @@ std::string Plan::create(const Params &prm, const PlanInput &in, bool host_only)
 {
     free_all();
     prm_ = prm;
+    set_precision(prm.precision);
     std::string e = params_check(prm);
     if (!e.empty()) return e;
     if (in.nsys < 1 || !in.toffs || !in.soffs) return "need at least one system";

@@ -158,7 +158,12 @@ public:
     // no host heap either.  Results equal direct()'s bit for bit.
     std::string direct_noalloc(int m, const int *idx, double *out, void *scratch, size_t bytes);
 
-    void set_precision(int p) { prm_.precision = p; }
+    // Mixed precision scales Yukawa's coordinates by kappa, so it needs
+    // kappa > 0: other rates run in FP64.
+    void set_precision(int p)
+    {
+        prm_.precision = prm_.kernel == K_YUKAWA && !(prm_.kp[0] > 0.0) ? PREC_FP64 : p;
+    }
 
     // Far-field pairs in list order (per system; PC: per target batch its
     // approx list; CP: per source batch its approx list; CC: per target node

@@ -91,7 +91,8 @@ void BaryTreeInterface(int numTargets, int numSources,
 #define BARYTREE_PRECISION_FP64 0  /* plain mode: FP64 throughout */
 #define BARYTREE_PRECISION_MIXED 1 /* FP32 pair evaluation with compensated
                                       per-target accumulation; cluster charges,
-                                      interpolation weights and totals FP64 */
+                                      interpolation weights and totals FP64.
+                                      Yukawa with kappa <= 0 runs in FP64 */
 
 /* Interaction counts (the reference's verbosity>2 diagnostics,
  * src/drivers/treedriver.c:191-200, 472-483, 763-792) and phase times. */

@@ -216,3 +216,23 @@ def test_verbosity_diagnostics(bt, capfd):
     assert "GPU: near field" in out
     bt.solve(t, s, *args, verbosity=0)
     assert capfd.readouterr().out == ""
+
+
+@pytest.mark.parametrize("ct,s", [(1, 1), (1, 2), (2, 1), (3, 2)])
+@pytest.mark.parametrize("kappa", [-0.5, 0.0])
+@pytest.mark.parametrize("same", [False, True])
+def test_mixed_yukawa_without_a_positive_rate_runs_in_fp64(bt, oracle_mod, ct, s, kappa, same):
+    """Mixed precision scales by kappa; a rate that is not positive runs in
+    FP64 instead, as a solve and as a plan switched to mixed precision."""
+    if s == 2 and kappa == 0.0:
+        pytest.skip("the subtraction's correction divides by kappa")
+    t, src = uniform_cube(2500, 2000, seed=60 + ct)
+    if same:
+        t = [a.copy() for a in src[:4]]
+    args = (2, [kappa], s, 1, ct, 0.7, 3, 60, 60)
+    ref = oracle_mod.treecode(*t, *src, *args)
+    got = bt.solve(t, src, *args, precision=bt.PRECISION_MIXED)
+    assert rel_l2(ref, got) <= 1e-12
+    with bt.Plan(t, src, *args) as p:
+        p.set_precision(bt.PRECISION_MIXED)
+        assert np.array_equal(p.execute(), got)
