@@ -698,30 +698,17 @@ void Plan::build_work()
     csr_start(grid_);
     const int ns = (int)sys_.size();
     // heavy grid keys are split by sources; every key writes its own row
-    // (systems of a batch are split as they are alone)
-    const int planes = p.approximation == A_HERMITE ? 8 : 1;
-    auto split = [&](std::vector<WorkCSR> &gws) {
-        const int n = (int)gws.size();
-        std::vector<std::vector<long long>> most(n);
-        std::vector<double> rows(n);
-#pragma omp parallel for schedule(dynamic) if (n > 1)
-        for (int s = 0; s < n; s++) most[s] = grid_key_sources(gws[s], {}, 1, P, false, rows[s]);
-        const bool fine = rows_fit(std::accumulate(rows.begin(), rows.end(), 0.0), planes,
-                                   p.singularity == S_SUBTRACTION);
-#pragma omp parallel for schedule(dynamic) if (n > 1)
-        for (int s = 0; s < n; s++) {
-            if (gws[s].key.empty()) continue;
-            if (!fine) most[s] = {MAX_KEY_SOURCES};
-            WorkCSR raw = std::move(gws[s]);
-            split_keys(std::move(raw), most[s], {}, P, false, gws[s]);
-        }
+    // (systems of a batch are split as they are alone).  cut: one system's
+    auto cut = [&](WorkCSR &gw, const std::vector<long long> &most) {
+        WorkCSR raw = std::move(gw);
+        split_keys(std::move(raw), most, {}, P, false, gw);
     };
     if (ns == 1) {
-        std::vector<WorkCSR> gw(1);
-        csr_start(gw[0]);
-        per_system(sys_[0], near_, gw[0], near_ctr_);
-        split(gw);
-        grid_ = std::move(gw[0]);
+        // (no parallel region around these: threads of a region within one,
+        // even one of a single thread, are started anew each time)
+        double rows = 0.0;
+        per_system(sys_[0], near_, grid_, near_ctr_);
+        if (!grid_.key.empty()) cut(grid_, grid_key_sources(grid_, {}, 1, P, false, rows));
     } else {
         // systems in parallel (the symmetric near field needs a single
         // system), then concatenated in system order
@@ -733,7 +720,15 @@ void Plan::build_work()
             csr_start(gws[s]);
             per_system(sys_[s], nws[s], gws[s], ctrs[s]);
         }
-        split(gws);
+        std::vector<std::vector<long long>> most(ns);
+        std::vector<double> rows(ns);
+#pragma omp parallel for schedule(dynamic)
+        for (int s = 0; s < ns; s++) most[s] = grid_key_sources(gws[s], {}, 1, P, false, rows[s]);
+        if (!rows_fit(std::accumulate(rows.begin(), rows.end(), 0.0), p.approximation == A_HERMITE ? 8 : 1,
+                      p.singularity == S_SUBTRACTION))
+            most.assign(ns, {MAX_KEY_SOURCES});
+#pragma omp parallel for schedule(dynamic)
+        for (int s = 0; s < ns; s++) cut(gws[s], most[s]);
         auto append = [](WorkCSR &w, const WorkCSR &f) {
             const int so = (int)w.seg_beg.size(), co = (int)w.clu_id.size();
             w.key.insert(w.key.end(), f.key.begin(), f.key.end());
