@@ -767,7 +767,7 @@ __global__ __launch_bounds__(256) void k_grid_pencil(InteractArgs A)
 // thread that stages a source forms its NL factors e^{-dx^2/a^2} into LDS
 // (over the group sums' space), a pencil's thread e^{-(dy^2+dz^2)/a^2} once
 // per source, and a pair pays two products instead of an 11-instruction
-// exponential.  Coulomb, cluster-cluster, N = 2M, degree 8: the execution
+// exponential.  Coulomb, cluster-cluster, N = 2M, degree 10: the execution
 // 160-166 -> 145 ms; N = 300k, degree 12, 37.9 -> 31.5 ms.  The error
 // against the reference's sums stayed where it was (1.0e-15 to 3.1e-15).
 // The FP32 form above keeps its own exponential per pair: with products its

@@ -66,8 +66,8 @@ def test_hermite_particle_cluster_tiles(bt, oracle_mod, m):
 @pytest.mark.parametrize("deg", [1, 2, 3, 4, 5, 6])
 def test_hermite_cluster_particle_shares(bt, oracle_mod, deg):
     """Grids of 8 to 125 points, whose blocks split the sources into 32 to 2
-    shares, and of 216 and 343, which do not; source batches smaller than the
-    number of shares included."""
+    shares, of 216, which do not, and of 343, whose second tile of 87 points
+    has 2 shares; source batches smaller than the number of shares included."""
     t, src = uniform_cube(4000, 4000, seed=500 + deg)
     for k, leaf in ((1, 20), (2, 300), (3, 80)):
         args = (k, KP[k][1], 1, 2, 2, 0.7, deg, leaf, 400)
