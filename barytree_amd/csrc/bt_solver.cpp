@@ -1280,13 +1280,20 @@ std::string Plan::finish_create(const PlanInput &in, bool host_only, double t2)
     const int ns = (int)sys_.size();
     std::string e;
 
-    // interaction lists (treedriver.c:181, 462, 753)
-#pragma omp parallel for schedule(dynamic) if (ns > 1)
-    for (int s = 0; s < ns; s++) {
-        System &y = sys_[s];
+    // interaction lists (treedriver.c:181, 462, 753); a single system's
+    // outside of any parallel region, for the walks have their own (a region
+    // within one, even one of a single thread, starts its threads anew: every
+    // tenth call of N = 60k with 2600 nodes took 45 ms instead of 12)
+    auto make_lists = [&](System &y) {
         if (prm.compute_type == C_PC) make_pc_lists(y.L, y.stree, y.ttree, prm);
         else if (prm.compute_type == C_CP) make_pc_lists(y.L, y.ttree, y.stree, prm);
         else make_cc_lists(y.L, y.stree, y.ttree, prm);
+    };
+    if (ns == 1) {
+        make_lists(sys_[0]);
+    } else {
+#pragma omp parallel for schedule(dynamic)
+        for (int s = 0; s < ns; s++) make_lists(sys_[s]);
     }
     double t3 = now();
     tm_.host_lists = t3 - t2;

@@ -1,10 +1,12 @@
 """Host parts of the library that the C ABI does not show
 (tests/host_checks.cpp): the interaction lists, entry by entry in order,
-against the reference's walks in one thread, and the check that the near
-field's items cover every pair and target."""
+against the reference's walks in one thread, the check that the near
+field's items cover every pair and target, and that a call uses the threads
+that are there."""
 import ctypes
 import os
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -46,3 +48,31 @@ def test_lists_have_the_order_of_one_walk(checks, cc, n, m, degree):
 
 def test_items_cover_check(checks):
     assert checks.check_cover() == 0
+
+
+def next_thread_id():
+    """The id of a thread started now; ids are given in sequence."""
+    out = []
+    t = threading.Thread(target=lambda: out.append(threading.get_native_id()))
+    t.start()
+    t.join()
+    return out[0]
+
+
+@pytest.mark.parametrize("ct", [1, 2, 3])
+def test_a_call_starts_no_threads(checks, ct):
+    """Plans of one system, once the first call has started the threads of its
+    parallel loops: later calls start none (the least of several calls, for
+    other processes take ids too).  A parallel region within another starts
+    its threads anew each time, which costs milliseconds and now and then
+    tens of them."""
+    import barytree_amd as bt
+    from tests.helpers import uniform_cube
+    t, s = uniform_cube(12000, 12000, seed=ct)
+    started = []
+    for _ in range(8):
+        before = next_thread_id()
+        a = bt.analyze(t, s, 1, [0.5], 1, 1, ct, 0.7, 1, 6, 6)
+        started.append(next_thread_id() - before - 1)
+    assert max(a["source_nodes"], a["target_nodes"]) > 1024
+    assert min(started[1:]) == 0, started
